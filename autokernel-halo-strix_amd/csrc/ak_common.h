@@ -80,6 +80,53 @@ __device__ __forceinline__ void store16_nt(T* p, const Vec16<T>& v) {
   __builtin_nontemporal_store(v.u, reinterpret_cast<u32x4*>(p));
 }
 
+// The same accesses without the 16-byte alignment (element alignment is
+// enough: global memory takes a dwordx4 access at any address, one more cache
+// line per wave when it is off).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+
+template <typename T>
+__device__ __forceinline__ Vec16<T> load16_any_nt(const T* p) {
+  Vec16<T> v;
+  v.u = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+  return v;
+}
+
+template <typename T>
+__device__ __forceinline__ void store16_any_nt(T* p, const Vec16<T>& v) {
+  __builtin_nontemporal_store(v.u, reinterpret_cast<u32x4_any*>(p));
+}
+
+// Makes a held vector opaque, so that what a later pass derives from it is
+// derived again instead of being kept in registers from the pass before.
+template <typename T>
+__device__ __forceinline__ void keep_packed(Vec16<T>& v) {
+  asm volatile("" : "+v"(v.u));
+}
+
+// -inf in every element of a vector.
+template <typename T>
+__device__ __forceinline__ u32x4 vec_neg_inf() {
+  const uint32_t w = sizeof(T) == 4 ? 0xFF800000u : (std::is_same<T, f16>::value ? 0xFC00FC00u : 0xFF80FF80u);
+  return u32x4{w, w, w, w};
+}
+
+// How a row of `cols` elements at any address splits into 16-byte vectors:
+// `head` elements up to the first 16-byte boundary, `nvec` aligned vectors,
+// the rest. Head and rest are at most 2 (VE - 1) = 14 elements, one for each
+// of the row's first `nx` threads: thread t holds element extra(t).
+template <typename T>
+struct RowSplit {
+  static constexpr int VE = Vec16<T>::VE;
+  int head, nvec, nx;
+  __device__ __forceinline__ RowSplit(const T* row, int cols) {
+    head = min((int)((0u - (unsigned)reinterpret_cast<uintptr_t>(row)) & 15u) / (int)sizeof(T), cols);
+    nvec = (cols - head) / VE;
+    nx = cols - nvec * VE;
+  }
+  __device__ __forceinline__ int extra(int t) const { return t < head ? t : nvec * VE + t; }
+};
+
 // ---------------------------------------------------------------------------
 // Wave64 reductions. Within a 16-lane row the partner values come from DPP
 // lane permutations (quad_perm xor1 / xor2, row_half_mirror, row_mirror);

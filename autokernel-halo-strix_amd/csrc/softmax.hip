@@ -1,10 +1,10 @@
 // Row softmax over the last dimension for gfx950 (reference.py:14-17).
 //
-// HBM-bound: each row is read once into registers (as fp32), reduced for its
-// max and for sum(exp(x - max)) with wave64 DPP reductions, then normalised
+// HBM-bound: each row is read once into registers, reduced for its max and
+// for sum(exp(x - max)) in fp32 with wave64 DPP reductions, then normalised
 // and written once, with nontemporal accesses. Rows of up to 128 16-byte
 // vectors are owned by one wave (no barriers), wider rows by up to 1024
-// threads holding one vector each (up to 8 past 1024 vectors). Rows are
+// threads holding one vector each (up to 16 past 1024 vectors). Rows are
 // indexed with 64-bit arithmetic and walked by grid stride on a capped grid,
 // so every row is written whatever the row count.
 //
@@ -18,37 +18,81 @@ namespace {
 
 // TPR threads own a row (TPR / 64 waves; 256 / TPR rows per workgroup when
 // TPR < 256); rows are walked with a workgroup-uniform grid stride so the
-// cross-wave reductions' barriers are reached by every wave. NT selects
-// nontemporal global loads and stores.
-template <typename T, int VPT, int TPR, bool NT>
-__global__ void __launch_bounds__(TPR >= 256 ? TPR : 256)
+// cross-wave reductions' barriers are reached by every wave.
+//
+// RAG: rows at any address and of any width (an odd vocabulary, an odd number
+// of tokens). The vectors start at the row's first 16-byte boundary and the
+// few elements before the first and behind the last one go one to a thread,
+// so the row still crosses HBM once, in whole vectors. [4096, 50257] fp16:
+// 152 us, 5.4 TB/s, as a copy runs here (523 us with element accesses and two
+// passes); [9324, 777] fp16 24.4 -> 11.1 us.
+//
+// From 4 vectors a thread of 16-bit elements on, the row stays packed between
+// the passes and exp(x - max) is formed twice: 32 registers for 8 vectors
+// instead of 64, so two 1024-thread workgroups fit a CU and one's loads run
+// under the other's arithmetic ([4096, 50256] fp16: 179 -> 151 us).
+template <typename T, int VPT, int TPR, bool RAG>
+__global__ void __launch_bounds__(TPR >= 256 ? TPR : 256, VPT == 8 ? 8 : 1)
 softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int cols,
                    int64_t ld_x, int64_t ld_y) {
   constexpr int VE = Vec16<T>::VE;
   constexpr int RPW = TPR >= 256 ? 1 : 256 / TPR;
   constexpr int WPR = TPR / 64;
+  constexpr bool PACKED = VPT >= 4;
   static_assert(TPR % 64 == 0, "rows are owned by whole waves");
   __shared__ float part[RPW][WPR];
   const int t = threadIdx.x % TPR;
   const int rl = threadIdx.x / TPR;
-  const int nvec = cols / VE;
 
   for (int64_t base = (int64_t)blockIdx.x * RPW; base < rows; base += (int64_t)gridDim.x * RPW) {
-    const int64_t row = base + rl;
-    const bool live = row < rows;
+    const int64_t row = RPW == 1 ? base : base + rl;
+    const bool live = RPW == 1 || row < rows;
     const T* xr = x + row * ld_x;
-    float v[VPT][VE];
+    int head = 0, nvec = cols / VE, ex = -1;  // ex: this thread's single element, if any
+    if constexpr (RAG) {
+      const RowSplit<T> sp(xr, cols);
+      head = sp.head;
+      nvec = sp.nvec;
+      if (live && t < sp.nx) ex = sp.extra(t);
+    }
+    Vec16<T> raw[PACKED ? VPT : 1];
+    float v[PACKED ? 1 : VPT][VE];
+    float xe = -INFINITY;
     float m = -INFINITY;
+    // vector t + k TPR, from a workgroup-uniform address and one lane offset
+    const unsigned to = t * VE;
+    auto ld = [&](int k) {
+      const T* xk = xr + head + k * TPR * VE;
+      return RAG ? load16_any_nt(xk + to) : load16_nt(xk + to);
+    };
+    if constexpr (PACKED) {
 #pragma unroll
-    for (int k = 0; k < VPT; ++k) {
-      const int c = t + k * TPR;
-      if (live && c < nvec) {
-        Vec16<T> xv = NT ? load16_nt(xr + (int64_t)c * VE) : load16(xr + (int64_t)c * VE);
+      for (int k = 0; k < VPT; ++k) {  // vectors past the row stay -inf
+        raw[k].u = vec_neg_inf<T>();
+        if (t + k * TPR < nvec) raw[k] = ld(k);
+      }
+    } else {
 #pragma unroll
-        for (int e = 0; e < VE; ++e) {
-          v[k][e] = to_f32(xv.e[e]);
-          m = fmaxf(m, v[k][e]);
+      for (int k = 0; k < VPT; ++k) {
+        if (live && t + k * TPR < nvec) {
+          const Vec16<T> xv = ld(k);
+#pragma unroll
+          for (int e = 0; e < VE; ++e) {
+            v[k][e] = to_f32(xv.e[e]);
+            m = fmaxf(m, v[k][e]);
+          }
         }
+      }
+    }
+    if constexpr (RAG) {
+      if (ex >= 0) m = fmaxf(m, xe = to_f32(xr[ex]));
+    }
+    if constexpr (PACKED) {
+#pragma unroll
+      for (int k = 0; k < VPT; ++k) {
+#pragma unroll
+        for (int e = 0; e < VE; ++e) m = fmaxf(m, to_f32(raw[k].e[e]));
+        keep_packed(raw[k]);
       }
     }
     m = wave_max(m);
@@ -65,14 +109,20 @@ softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int
     float s = 0.0f;
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int c = t + k * TPR;
-      if (live && c < nvec) {
+      if constexpr (PACKED) {
+#pragma unroll
+        for (int e = 0; e < VE; ++e) s += fast_exp(to_f32(raw[k].e[e]) - m);
+        keep_packed(raw[k]);
+      } else if (live && t + k * TPR < nvec) {
 #pragma unroll
         for (int e = 0; e < VE; ++e) {
           v[k][e] = fast_exp(v[k][e] - m);
           s += v[k][e];
         }
       }
+    }
+    if constexpr (RAG) {
+      if (ex >= 0) s += (xe = fast_exp(xe - m));
     }
     s = wave_sum(s);
     if constexpr (WPR > 1) {
@@ -92,10 +142,17 @@ softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int
       if (live && c < nvec) {
         Vec16<T> o;
 #pragma unroll
-        for (int e = 0; e < VE; ++e) o.e[e] = from_f32<T>(v[k][e] * inv);
-        if (NT) store16_nt(yr + (int64_t)c * VE, o);
-        else store16(yr + (int64_t)c * VE, o);
+        for (int e = 0; e < VE; ++e) {
+          if constexpr (PACKED) o.e[e] = from_f32<T>(fast_exp(to_f32(raw[k].e[e]) - m) * inv);
+          else o.e[e] = from_f32<T>(v[k][e] * inv);
+        }
+        T* yk = yr + head + k * TPR * VE;
+        if constexpr (RAG) store16_any_nt(yk + to, o);
+        else store16_nt(yk + to, o);
       }
+    }
+    if constexpr (RAG) {
+      if (ex >= 0) yr[ex] = from_f32<T>(xe * inv);
     }
   }
 }
@@ -113,8 +170,9 @@ __device__ __forceinline__ MaxSum combine(MaxSum a, MaxSum b) {
   return {m, sa + sb};
 }
 
-// Any width / alignment: a 256-thread workgroup per row (rows by grid
-// stride), two passes over global memory (online max/sum, then normalise).
+// Rows of more than 16384 vectors: a 256-thread workgroup per row (rows
+// by grid stride), two passes over global memory (online max/sum, then
+// normalise).
 template <typename T>
 __device__ void softmax_generic_row(const T* __restrict__ xr, T* __restrict__ yr, int cols,
                                     MaxSum* part) {
@@ -159,13 +217,15 @@ softmax_generic_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows,
   }
 }
 
-template <typename T, int VPT, int TPR, bool NT>
-void launch_vec(const T* x, T* y, int64_t rows, int cols, int64_t ld_x, int64_t ld_y,
+template <typename T, int VPT, int TPR>
+void launch_vec(bool aligned, const T* x, T* y, int64_t rows, int cols, int64_t ld_x, int64_t ld_y,
                 hipStream_t s) {
   constexpr int RPW = TPR >= 256 ? 1 : 256 / TPR;
-  const unsigned grid = row_grid((rows + RPW - 1) / RPW);
-  softmax_vec_kernel<T, VPT, TPR, NT><<<dim3(grid), dim3(TPR * RPW), 0, s>>>(
-      x, y, rows, cols, ld_x, ld_y);
+  const dim3 grid(row_grid((rows + RPW - 1) / RPW)), block(TPR * RPW);
+  if (aligned)
+    softmax_vec_kernel<T, VPT, TPR, false><<<grid, block, 0, s>>>(x, y, rows, cols, ld_x, ld_y);
+  else
+    softmax_vec_kernel<T, VPT, TPR, true><<<grid, block, 0, s>>>(x, y, rows, cols, ld_x, ld_y);
 }
 
 template <typename T>
@@ -174,21 +234,21 @@ int dispatch(const void* xv, void* yv, int64_t rows, int64_t cols, int64_t ld_x,
   const T* x = static_cast<const T*>(xv);
   T* y = static_cast<T*>(yv);
   constexpr int VE = Vec16<T>::VE;
-  const bool vec_ok = cols % VE == 0 && ld_x % VE == 0 && ld_y % VE == 0 && aligned16(x) &&
-                      aligned16(y);
+  const bool aligned = cols % VE == 0 && ld_x % VE == 0 && ld_y % VE == 0 && aligned16(x) &&
+                       aligned16(y);
   const int64_t nvec = cols / VE;
   const int c = (int)cols;
-#define AK_LAUNCH(VPT, TPR) launch_vec<T, VPT, TPR, true>(x, y, rows, c, ld_x, ld_y, s)
-  if (!vec_ok || nvec > 8192) {
-    softmax_generic_kernel<T><<<dim3(row_grid(rows)), dim3(256), 0, s>>>(x, y, rows, c, ld_x, ld_y);
-  } else if (nvec <= 64) AK_LAUNCH(1, 64);
+#define AK_LAUNCH(VPT, TPR) launch_vec<T, VPT, TPR>(aligned, x, y, rows, c, ld_x, ld_y, s)
+  if (nvec <= 64) AK_LAUNCH(1, 64);
   else if (nvec <= 128) AK_LAUNCH(2, 64);
   else if (nvec <= 256) AK_LAUNCH(1, 256);
   else if (nvec <= 512) AK_LAUNCH(1, 512);
   else if (nvec <= 1024) AK_LAUNCH(1, 1024);
   else if (nvec <= 2048) AK_LAUNCH(2, 1024);
   else if (nvec <= 4096) AK_LAUNCH(4, 1024);
-  else AK_LAUNCH(8, 1024);
+  else if (nvec <= 8192) AK_LAUNCH(8, 1024);
+  else if (nvec <= 16384) AK_LAUNCH(16, 1024);
+  else softmax_generic_kernel<T><<<dim3(row_grid(rows)), dim3(256), 0, s>>>(x, y, rows, c, ld_x, ld_y);
 #undef AK_LAUNCH
   return ak_check_launch("ak_softmax_fwd");
 }

@@ -110,3 +110,39 @@ def test_softmax_grid_stride_and_expanded_rows():
     say("softmax expanded")
     ye = softmax.kernel_fn(xe.to(DEV)).cpu()
     assert max_ulp(ye, ops.softmax_ref(xe.contiguous())) <= 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vecs,over", [(0, 3), (1, 0), (63, 1), (64, 3), (128, 1), (256, 2), (512, 3), (1025, 1),
+                                       (2049, 3), (4097, 0), (8192, 1), (8193, 3), (16384, 3), (16385, 1)])
+def test_softmax_rows_at_any_address(dtype, vecs, over):
+    """Ragged rows at the edges of every vectors-per-thread variant (``vecs``
+    16-byte vectors plus ``over`` elements), read from and written to pitched
+    views that start off the 16-byte grid, not always the same way; the
+    elements around the output rows keep their values."""
+    need_gpu()
+    from kernels.hip import _lib
+    ve = 16 // torch.empty((), dtype=dtype).element_size()
+    cols, rows = max(1, vecs * ve + over), 5
+    g = torch.Generator().manual_seed(cols)
+    x = (4 * torch.randn(rows, cols, generator=g)).to(dtype)
+    x[1, ::2] = float("-inf")
+    x[2] = torch.finfo(dtype).min  # all masked with the type's lowest value: uniform
+    x[3, cols // 2] = float("nan")
+    ref = ops.softmax_ref(x)
+    for ox, oy, px, py in ((0, 0, 0, 0), (1, 1, 3, 3), (3, 2, 0, 1)):
+        say("softmax any address", dtype, cols, ox, oy)
+        xb = torch.zeros(rows, cols + ox + px, dtype=dtype)
+        xb[:, ox:ox + cols] = x
+        yb = torch.full((rows, cols + oy + py), 7.0, dtype=dtype, device=DEV)
+        _lib.softmax(xb.to(DEV)[:, ox:ox + cols], yb[:, oy:oy + cols])
+        yb = yb.cpu()
+        y = yb[:, oy:oy + cols]
+        assert bool((yb[:, :oy] == 7).all()) and bool((yb[:, oy + cols:] == 7).all())
+        assert bool(torch.isnan(y[3]).all())
+        live = [i for i in (0, 1, 2, 4) if not (i == 1 and cols == 1)]
+        if dtype == torch.float32:
+            d = (y[live].double() - ref[live].double()).abs()
+            assert bool((d <= 1e-5 * ref[live].double().abs() + 1e-7).all())
+        else:
+            assert max_ulp(y[live], ref[live]) <= 1
