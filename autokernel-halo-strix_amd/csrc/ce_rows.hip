@@ -9,14 +9,16 @@
 //            * (softcap ? 1 - tanh^2 : 1) * scale
 //   (w = z-loss weight: the gradient of loss + w lse^2); ignored rows get a
 //   zero gradient row.
-// A 256-thread workgroup owns a row (rows by grid stride), streams it with
-// 16-byte loads and keeps a per-thread online (max, sum) pair, merged across
-// the workgroup with wave64 shuffles and LDS. The gradient pass re-reads the
-// row (it is normally still resident in L2 / MALL). The gradient scale can
-// come from device memory (scale_dev), so the mean's 1 / #counted-rows and
-// the upstream gradient never need a host read. ce_count_kernel and
-// ce_mean_kernel reduce the targets and per-row results in one workgroup in
-// a fixed order (deterministic).
+// The forward holds a row of up to 16384 16-byte vectors in registers, packed,
+// so that it crosses HBM once whether or not the gradient is written; wider
+// rows are streamed (the gradient pass re-reads the row). Row addresses and
+// widths are free: vectors start at the row's first 16-byte boundary. The
+// gradient scale can come from device memory (scale_dev), so the mean's 1 /
+// #counted-rows and the upstream gradient never need a host read.
+// ce_count_kernel and ce_mean_kernel reduce the targets and per-row results in
+// one workgroup in a fixed order (deterministic).
+#include <algorithm>
+
 #include "ak_common.h"
 
 namespace ak {
@@ -26,6 +28,7 @@ constexpr int kCeThreads = 256;
 
 struct CeParams {
   float softcap, inv_softcap, ls, ls_uniform, scale, zw2;  // zw2 = 2 * z-loss weight
+  float tcoeff, vocab;  // 1 - ls (1 without smoothing), the vocabulary as a float
   const float* scale_dev;  // optional device factor of scale
   int64_t ignore_index;
   bool use_softcap, use_ls;
@@ -76,56 +79,228 @@ __device__ MS block_merge(MS st, float& sum_x) {
   return st;
 }
 
-// zf = 1 + 2 w lse folds the z-loss term into the softmax part.
-template <typename T>
-__device__ __forceinline__ void grad_element(const CeParams& p, float xo, float m, float inv_s,
-                                             float zf, float scale, int64_t idx, int64_t tgt,
-                                             float tcoeff, T& out) {
-  const float x = cap(p, xo);
-  float g = fast_exp(x - m) * inv_s * zf;
-  if (idx == tgt) g -= tcoeff;
-  if (p.use_ls) g -= p.ls_uniform;
-  if (p.use_softcap) {
-    const float t = x * p.inv_softcap;  // == tanh(logit / softcap)
-    g *= (1.0f - t * t);
+// What the gradient elements of one row share. zf = 1 + 2 w lse folds the
+// z-loss term into the softmax part.
+struct RowGrad {
+  float m, inv_s, zf, scale;
+  __device__ __forceinline__ RowGrad(const CeParams& p, float m_, float s) : m(m_) {
+    inv_s = 1.0f / s;
+    zf = p.zw2 != 0.0f ? fmaf(p.zw2, m + fast_log(s), 1.0f) : 1.0f;
+    scale = p.scale_dev ? p.scale * p.scale_dev[0] : p.scale;
   }
-  out = from_f32<T>(g * scale);
+};
+
+// Gradient of one element from its logit; CAP: the softcap is on.
+template <bool CAP>
+__device__ __forceinline__ float grad_value(const CeParams& p, const RowGrad& r, float xo, bool is_tgt) {
+  float th = 0.0f;
+  if constexpr (CAP) th = tanh_f32(xo * p.inv_softcap);
+  float g = fast_exp((CAP ? p.softcap * th : xo) - r.m) * r.inv_s * r.zf;
+  if (is_tgt) g -= p.tcoeff;
+  if (p.use_ls) g -= p.ls_uniform;
+  if constexpr (CAP) g *= 1.0f - th * th;
+  return g * r.scale;
 }
 
-// Writes the gradient row: zero for ignored rows, NaN for out-of-range
-// targets, otherwise the softmax gradient.
-template <typename T, bool VEC>
+// One vector of gradients; te: the target's place in it, or anything outside
+// [0, VE). Only the wave that holds the target compares element by element.
+template <typename T, bool CAP>
+__device__ __forceinline__ Vec16<T> grad_vec(const CeParams& p, const RowGrad& r, const Vec16<T>& xv, int te) {
+  constexpr int VE = Vec16<T>::VE;
+  Vec16<T> o;
+  if ((unsigned)te < (unsigned)VE) {
+#pragma unroll
+    for (int e = 0; e < VE; ++e) o.e[e] = from_f32<T>(grad_value<CAP>(p, r, to_f32(xv.e[e]), e == te));
+  } else {
+#pragma unroll
+    for (int e = 0; e < VE; ++e) o.e[e] = from_f32<T>(grad_value<CAP>(p, r, to_f32(xv.e[e]), false));
+  }
+  return o;
+}
+
+// Gradient of the row's elements [v0, v1) (vectors) and, where `ends` is set,
+// of the elements around the vectors: zero for ignored rows, NaN for
+// out-of-range targets, otherwise the softmax gradient. Four vectors of a
+// thread are loaded before the first is used.
+template <typename T, bool CAP>
 __device__ void write_grad_row(const CeParams& p, const T* __restrict__ row, T* __restrict__ grow,
                                int64_t vocab, int64_t tgt, bool ignored, bool bad, float m,
-                               float s) {
+                               float s, int64_t v0, int64_t v1, bool ends, int threads) {
   constexpr int VE = Vec16<T>::VE;
-  const float inv_s = 1.0f / s;
-  const float tcoeff = p.use_ls ? 1.0f - p.ls : 1.0f;
-  const float zf = p.zw2 != 0.0f ? fmaf(p.zw2, m + fast_log(s), 1.0f) : 1.0f;
-  const float scale = p.scale_dev ? p.scale * p.scale_dev[0] : p.scale;
-  if (VEC) {
-    const int64_t nvec = vocab / VE;
-    for (int64_t v = threadIdx.x; v < nvec; v += kCeThreads) {
-      Vec16<T> o;
-      if (ignored || bad) {
+  constexpr int U = 4;
+  const RowSplit<T, int64_t> sp(row, vocab);
+  const int t = threadIdx.x;
+  const int64_t ex = ends && t < sp.nx ? sp.extra(t) : -1;
+  row += sp.head;  // row / grow: the vectors' first element
+  T* const gv = grow + sp.head;
+  if (v1 > sp.nvec) v1 = sp.nvec;
+  if (ignored || bad) {
+    const T c = from_f32<T>(ignored ? 0.0f : NAN);
+    Vec16<T> o;
+#pragma unroll
+    for (int e = 0; e < VE; ++e) o.e[e] = c;
+    for (int64_t v = v0 + t; v < v1; v += threads) store16_any_nt(gv + v * VE, o);
+    if (ex >= 0) grow[ex] = c;
+    return;
+  }
+  const RowGrad r(p, m, s);
+  float xe = 0.0f;
+  if (ex >= 0) xe = to_f32(row[ex - sp.head]);
+  const int64_t tv = tgt - sp.head;  // relative to the vectors
+  int64_t v = v0 + t;
+  for (; v + (U - 1) * threads < v1; v += U * threads) {
+    Vec16<T> x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = load16_any_nt(row + (v + u * threads) * VE);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t at = (v + u * threads) * VE, d = tv - at;
+      store16_any_nt(gv + at, grad_vec<T, CAP>(p, r, x[u], d >= 0 && d < VE ? (int)d : -1));
+    }
+  }
+  for (; v < v1; v += threads) {
+    const int64_t d = tv - v * VE;
+    store16_any_nt(gv + v * VE, grad_vec<T, CAP>(p, r, load16_any_nt(row + v * VE), d >= 0 && d < VE ? (int)d : -1));
+  }
+  if (ex >= 0) grow[ex] = from_f32<T>(grad_value<CAP>(p, r, xe, ex == tgt));
+}
+
+// A row held in registers: TPR threads, VPT vectors each, packed between the
+// passes (max, sum, gradient) and converted again in each, plus the elements
+// around the vectors one to a thread. HBM-bound: 4 VPT registers hold the row,
+// so up to 8 vectors two 1024-thread workgroups fit a CU and one's loads and
+// stores run under the other's exponentials. [4096, 32768] bf16 with its
+// gradient 155 -> 115 us, 4.7 TB/s (256 threads streamed the row and read it
+// again for the gradient); [4096, 50257] fp16 without one 334 -> 74 us, 5.6 TB/s,
+// and the backward from saved statistics 315 -> 164 us (both had element
+// accesses).
+template <typename T, int VPT, int TPR, bool CAP>
+__global__ void __launch_bounds__(TPR, VPT == 8 ? 8 : 1)
+ce_row_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
+              float* __restrict__ losses, float* __restrict__ lse_out,
+              float* __restrict__ max_out, float* __restrict__ sum_out,
+              T* __restrict__ grad, int64_t rows, int vocab, int64_t ld, int64_t ld_g,
+              CeParams p) {
+  constexpr int VE = Vec16<T>::VE;
+  constexpr int W = TPR / 64;
+  __shared__ float part_m[W], part_s[W], part_x[W];
+  for (int64_t b = blockIdx.x; b < rows; b += gridDim.x) {
+    // The thread's index, opaque to the compiler in each pass: the VPT offsets
+    // and bounds derived from it would otherwise be held from pass to pass
+    // (and row to row) beside the row, and spill.
+    auto thread = [] {
+      int t = threadIdx.x;
+      asm volatile("" : "+v"(t));
+      return t;
+    };
+    int t = thread();
+    const T* row = logits + b * ld;
+    const RowSplit<T> sp(row, vocab);
+    const T* rv = row + sp.head;
+    const int64_t tgt = targets[b];
+    const bool ignored = tgt == p.ignore_index;
+    const bool bad = !ignored && (tgt < 0 || tgt >= vocab);
+    T xe = T(0.0f), xt = T(0.0f);  // this thread's single element, the target's logit
+    if (t < sp.nx) xe = row[sp.extra(t)];
+    if (t == 0 && !ignored && !bad) xt = row[tgt];
+    Vec16<T> raw[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      raw[k].u = u32x4{0, 0, 0, 0};
+      if (t + k * TPR < sp.nvec) raw[k] = load16_any_nt(rv + k * TPR * VE + (unsigned)(t * VE));
+    }
+
+    // max; the cap is monotonic, so the largest capped logit is the cap of the largest
+    t = thread();
+    float m = t < sp.nx ? to_f32(xe) : -INFINITY;
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      if (t + k * TPR < sp.nvec) {
+#pragma unroll
+        for (int e = 0; e < VE; ++e) m = fmaxf(m, to_f32(raw[k].e[e]));
+      }
+      keep_packed(raw[k]);
+    }
+    m = wave_max(m);
+    if ((t & 63) == 0) part_m[t / 64] = m;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < W; ++i) m = fmaxf(m, part_m[i]);
+    if constexpr (CAP) m = cap(p, m);
+
+    // sum of exp(x - m) (and of x); a row of -inf alone sums to 0, a NaN stays one
+    const float off = m == -INFINITY ? 0.0f : m;
+    float s = 0.0f, sx = 0.0f;
+    t = thread();
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      if (t + k * TPR < sp.nvec) {
+#pragma unroll
+        for (int e = 0; e < VE; ++e) {
+          const float x = CAP ? cap(p, to_f32(raw[k].e[e])) : to_f32(raw[k].e[e]);
+          s += fast_exp(x - off);
+          if (p.use_ls) sx += x;
+        }
+      }
+      keep_packed(raw[k]);
+    }
+    if (t < sp.nx) {
+      const float x = CAP ? cap(p, to_f32(xe)) : to_f32(xe);
+      s += fast_exp(x - off);
+      sx += x;
+    }
+    s = wave_sum(s);
+    if (p.use_ls) sx = wave_sum(sx);
+    if ((t & 63) == 0) {
+      part_s[t / 64] = s;
+      part_x[t / 64] = sx;
+    }
+    __syncthreads();  // part_m has been read by all, so the next row may write it
+    s = part_s[0];
+    sx = part_x[0];
+#pragma unroll
+    for (int i = 1; i < W; ++i) {
+      s += part_s[i];
+      sx += part_x[i];
+    }
+    if (s != s && m != INFINITY) m = NAN;  // the row holds a NaN
+
+    if (t == 0) {
+      const float lse = m + fast_log(s);
+      lse_out[b] = lse;
+      if (max_out) max_out[b] = m;
+      if (sum_out) sum_out[b] = s;
+      const float x = CAP ? cap(p, to_f32(xt)) : to_f32(xt);
+      float loss = p.use_ls ? lse - p.tcoeff * x - p.ls * (sx / p.vocab) : lse - x;
+      if (ignored) loss = 0.0f;
+      if (bad) loss = NAN;
+      losses[b] = loss;
+    }
+    if (grad) {
+      T* grow = grad + b * ld_g;
+      T* gv = grow + sp.head;
+      t = thread();
+      const int ex = t < sp.nx ? sp.extra(t) : -1;
+      if (!ignored && !bad) {
+        const RowGrad r(p, m, s);
+        const int tv = (int)tgt - sp.head;
+#pragma unroll
+        for (int k = 0; k < VPT; ++k)
+          if (t + k * TPR < sp.nvec)
+            store16_any_nt(gv + k * TPR * VE + (unsigned)(t * VE),
+                           grad_vec<T, CAP>(p, r, raw[k], tv - (t + k * TPR) * VE));
+        if (ex >= 0) grow[ex] = from_f32<T>(grad_value<CAP>(p, r, to_f32(xe), ex == (int)tgt));
+      } else {
+        Vec16<T> o;
 #pragma unroll
         for (int e = 0; e < VE; ++e) o.e[e] = from_f32<T>(ignored ? 0.0f : NAN);
-      } else {
-        Vec16<T> xv = load16(row + v * VE);
 #pragma unroll
-        for (int e = 0; e < VE; ++e)
-          grad_element<T>(p, to_f32(xv.e[e]), m, inv_s, zf, scale, v * VE + e, tgt, tcoeff, o.e[e]);
-      }
-      store16(grow + v * VE, o);
-    }
-  } else {
-    for (int64_t i = threadIdx.x; i < vocab; i += kCeThreads) {
-      if (ignored || bad) {
-        grow[i] = from_f32<T>(ignored ? 0.0f : NAN);
-      } else {
-        grad_element<T>(p, to_f32(row[i]), m, inv_s, zf, scale, i, tgt, tcoeff, grow[i]);
+        for (int k = 0; k < VPT; ++k)
+          if (t + k * TPR < sp.nvec) store16_any_nt(gv + k * TPR * VE + (unsigned)(t * VE), o);
+        if (ex >= 0) grow[ex] = o.e[0];
       }
     }
+    __syncthreads();  // part_s / part_x are rewritten for the workgroup's next row
   }
 }
 
@@ -191,7 +366,12 @@ __device__ void ce_fwd_row(const T* __restrict__ row, int64_t b, const int64_t* 
     }
     losses[b] = loss;
   }
-  if (grow) write_grad_row<T, VEC>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s);
+  if (grow) {
+    if (p.use_softcap)
+      write_grad_row<T, true>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s, 0, vocab, true, kCeThreads);
+    else
+      write_grad_row<T, false>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s, 0, vocab, true, kCeThreads);
+  }
 }
 
 // One 256-thread workgroup per row, rows by grid stride (the loop bound is
@@ -208,18 +388,21 @@ ce_fwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
                        grad ? grad + b * ld_g : nullptr, vocab, p);
 }
 
-template <typename T, bool VEC>
+// The gradient from the saved row statistics: blockIdx.y takes `span` vectors
+// of the row, so that few rows still fill the GPU.
+template <typename T, bool CAP>
 __global__ void __launch_bounds__(kCeThreads)
 ce_bwd_tiny_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
                    const float* __restrict__ row_max, const float* __restrict__ row_sum,
                    T* __restrict__ grad, int64_t rows, int64_t vocab, int64_t ld, int64_t ld_g,
-                   CeParams p) {
+                   int64_t span, CeParams p) {
+  const int64_t v0 = (int64_t)blockIdx.y * span;
   for (int64_t b = blockIdx.x; b < rows; b += gridDim.x) {
     const int64_t tgt = targets[b];
     const bool ignored = tgt == p.ignore_index;
     const bool bad = !ignored && (tgt < 0 || tgt >= vocab);
-    write_grad_row<T, VEC>(p, logits + b * ld, grad + b * ld_g, vocab, tgt, ignored, bad,
-                           row_max[b], row_sum[b]);
+    write_grad_row<T, CAP>(p, logits + b * ld, grad + b * ld_g, vocab, tgt, ignored, bad, row_max[b],
+                           row_sum[b], v0, v0 + span, blockIdx.y == 0, kCeThreads);
   }
 }
 
@@ -292,6 +475,8 @@ CeParams make_params(float softcap, int64_t ignore_index, float ls, float scale,
   p.use_ls = ls > 0.0f;
   p.ls = ls;
   p.ls_uniform = ls / (float)vocab;
+  p.tcoeff = p.use_ls ? 1.0f - ls : 1.0f;
+  p.vocab = (float)vocab;
   p.scale = scale;
   p.zw2 = 2.0f * zw;
   p.scale_dev = scale_dev;
@@ -313,12 +498,26 @@ int check(const void* logits, const int64_t* targets, void* grad, int64_t rows, 
   return AK_OK;
 }
 
-template <typename T>
-bool vec_ok(const void* logits, const void* grad, int64_t vocab, int64_t ld, int64_t ld_g) {
-  constexpr int VE = Vec16<T>::VE;
-  bool ok = vocab % VE == 0 && ld % VE == 0 && aligned16(logits);
-  if (grad) ok = ok && ld_g % VE == 0 && aligned16(grad);
-  return ok;
+// The row-resident forward with the fewest vectors a thread that its workgroup
+// sizes allow (256 threads up to 1024 vectors, for more rows in flight).
+template <typename T, bool CAP>
+bool launch_row(const T* lg, const int64_t* targets, float* losses, float* lse, float* mx,
+                float* sm, T* g, int64_t rows, int64_t vocab, int64_t ld, int64_t ld_g,
+                const CeParams& p, hipStream_t s) {
+  const int64_t nvec = vocab / Vec16<T>::VE;
+  if (nvec > 16384) return false;
+#define AK_LAUNCH(VPT, TPR)                                                                   \
+  ce_row_kernel<T, VPT, TPR, CAP><<<dim3(row_grid(rows)), dim3(TPR), 0, s>>>(                 \
+      lg, targets, losses, lse, mx, sm, g, rows, (int)vocab, ld, ld_g, p)
+  if (nvec <= 256) AK_LAUNCH(1, 256);
+  else if (nvec <= 512) AK_LAUNCH(2, 256);
+  else if (nvec <= 1024) AK_LAUNCH(4, 256);
+  else if (nvec <= 2048) AK_LAUNCH(4, 512);
+  else if (nvec <= 4096) AK_LAUNCH(4, 1024);
+  else if (nvec <= 8192) AK_LAUNCH(8, 1024);
+  else AK_LAUNCH(16, 1024);
+#undef AK_LAUNCH
+  return true;
 }
 
 template <typename T>
@@ -327,8 +526,13 @@ void launch_fwd(const void* logits, const int64_t* targets, float* losses, float
                 const CeParams& p, hipStream_t s) {
   const T* lg = static_cast<const T*>(logits);
   T* g = static_cast<T*>(grad);
+  const bool done = p.use_softcap
+      ? launch_row<T, true>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, s)
+      : launch_row<T, false>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, s);
+  if (done) return;
+  constexpr int VE = Vec16<T>::VE;
   const dim3 grid(row_grid(rows)), block(kCeThreads);
-  if (vec_ok<T>(logits, grad, vocab, ld, ld_g))
+  if (vocab % VE == 0 && ld % VE == 0 && aligned16(logits))
     ce_fwd_kernel<T, true><<<grid, block, 0, s>>>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p);
   else
     ce_fwd_kernel<T, false><<<grid, block, 0, s>>>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p);
@@ -340,11 +544,16 @@ void launch_bwd(const void* logits, const int64_t* targets, const float* mx, con
                 const CeParams& p, hipStream_t s) {
   const T* lg = static_cast<const T*>(logits);
   T* g = static_cast<T*>(grad);
-  const dim3 grid(row_grid(rows)), block(kCeThreads);
-  if (vec_ok<T>(logits, grad, vocab, ld, ld_g))
-    ce_bwd_tiny_kernel<T, true><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, vocab, ld, ld_g, p);
+  // workgroups of one round of 4 vectors a thread where the row is that wide:
+  // [4096, 50257] fp16 takes 164 us so and 179 us with one workgroup a row
+  const int64_t nvec = vocab / Vec16<T>::VE;
+  const int64_t ny = std::min<int64_t>(nvec / (4 * kCeThreads), 65535);
+  const int64_t span = ny > 1 ? (nvec + ny - 1) / ny : nvec;
+  const dim3 grid(row_grid(rows), ny > 1 ? (unsigned)ny : 1), block(kCeThreads);
+  if (p.use_softcap)
+    ce_bwd_tiny_kernel<T, true><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, vocab, ld, ld_g, span, p);
   else
-    ce_bwd_tiny_kernel<T, false><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, vocab, ld, ld_g, p);
+    ce_bwd_tiny_kernel<T, false><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, vocab, ld, ld_g, span, p);
 }
 
 }  // namespace

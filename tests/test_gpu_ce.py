@@ -199,3 +199,51 @@ def test_ce_fused_backward_scales_on_device(up):
                 0.0, -100, 0.0, 1.0, scale_dev=denom[1:])
     want = gref if up == 1.0 else gref * torch.tensor(up, device=DEV).bfloat16()
     assert torch.equal(x.grad, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vecs,over", [(0, 3), (1, 1), (256, 3), (257, 0), (512, 1), (1024, 2), (2048, 3), (4096, 1),
+                                       (4097, 3), (8193, 0), (16384, 3), (16385, 1), (16385, 0)])
+def test_ce_rows_at_any_address(dtype, vecs, over):
+    """Ragged rows at the edges of every vectors-per-thread variant and past
+    them (``vecs`` 16-byte vectors plus ``over`` elements), logits and gradients
+    in pitched views that start off the 16-byte grid, not always the same way;
+    targets in the first and last element, beside the vectors' ends, ignored
+    and out of range; rows of -inf, with a NaN and of the type's lowest value.
+    The elements around the gradient rows keep their values."""
+    need_gpu()
+    from kernels.hip import _lib
+    ve = 16 // torch.empty((), dtype=dtype).element_size()
+    vocab, rows = max(1, vecs * ve + over), 9
+    g = torch.Generator().manual_seed(vocab)
+    x = (3 * torch.randn(rows, vocab, generator=g)).to(dtype)
+    ends = [0, vocab - 1, min(ve, vocab - 1), max(0, vocab - ve), vocab // 2]
+    t = torch.tensor(ends + [-100, vocab, 0, 0])
+    x[6] = torch.finfo(dtype).min
+    x[7], x[8, vocab // 2] = float("-inf"), float("nan")
+    for softcap, ls, ox, og in ((0.0, 0.0, 0, 0), (0.0, 0.1, 1, 1), (20.0, 0.0, 3, 1)):
+        say("ce any address", dtype, vocab, softcap, ls, ox, og)
+        xb = torch.zeros(rows, vocab + 5, dtype=dtype)
+        xb[:, ox:ox + vocab] = x
+        xv = xb.to(DEV)[:, ox:ox + vocab]
+        td = t.to(DEV)
+        f32 = [torch.full((rows,), 7.0, device=DEV) for _ in range(4)]
+        gb = [torch.full((rows, vocab + 4), 7.0, dtype=dtype, device=DEV) for _ in range(2)]
+        gv = [b[:, og:og + vocab] for b in gb]
+        _lib.ce_fwd(xv, td, *f32, gv[0], softcap, -100, ls, 0.5, z_loss_weight=1e-3)
+        _lib.ce_bwd_tiny(xv, td, f32[2], f32[3], gv[1], softcap, -100, ls, 0.5, z_loss_weight=1e-3)
+        losses, lse, mx, sm = (v.cpu() for v in f32)
+        good = [0, 1, 2, 3, 4]
+        rl, rlse, rmx, rsm = ops.ce_rows_ref(x[good + [5]], t[good + [5]], softcap, -100, ls)
+        assert _close(losses[good + [5]], rl) and _close(lse[good + [5]], rlse)
+        assert _close(mx[good + [5]], rmx, 1e-6, 1e-6) and _close(sm[good + [5]], rsm)
+        want = ops.ce_grad_ref(x[good + [5]], t[good + [5]], softcap, -100, ls, 0.5, 1e-3)
+        for b, v in zip(gb, gv):
+            b, v = b.cpu(), v.cpu()
+            assert bool((b[:, :og] == 7).all()) and bool((b[:, og + vocab:] == 7).all())
+            ok, worst = _grad_ok(v[good + [5]], want, dtype)
+            assert ok, worst
+            assert bool(torch.isnan(v[[6, 8]]).all())  # out of range, and a NaN in the row
+        assert math.isnan(losses[6]) and math.isnan(losses[8]) and math.isnan(lse[8])
+        if softcap == 0.0:  # a row of -inf alone
+            assert lse[7] == float("-inf") and mx[7] == float("-inf") and sm[7] == 0
