@@ -466,6 +466,35 @@ ce_mean_kernel(const float* __restrict__ losses, const float* __restrict__ lse,
   }
 }
 
+// x *= round_T(scale[0]), each product rounded once. A scale of exactly 1 (the
+// plain loss.backward()) costs one scalar read instead of a pass over x, the
+// bits being those of the product either way.
+template <typename T>
+__global__ void __launch_bounds__(kCeThreads)
+scale_kernel(T* __restrict__ x, int64_t n, const float* __restrict__ scale) {
+  const float g = to_f32(from_f32<T>(scale[0]));
+  if (g == 1.0f) return;
+  constexpr int VE = Vec16<T>::VE;
+  const RowSplit<T, int64_t> sp(x, n);
+  const int64_t at = (int64_t)blockIdx.x * kCeThreads + threadIdx.x;
+  T* const xv = x + sp.head;
+  for (int64_t v = at; v < sp.nvec; v += (int64_t)gridDim.x * kCeThreads) {
+    Vec16<T> a = load16(xv + v * VE);
+#pragma unroll
+    for (int e = 0; e < VE; ++e) a.e[e] = from_f32<T>(to_f32(a.e[e]) * g);
+    store16(xv + v * VE, a);
+  }
+  if (at < sp.nx) x[sp.extra((int)at)] = from_f32<T>(to_f32(x[sp.extra((int)at)]) * g);
+}
+
+template <typename T>
+void launch_scale(void* x, int64_t n, const float* scale, hipStream_t s) {
+  // 8 workgroups a CU: few enough that the launch of a scale of 1 stays cheap
+  const int64_t units = (n / Vec16<T>::VE + kCeThreads - 1) / kCeThreads;
+  const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(units, 2048));
+  scale_kernel<T><<<dim3(grid), dim3(kCeThreads), 0, s>>>(static_cast<T*>(x), n, scale);
+}
+
 CeParams make_params(float softcap, int64_t ignore_index, float ls, float scale, int64_t vocab,
                      float zw = 0.0f, const float* scale_dev = nullptr) {
   CeParams p;
@@ -624,5 +653,22 @@ extern "C" int ak_ce_mean(const float* losses, const float* lse, const int64_t* 
     return ak_set_error(AK_ERR_INVALID_ARG, "%s: null pointer", name);
   ak::ce_mean_kernel<<<dim3(1), dim3(ak::kCeReduceThreads), 0, ak_stream(stream)>>>(
       losses, lse, targets, rows, ignore_index, z_loss_weight, loss, n_valid);
+  return ak_check_launch(name);
+}
+
+extern "C" int ak_scale_inplace(void* x, int64_t n, const float* scale, int dtype, void* stream) {
+  const char* name = "ak_scale_inplace";
+  const int esz = ak_dtype_size(dtype);
+  if (esz == 0) return ak_set_error(AK_ERR_UNSUPPORTED, "%s: unsupported dtype code %d", name, dtype);
+  if (n < 0 || n > INT64_MAX / esz) return ak_set_error(AK_ERR_INVALID_ARG, "%s: bad element count", name);
+  if (n == 0) return AK_OK;
+  if (!x || !scale) return ak_set_error(AK_ERR_INVALID_ARG, "%s: null pointer", name);
+  if (reinterpret_cast<uintptr_t>(x) % esz) return ak_set_error(AK_ERR_INVALID_ARG, "%s: misaligned x", name);
+  hipStream_t s = ak_stream(stream);
+  switch (dtype) {
+    case AK_DTYPE_F32: ak::launch_scale<float>(x, n, scale, s); break;
+    case AK_DTYPE_F16: ak::launch_scale<ak::f16>(x, n, scale, s); break;
+    default: ak::launch_scale<ak::bf16>(x, n, scale, s); break;
+  }
   return ak_check_launch(name);
 }

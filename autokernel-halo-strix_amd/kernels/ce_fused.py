@@ -132,6 +132,21 @@ def _get_bwd_module():
     return _bwd_module
 
 
+# Saved-tensor hooks in force (torch's own query; where it is missing, taken to be).
+_top_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", lambda _: True)
+
+
+def _native(logits, targets, softcap, ignore_index, label_smoothing, fused, z_loss_weight):
+    """``(loss, lse)`` of a plain call through the native host side, else None.
+    With no saved-tensor hooks in force nobody but the graph holds the fused
+    gradient, and its last backward may scale it in place."""
+    host = _lib.native(logits, targets)
+    if host is None:
+        return None
+    return host.ce_full(logits, targets, softcap, _NO_IGNORE if ignore_index is None else ignore_index,
+                        label_smoothing, fused, z_loss_weight, _top_hooks(False) is None)
+
+
 class _CrossEntropyHIP(torch.autograd.Function):
     """Mean CE over the counted rows, with the gradient either written by the
     forward (``mode="fused"``) or recomputed from the saved row statistics
@@ -196,6 +211,9 @@ class _CrossEntropyHIP(torch.autograd.Function):
 
 def kernel_fn(logits: torch.Tensor, targets: torch.Tensor) -> torch.Tensor:
     """Mean cross-entropy; matches ``reference.cross_entropy_ref`` (ignore_index -100)."""
+    pair = _native(logits, targets, 0.0, -100, 0.0, True, 0.0)
+    if pair is not None:
+        return pair[0]
     if logits.requires_grad and torch.is_grad_enabled():
         return _CrossEntropyHIP.apply(logits, targets, 0.0, -100, 0.0, "fused", False, 0.0)
     rows2d, tg = _row_problem(logits, targets)
@@ -214,5 +232,9 @@ def ce_full(logits: torch.Tensor, targets: torch.Tensor, *, softcap: float = 0.0
     _lib.require_device(logits, targets)
     if mode not in ("fused", "tiny"):
         raise ValueError(f"mode must be 'fused' or 'tiny', got {mode!r}")
+    pair = _native(logits, targets, softcap, ignore_index, label_smoothing, mode == "fused",
+                   float(z_loss_weight))
+    if pair is not None:
+        return pair if return_z else pair[0]
     return _CrossEntropyHIP.apply(logits, targets, softcap, ignore_index, label_smoothing, mode,
                                   return_z, float(z_loss_weight))

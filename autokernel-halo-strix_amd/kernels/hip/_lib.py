@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.util
 import os
 import threading
 from typing import Optional
@@ -63,6 +64,7 @@ _SIGNATURES = {
     "ak_ce_count_valid": [_c_void_p, _i64, _i64, _c_void_p, _c_void_p],
     "ak_ce_mean": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _f32, _c_void_p, _c_void_p,
                    _c_void_p],
+    "ak_scale_inplace": [_c_void_p, _i64, _c_void_p, _int, _c_void_p],
     "ak_lmhead_ce_workspace_bytes": [_i64, _i64],
     "ak_lmhead_ce_fwd": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                          _c_void_p, ctypes.c_size_t, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32,
@@ -95,6 +97,7 @@ _RESTYPES = {
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lock = threading.Lock()
+_is_compiling = torch.compiler.is_compiling
 _lib: Optional[ctypes.CDLL] = None
 
 
@@ -125,6 +128,39 @@ def load() -> ctypes.CDLL:
                 fn.restype = _RESTYPES.get(name, ctypes.c_int)
             _lib = handle
     return _lib
+
+
+HOST_PATH = os.path.join(os.path.dirname(LIB_PATH), "_host_ops.so")
+_host = None
+
+
+def host():
+    """The native host side (``csrc/host_ops.cpp``), opened once: functions that
+    check, allocate and launch a plain call of an entry point in one step, with
+    its autograd node, and return None for any other call."""
+    global _host
+    if _host is None:
+        load()
+        with _lock:
+            if _host is None:
+                if not os.path.exists(HOST_PATH):
+                    raise HipExtensionMissing(f"{HOST_PATH} is missing: build it with `make -C {CSRC_DIR}`")
+                spec = importlib.util.spec_from_file_location("_host_ops", HOST_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                module.init(lib_path())
+                _host = module
+    return _host
+
+
+def native(*tensors):
+    """:func:`host` where a call on these tensors may be its, else None: GPU
+    tensors, and not while torch.compile traces the call (the Python forms below
+    it are the traced ones)."""
+    for t in tensors:
+        if not (isinstance(t, torch.Tensor) and t.is_cuda):
+            return None
+    return None if _is_compiling() else (_host or host())
 
 
 def is_available() -> bool:
@@ -396,6 +432,17 @@ def ce_mean(losses: torch.Tensor, lse: Optional[torch.Tensor], targets: torch.Te
                                _ptr(n_valid), _stream(losses))
     _check(rc, "ak_ce_mean")
     return loss
+
+
+def scale_inplace(x: torch.Tensor, scale: torch.Tensor) -> None:
+    """``x *= scale`` for a contiguous ``x`` and a 1-element fp32 device ``scale``
+    (rounded to x's dtype first); a scale of 1 leaves x unread."""
+    require_device(x, scale)
+    if not x.is_contiguous() or scale.dtype != torch.float32 or scale.numel() != 1:
+        raise ValueError("scale_inplace needs a contiguous x and a 1-element fp32 scale")
+    with _on_device(x):
+        rc = load().ak_scale_inplace(_ptr(x), x.numel(), _ptr(scale), dtype_code(x.dtype), _stream(x))
+    _check(rc, "ak_scale_inplace")
 
 
 def lmhead_ce_workspace_bytes(n_rows: int, vocab: int) -> int:

@@ -30,9 +30,12 @@ kernels.
 """
 
 import os
+from types import SimpleNamespace
 from typing import Tuple
 
 import torch
+
+from kernels.hip import _lib
 
 # Environment switch: AUTOKERNEL_NO_BWD_HIP=1 makes the backwards use the
 # fp32 PyTorch formulas below instead of the gfx950 backward kernels (the
@@ -57,6 +60,8 @@ def disable_hip_backward():
     """Use the PyTorch formulas for every backward from now on."""
     global _BWD_KERNELS_ENABLED
     _BWD_KERNELS_ENABLED = False
+    if _lib._host is not None:
+        _lib._host.set_hip_backward(False)
 
 
 def _register_autocast(op) -> None:
@@ -72,6 +77,58 @@ def _register_autocast(op) -> None:
             return op._opoverload(*cast)
 
     op._lib.impl(op._name, kernel, "AutocastCUDA", with_keyset=True)
+
+
+def _register_native(op, entry: str, defaults: tuple, setup, backward) -> None:
+    """AutogradCUDA rule: a plain call goes to the native host side, which
+    launches the kernel and records its own autograd node in one step (the
+    dispatcher's Python route costs 30-60 us a call). Every other call (fake,
+    functional or wrapped tensors, tracing, conversions, errors) records
+    ``backward`` on the op's general kernel, as ``register_autograd`` does."""
+
+    class General(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, *args):
+            with torch._C._AutoDispatchBelowAutograd():
+                out = op._opoverload(*args)
+            setup(ctx, args, out)
+            ctx.set_materialize_grads(False)
+            return out
+
+        @staticmethod
+        def backward(ctx, *grads):
+            return backward(ctx, *grads)
+
+    def formula(args, eps):
+        saved = args[:len(args) - grads_of]
+        return backward(SimpleNamespace(saved_tensors=saved + (None,) * (entry == "diag_scan_op"), eps=eps),
+                        *args[len(args) - grads_of:])
+
+    grads_of = 2 if entry == "add_rmsnorm_op" else 1
+    ready = []
+
+    def native(args):
+        if not _BWD_KERNELS_ENABLED or _is_compiling():
+            return None
+        host = _lib.native(*(a for a in args if isinstance(a, torch.Tensor)))
+        if host is None:
+            return None
+        if not ready:
+            host.set_formula(op._name, formula)
+            ready.append(True)
+        return getattr(host, entry)(*args)
+
+    def kernel(_, *args):
+        args = args + defaults[len(args) - (len(op._opoverload._schema.arguments) - len(defaults)):]
+        out = native(args)
+        if out is not None:
+            return out
+        if torch.is_grad_enabled() and any(isinstance(a, torch.Tensor) and a.requires_grad for a in args):
+            return General.apply(*args)
+        with torch._C._AutoDispatchBelowAutograd():
+            return op._opoverload(*args)
+
+    op._lib.impl(op._name, kernel, "AutogradCUDA", with_keyset=True)
 
 
 # ---------------------------------------------------------------------------
@@ -119,6 +176,7 @@ def _rmsnorm_backward(ctx, grad_output):
 
 rmsnorm_op.register_autograd(_rmsnorm_backward, setup_context=_rmsnorm_setup)
 _register_autocast(rmsnorm_op)
+_register_native(rmsnorm_op, "rmsnorm_op", (RMSNORM_EPS,), _rmsnorm_setup, _rmsnorm_backward)
 
 
 # ---------------------------------------------------------------------------
@@ -172,6 +230,8 @@ def _fused_res_rmsnorm_backward(ctx, grad_hidden, grad_normed):
 fused_res_rmsnorm_op.register_autograd(_fused_res_rmsnorm_backward,
                                        setup_context=_fused_res_rmsnorm_setup)
 _register_autocast(fused_res_rmsnorm_op)
+_register_native(fused_res_rmsnorm_op, "add_rmsnorm_op", (RMSNORM_EPS,), _fused_res_rmsnorm_setup,
+                 _fused_res_rmsnorm_backward)
 
 
 # ---------------------------------------------------------------------------
@@ -224,3 +284,4 @@ def _selective_scan_backward(ctx, grad_y):
 
 
 selective_scan_op.register_autograd(_selective_scan_backward, setup_context=_selective_scan_setup)
+_register_native(selective_scan_op, "diag_scan_op", (), _selective_scan_setup, _selective_scan_backward)

@@ -353,6 +353,13 @@ class ChunkedLinearCrossEntropyLoss(nn.Module):
         _lib.require_device(hidden, weight, targets)
         if weight.dtype != hidden.dtype:
             weight = weight.to(hidden.dtype)
+        if not self.z_loss_weight > 0 and _fused_ok(hidden, weight, self.softcap, self.label_smoothing):
+            host = _lib.native(hidden, weight, targets)
+            if host is not None:
+                loss = host.lmhead_ce(hidden, weight, targets, self.ignore_index, self.softcap,
+                                      self.label_smoothing, GRAD_LOGITS_BUDGET)
+                if loss is not None:
+                    return loss
         return _ChunkedLinearCrossEntropy.apply(
             hidden, weight, targets, self.chunk_size, self.softcap, self.ignore_index,
             self.label_smoothing, self.z_loss_weight)

@@ -49,6 +49,11 @@ def _prepare(x, residual, weight):
 def kernel_fn(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
               eps: float = DEFAULT_EPS) -> torch.Tensor:
     """RMSNorm(x + residual) * weight; matches ``reference.fused_residual_add_rmsnorm_ref``."""
+    host = _lib.native(x, residual, weight)
+    if host is not None:
+        y = host.add_rmsnorm(x, residual, weight, eps)
+        if y is not None:
+            return y
     x2, r2, w = _prepare(x, residual, weight)
     y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     if y.numel():
@@ -59,6 +64,11 @@ def kernel_fn(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
 def kernel_fn_dual(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                    eps: float = DEFAULT_EPS) -> tuple:
     """Returns ``(hidden, normed)`` with ``hidden = x + residual``."""
+    host = _lib.native(x, residual, weight)
+    if host is not None:
+        pair = host.add_rmsnorm_dual(x, residual, weight, eps)
+        if pair is not None:
+            return pair
     x2, r2, w = _prepare(x, residual, weight)
     hidden = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     normed = torch.empty(x.shape, dtype=x.dtype, device=x.device)

@@ -93,6 +93,11 @@ def _checkpoint_bytes(u: torch.Tensor, A: torch.Tensor) -> int:
 def kernel_fn(dA: torch.Tensor, dBx: torch.Tensor, C: torch.Tensor, D: torch.Tensor,
               x: torch.Tensor) -> torch.Tensor:
     """Diagonal SSM scan over ``[batch, seq, d_inner]`` fp32 tensors."""
+    host = _lib.native(dA, dBx, C, D, x)
+    if host is not None:
+        y = host.diag_scan(dA, dBx, C, D, x)
+        if y is not None:
+            return y
     _lib.require_device(dA, dBx, C, D, x)
     if dA.dtype != torch.float32:
         raise TypeError("dA must be float32")
@@ -304,5 +309,12 @@ class SelectiveScanFn(torch.autograd.Function):
 def selective_scan_fn(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta_softplus=False,
                       return_last_state=False):
     """Mamba-1 selective scan. Returns ``out`` or ``(out, last_state)``."""
+    host = _lib.native(u, delta, A, B, C)
+    if host is not None:
+        res = host.selective_scan(u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus),
+                                  bool(return_last_state), SAVE_STATES,
+                                  -1.0 if SAVE_STATES_MAX_BYTES is None else SAVE_STATES_MAX_BYTES)
+        if res is not None:
+            return tuple(res) if return_last_state else res[0]
     return SelectiveScanFn.apply(u, delta, A, B, C, D, z, delta_bias, delta_softplus,
                                  return_last_state, torch.is_grad_enabled())

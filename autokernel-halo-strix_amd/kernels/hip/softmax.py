@@ -29,6 +29,11 @@ HIP_SRC = os.path.join(_lib.CSRC_DIR, "softmax.hip")
 
 def kernel_fn(x: torch.Tensor) -> torch.Tensor:
     """Softmax over the last dimension of ``x`` (any rank)."""
+    host = _lib.native(x)
+    if host is not None:
+        y = host.softmax(x)
+        if y is not None:
+            return y
     _lib.require_device(x)
     _lib.dtype_code(x.dtype)
     shape = x.shape

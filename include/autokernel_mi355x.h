@@ -217,6 +217,13 @@ int ak_ce_mean(const float* losses, const float* lse, const int64_t* targets,
                float* loss, int64_t* n_valid, void* stream);
 
 /*
+ * x[i] *= round_T(scale[0]) over n contiguous elements, scale fp32 on the
+ * device; a scale of exactly 1 returns without touching x. Replaces the
+ * host-side grad_output.item() and multiply of kernels/ce_fused.py:640-650.
+ */
+int ak_scale_inplace(void* x, int64_t n, const float* scale, int dtype, void* stream);
+
+/*
  * Fused lm-head + cross-entropy forward: logits = hidden @ weight^T are
  * produced tile by tile on the matrix cores and folded into an online
  * logsumexp; they are never written to memory.

@@ -247,3 +247,54 @@ def test_ce_rows_at_any_address(dtype, vecs, over):
         assert math.isnan(losses[6]) and math.isnan(losses[8]) and math.isnan(lse[8])
         if softcap == 0.0:  # a row of -inf alone
             assert lse[7] == float("-inf") and mx[7] == float("-inf") and sm[7] == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_scale_inplace(dtype):
+    """x *= scale from device memory at any address and length: torch's product
+    bit for bit, the neighbours untouched; a scale of 1 changes nothing."""
+    need_gpu()
+    from kernels.hip import _lib
+    g = torch.Generator().manual_seed(4)
+    for n, off in ((1, 0), (7, 1), (8, 3), (4099, 1), (2048 * 256 * 8 * 2 + 5, 1)):
+        say("scale_inplace", dtype, n, off)
+        base = torch.randn(n + off + 3, generator=g).to(dtype).to(DEV)
+        for scale in (1.0, 0.7, -3.0, float("inf")):
+            b = base.clone()
+            sd = torch.tensor([scale], device=DEV)
+            _lib.scale_inplace(b[off:off + n], sd)
+            want = base[off:off + n] * sd.to(dtype)
+            assert torch.equal(b[off:off + n].nan_to_num(7), want.nan_to_num(7))
+            assert torch.equal(b[:off], base[:off]) and torch.equal(b[off + n:], base[off + n:])
+
+
+def test_ce_fused_backward_kept_graphs_and_hooks():
+    """The fused gradient is scaled in place only where nobody can ask for it
+    again: a kept graph's backwards, a backward after one, and saved-tensor
+    hooks that hold the saved tensors all see the gradient the forward wrote."""
+    need_gpu()
+    from kernels.ce_fused import ce_full
+    g = torch.Generator().manual_seed(35)
+    base = (2 * torch.randn(64, 3001, generator=g)).bfloat16().to(DEV)
+    t = torch.randint(0, 3001, (64,), generator=g).to(DEV)
+
+    def once(up, x):
+        return torch.autograd.grad(ce_full(x, t, mode="fused"), x, up)[0]
+
+    one, two = torch.tensor(1.0, device=DEV), torch.tensor(2.0, device=DEV)
+    x = base.clone().requires_grad_()
+    say("ce fused kept graph")
+    want = once(one, x)
+    assert torch.equal(once(two, x), want * 2)
+    loss = ce_full(x, t, mode="fused")
+    first = torch.autograd.grad(loss, x, two, retain_graph=True)[0]
+    second = torch.autograd.grad(loss, x, one, retain_graph=True)[0]
+    last = torch.autograd.grad(loss, x, two)[0]
+    assert torch.equal(first, want * 2) and torch.equal(second, want) and torch.equal(last, want * 2)
+
+    say("ce fused saved-tensor hooks")
+    held = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda v: held.append(v) or len(held) - 1, lambda i: held[i]):
+        loss = ce_full(x, t, mode="fused")
+    assert torch.equal(torch.autograd.grad(loss, x, two)[0], want * 2)
+    assert torch.equal(held[0], want)
