@@ -93,6 +93,13 @@ __device__ __forceinline__ Vec16<T> load16_any_nt(const T* p) {
 }
 
 template <typename T>
+__device__ __forceinline__ Vec16<T> load16_any(const T* p) {
+  Vec16<T> v;
+  v.u = *reinterpret_cast<const u32x4_any*>(p);
+  return v;
+}
+
+template <typename T>
 __device__ __forceinline__ void store16_any_nt(T* p, const Vec16<T>& v) {
   __builtin_nontemporal_store(v.u, reinterpret_cast<u32x4_any*>(p));
 }

@@ -5,13 +5,13 @@
 // training step's loss over 64 x 512 logits takes 115 us through Python and
 // ctypes, 61 us through these functions, and has about 20 us of kernels; an
 // inference scan 21 and 5 us, a norm's forward and backward 250 and 43-90 us,
-// since a backward in Python also waits for autograd's thread). Every function here takes the plain form of one entry
-// point (dense tensors of the kernels' types on the current GPU) and returns
-// nothing for any other form, or when something that wants to see the single
-// steps is in force (a dispatch or function mode, a functorch transform): the
-// Python code then takes the call, with its conversions and its errors. The
-// kernels come from the C library, whose path the loader passes in, so there is
-// one copy of them in the process.
+// since a backward in Python also waits for autograd's thread). Every function
+// here takes the plain form of one entry point (dense tensors of the kernels'
+// types on the current GPU) and returns nothing for any other form, or when
+// something that wants to see the single steps is in force (a dispatch or
+// function mode, a functorch transform): the Python code then takes the call,
+// with its conversions and its errors. The kernels come from the C library,
+// whose path the loader passes in, so there is one copy of them in the process.
 #include <dlfcn.h>
 
 #include <c10/hip/HIPStream.h>
@@ -30,7 +30,7 @@ using Maybe = std::optional<Tensor>;
 
 #define AK_ENTRIES(X)                                                                              \
   X(ak_last_error) X(ak_rmsnorm_fwd) X(ak_fused_add_rmsnorm_fwd) X(ak_rmsnorm_bwd_workspace_bytes) \
-  X(ak_fused_add_rmsnorm_bwd) X(ak_rmsnorm_bwd) X(ak_softmax_fwd) X(ak_ce_fwd) X(ak_ce_bwd_tiny)   \
+  X(ak_fused_add_rmsnorm_bwd_gw) X(ak_softmax_fwd) X(ak_ce_fwd) X(ak_ce_bwd_tiny)   \
   X(ak_ce_count_valid) X(ak_ce_mean) X(ak_scale_inplace) X(ak_diag_scan_fwd)                       \
   X(ak_diag_scan_bwd_workspace_bytes) X(ak_diag_scan_bwd) X(ak_selective_scan_fwd)                 \
   X(ak_selective_scan_bwd_workspace_bytes) X(ak_selective_scan_bwd)                                \
@@ -183,13 +183,13 @@ std::pair<Tensor, Tensor> norm_backward(const Tensor& h, const Tensor& w, const 
   int64_t ld_y = cols, ld_h = cols;
   Tensor y = rows_of(gy.to(h.scalar_type()), cols, ld_y), g;
   if (gh.defined()) g = rows_of(gh.to(h.scalar_type()), cols, ld_h);
-  Tensor gx = at::empty(h.sizes(), h.options()), gw = f32_like(h, {cols});
+  Tensor gx = at::empty(h.sizes(), h.options()), gw = at::empty({cols}, w.options());
   const size_t bytes = api.ak_rmsnorm_bwd_workspace_bytes(rows, cols);
   Tensor ws = bytes_like(h, bytes);
-  check(api.ak_fused_add_rmsnorm_bwd(h.data_ptr(), w.data_ptr(), ptr(g), y.data_ptr(), gx.data_ptr(), f32p(gw),
-                                     ws.data_ptr(), bytes, rows, cols, cols, ld_h, ld_y, cols, (float)eps,
-                                     code_of(h.scalar_type()), stream_of(h)), "ak_fused_add_rmsnorm_bwd");
-  return {gx, gw.to(w.scalar_type())};
+  check(api.ak_fused_add_rmsnorm_bwd_gw(h.data_ptr(), w.data_ptr(), ptr(g), y.data_ptr(), gx.data_ptr(), gw.data_ptr(),
+                                        ws.data_ptr(), bytes, rows, cols, cols, ld_h, ld_y, cols, (float)eps,
+                                        code_of(h.scalar_type()), stream_of(h)), "ak_fused_add_rmsnorm_bwd_gw");
+  return {gx, gw};
 }
 
 struct RmsNorm : torch::autograd::Function<RmsNorm> {

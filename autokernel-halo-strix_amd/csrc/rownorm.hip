@@ -1,7 +1,7 @@
 // RMSNorm and fused residual-add + RMSNorm for gfx950.
 //
-// Row-parallel, HBM-bound. A row is owned by 64..1024 threads holding one
-// 16-byte vector each (up to 8 for rows over 1024 vectors). Each thread keeps
+// Row-parallel, HBM-bound. A row is owned by 64..1024 threads holding one or
+// two 16-byte vectors each (up to 8 for rows over 2048 vectors). Each thread keeps
 // its slice of the row in registers as fp32 between the sum-of-squares
 // reduction and the normalise pass, so x and residual are read from HBM
 // exactly once and new_residual / y written exactly once, with nontemporal
@@ -20,8 +20,11 @@ namespace {
 // workgroup when TPR < 256). The workgroup walks rows with a grid stride so
 // the grid can be sized to the machine; the loop bound is uniform per
 // workgroup, so the barrier of the multi-wave reduction is always reached by
-// every wave. NT selects nontemporal (streaming) global loads and stores.
-template <typename T, bool RES, int VPT, int TPR, bool NT>
+// every wave. RAG: rows at any address and of any width; the vectors start at
+// x's first 16-byte boundary, whatever the alignment of the other rows there,
+// and the few elements around them go one to a thread ([16384, 4097] bf16 in
+// whole vectors 55.7 us, 4.8 TB/s; fused [16384, 2049] 49.7 us, 5.4 TB/s).
+template <typename T, bool RES, int VPT, int TPR, bool RAG>
 __global__ void __launch_bounds__(TPR >= 256 ? TPR : 256)
 rownorm_vec_kernel(const T* __restrict__ x, const T* __restrict__ r,
                    const T* __restrict__ w, T* __restrict__ nr, T* __restrict__ y,
@@ -35,25 +38,34 @@ rownorm_vec_kernel(const T* __restrict__ x, const T* __restrict__ r,
 
   const int t = threadIdx.x % TPR;
   const int rl = threadIdx.x / TPR;
-  const int nvec = cols / VE;
-  auto ld = [](const T* p) { return NT ? load16_nt(p) : load16(p); };
+  auto ld = [](const T* p) { return RAG ? load16_any_nt(p) : load16_nt(p); };
   auto st = [](T* p, const Vec16<T>& v) {
-    if (NT) store16_nt(p, v);
-    else store16(p, v);
+    if (RAG) store16_any_nt(p, v);
+    else store16_nt(p, v);
   };
 
   for (int64_t base = (int64_t)blockIdx.x * RPW; base < rows; base += (int64_t)gridDim.x * RPW) {
     const int64_t row = base + rl;
     const bool live = row < rows;
+    const T* xr = x + row * ld_x;
+    int head = 0, nvec = cols / VE, ex = -1;  // ex: this thread's single element, if any
+    if constexpr (RAG) {
+      const RowSplit<T> sp(xr, cols);
+      head = sp.head;
+      nvec = sp.nvec;
+      if (live && t < sp.nx) ex = sp.extra(t);
+    }
     float h[VPT][VE];
+    float he = 0.0f;
     float ss = 0.0f;
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       const int v = t + k * TPR;
       if (live && v < nvec) {
-        Vec16<T> xv = ld(x + row * ld_x + (int64_t)v * VE);
+        const int64_t off = head + (int64_t)v * VE;
+        Vec16<T> xv = ld(xr + off);
         if constexpr (RES) {
-          Vec16<T> rv = ld(r + row * ld_r + (int64_t)v * VE);
+          Vec16<T> rv = ld(r + row * ld_r + off);
 #pragma unroll
           for (int e = 0; e < VE; ++e) {
             // Round the sum to T first: new_residual and the normalised value
@@ -68,6 +80,16 @@ rownorm_vec_kernel(const T* __restrict__ x, const T* __restrict__ r,
 #pragma unroll
         for (int e = 0; e < VE; ++e) h[k][e] = 0.0f;
       }
+    }
+    if constexpr (RAG) {
+      if (ex >= 0) {
+        he = to_f32(xr[ex]);
+        if constexpr (RES) he = to_f32(from_f32<T>(he + to_f32(r[row * ld_r + ex])));
+        ss = he * he;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
 #pragma unroll
       for (int e = 0; e < VE; ++e) ss = fmaf(h[k][e], h[k][e], ss);
     }
@@ -87,8 +109,8 @@ rownorm_vec_kernel(const T* __restrict__ x, const T* __restrict__ r,
     for (int k = 0; k < VPT; ++k) {
       const int v = t + k * TPR;
       if (live && v < nvec) {
-        const int64_t off = (int64_t)v * VE;
-        Vec16<T> wv = load16(w + off);
+        const int64_t off = head + (int64_t)v * VE;
+        Vec16<T> wv = RAG ? load16_any(w + off) : load16(w + off);
         Vec16<T> yv;
 #pragma unroll
         for (int e = 0; e < VE; ++e) yv.e[e] = from_f32<T>((h[k][e] / rms) * to_f32(wv.e[e]));
@@ -103,10 +125,18 @@ rownorm_vec_kernel(const T* __restrict__ x, const T* __restrict__ r,
         st(y + row * ld_y + off, yv);
       }
     }
+    if constexpr (RAG) {
+      if (ex >= 0) {
+        if constexpr (RES) {
+          if (nr != nullptr) nr[row * ld_nr + ex] = from_f32<T>(he);
+        }
+        y[row * ld_y + ex] = from_f32<T>((he / rms) * to_f32(w[ex]));
+      }
+    }
   }
 }
 
-// Any width / alignment: a 256-thread workgroup per row (rows by grid
+// Rows of more than 8192 vectors: a 256-thread workgroup per row (rows by grid
 // stride), scalar accesses, the hidden state recomputed (bit-identically) in
 // the second pass.
 template <typename T, bool RES>
@@ -146,13 +176,17 @@ rownorm_generic_kernel(const T* __restrict__ x, const T* __restrict__ r,
 }
 
 template <typename T, bool RES, int VPT, int TPR>
-void launch_vec(const T* x, const T* r, const T* w, T* nr, T* y, int64_t rows, int cols,
+void launch_vec(bool aligned, const T* x, const T* r, const T* w, T* nr, T* y, int64_t rows, int cols,
                 int64_t ld_x, int64_t ld_r, int64_t ld_nr, int64_t ld_y, float eps,
                 hipStream_t s) {
   constexpr int RPW = TPR >= 256 ? 1 : 256 / TPR;
-  const unsigned grid = row_grid((rows + RPW - 1) / RPW);
-  rownorm_vec_kernel<T, RES, VPT, TPR, true><<<dim3(grid), dim3(TPR * RPW), 0, s>>>(
-      x, r, w, nr, y, rows, cols, ld_x, ld_r, ld_nr, ld_y, eps);
+  const dim3 grid(row_grid((rows + RPW - 1) / RPW)), block(TPR * RPW);
+  if (aligned)
+    rownorm_vec_kernel<T, RES, VPT, TPR, false><<<grid, block, 0, s>>>(
+        x, r, w, nr, y, rows, cols, ld_x, ld_r, ld_nr, ld_y, eps);
+  else
+    rownorm_vec_kernel<T, RES, VPT, TPR, true><<<grid, block, 0, s>>>(
+        x, r, w, nr, y, rows, cols, ld_x, ld_r, ld_nr, ld_y, eps);
 }
 
 template <typename T, bool RES>
@@ -165,25 +199,32 @@ int dispatch(const void* xv, const void* rv, const void* wv, void* nrv, void* yv
   T* nr = static_cast<T*>(nrv);
   T* y = static_cast<T*>(yv);
   constexpr int VE = Vec16<T>::VE;
-  bool vec_ok = cols % VE == 0 && ld_x % VE == 0 && ld_y % VE == 0 && aligned16(x) &&
+  bool aligned = cols % VE == 0 && ld_x % VE == 0 && ld_y % VE == 0 && aligned16(x) &&
                 aligned16(w) && aligned16(y);
-  if (RES) vec_ok = vec_ok && ld_r % VE == 0 && aligned16(r);
-  if (RES && nr) vec_ok = vec_ok && ld_nr % VE == 0 && aligned16(nr);
+  if (RES) aligned = aligned && ld_r % VE == 0 && aligned16(r);
+  if (RES && nr) aligned = aligned && ld_nr % VE == 0 && aligned16(nr);
   const int64_t nvec = cols / VE;
   const int c = (int)cols;
-#define AK_LAUNCH(VPT, TPR) launch_vec<T, RES, VPT, TPR>(x, r, w, nr, y, rows, c, ld_x, ld_r, ld_nr, ld_y, eps, s)
-  // One 16-byte vector per thread while the row fits in 1024 threads: the
-  // most waves in flight per byte, which is what saturates HBM here
-  // (fused C3 shape: 1 vector x 512 threads beat 8 vectors x 64 threads by
-  // 25% on MI355X).
-  if (!vec_ok) {
-    rownorm_generic_kernel<T, RES><<<dim3(row_grid(rows)), dim3(256), 0, s>>>(
-        x, r, w, nr, y, rows, c, ld_x, ld_r, ld_nr, ld_y, eps);
-  } else if (nvec <= 64) AK_LAUNCH(1, 64);
+#define AK_LAUNCH(VPT, TPR) launch_vec<T, RES, VPT, TPR>(aligned, x, r, w, nr, y, rows, c, ld_x, ld_r, ld_nr, ld_y, eps, s)
+  // One 16-byte vector per thread while the row fits in 512 threads: the most
+  // waves in flight per byte (fused [16384, 4096] bf16: 1 vector x 512 threads
+  // beat 8 vectors x 64 threads by 25%).
+  // Two vectors a thread where one leaves too little in flight per thread: past
+  // 512 vectors ([8192, 5120] bf16 fused 64.5 -> 57.1 us), and for the plain
+  // norm (one input stream) of enough rows ([16384, 2048] bf16 28.3 -> 25.7 us,
+  // [16384, 4097] 68.7 -> 56.1; a wave a row in fp32, [8192, 1024] 13.8 -> 11.2).
+  // Few rows stay on one vector a thread: 64 x 4096 takes 3.2 us so and 3.5.
+  const bool two = !RES && rows >= 1024;
+  if (nvec <= 64) AK_LAUNCH(1, 64);
   else if (nvec <= 128) AK_LAUNCH(1, 128);
-  else if (nvec <= 256) AK_LAUNCH(1, 256);
-  else if (nvec <= 512) AK_LAUNCH(1, 512);
-  else if (nvec <= 1024) AK_LAUNCH(1, 1024);
+  else if (nvec <= 256) {
+    if (two && VE == 4) AK_LAUNCH(4, 64);
+    else if (two) AK_LAUNCH(2, 128);
+    else AK_LAUNCH(1, 256);
+  } else if (nvec <= 512) {
+    if (two) AK_LAUNCH(2, 256);
+    else AK_LAUNCH(1, 512);
+  } else if (nvec <= 1024) AK_LAUNCH(2, 512);
   else if (nvec <= 2048) AK_LAUNCH(2, 1024);
   else if (nvec <= 4096) AK_LAUNCH(4, 1024);
   else if (nvec <= 8192) AK_LAUNCH(8, 1024);

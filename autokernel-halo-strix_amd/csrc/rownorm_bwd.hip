@@ -33,11 +33,16 @@ namespace {
 
 // workgroups of the row pass: one per CU (a sweep at the C3 shape measured
 // 256 / 384 / 512 / 1024 workgroups at 94.8 / 104.4 / 97.3 / 99.9 us; fewer
-// workgroups also mean fewer partial weight-gradient rows to sum)
+// workgroups also mean fewer partial weight-gradient rows to sum), more for
+// narrow rows (bwd_grid)
 constexpr int kBwdMaxGrid = 256;
-constexpr int kBwdMaxParts = 2048; // partial dw rows (kBwdMaxGrid x at most 4 row slots)
+constexpr int kBwdMaxParts = 2048; // partial dw rows (bwd_grid x at most 4 row slots: at most 1024)
 
-template <typename T, bool ADD_DH, int VPT, int TPR>
+// RAG: rows at any address and of any width. A thread's columns are the same
+// in every row (its weight gradient stays in its registers), so the vectors
+// keep their columns and take the row's alignment as it comes, and the cols %
+// VE last columns go one to a thread.
+template <typename T, bool ADD_DH, int VPT, int TPR, bool RAG>
 __global__ void __launch_bounds__(TPR >= 256 ? TPR : 256)
 rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
                        const T* __restrict__ dy, const T* __restrict__ dh, T* __restrict__ dx,
@@ -56,8 +61,12 @@ rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
   float wf[VPT][VE], dwacc[VPT][VE];
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
-    const int v = min(t + k * TPR, nvec - 1);
-    const Vec16<T> wv = load16(w + (int64_t)v * VE);
+    Vec16<T> wv;
+    wv.u = u32x4{0, 0, 0, 0};
+    if (!RAG || nvec > 0) {
+      const int v = min(t + k * TPR, nvec - 1);
+      wv = RAG ? load16_any(w + (int64_t)v * VE) : load16(w + (int64_t)v * VE);
+    }
 #pragma unroll
     for (int e = 0; e < VE; ++e) {
       wf[k][e] = to_f32(wv.e[e]);
@@ -65,20 +74,36 @@ rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
     }
   }
 
+  const int ce = RAG && t < cols - nvec * VE ? nvec * VE + t : -1;  // this thread's single column
+  float we = 0.0f, dwe = 0.0f;
+  if constexpr (RAG) {
+    if (ce >= 0) we = to_f32(w[ce]);
+  }
+
   // Raw vectors of one row. Loads are unconditional, from clamped (always
   // valid) rows and vectors; rows and vectors past the end are masked where
   // the values are used.
   struct RowRegs {
     Vec16<T> x[VPT], g[VPT], h[VPT];
+    T xe, ge, he;
   };
+  auto ld = [](const T* p) { return RAG ? load16_any_nt(p) : load16_nt(p); };
   auto load_row = [&](int64_t row, RowRegs& R) {
     const int64_t rc = min(row, rows - 1);
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
+      if (RAG && nvec == 0) break;
       const int64_t off = (int64_t)min(t + k * TPR, nvec - 1) * VE;
-      R.x[k] = load16_nt(x + rc * ld_x + off);
-      R.g[k] = load16_nt(dy + rc * ld_dy + off);
-      if constexpr (ADD_DH) R.h[k] = load16_nt(dh + rc * ld_dh + off);
+      R.x[k] = ld(x + rc * ld_x + off);
+      R.g[k] = ld(dy + rc * ld_dy + off);
+      if constexpr (ADD_DH) R.h[k] = ld(dh + rc * ld_dh + off);
+    }
+    if constexpr (RAG) {
+      if (ce >= 0) {
+        R.xe = x[rc * ld_x + ce];
+        R.ge = dy[rc * ld_dy + ce];
+        if constexpr (ADD_DH) R.he = dh[rc * ld_dh + ce];
+      }
     }
   };
 
@@ -102,6 +127,15 @@ rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
         gf[k][e] = ok ? to_f32(cur.g[k].e[e]) : 0.0f;
         s1 = fmaf(xf[k][e], xf[k][e], s1);
         s2 = fmaf(gf[k][e] * wf[k][e], xf[k][e], s2);
+      }
+    }
+    float xe = 0.0f, ge = 0.0f;
+    if constexpr (RAG) {
+      if (live && ce >= 0) {
+        xe = to_f32(cur.xe);
+        ge = to_f32(cur.ge);
+        s1 = fmaf(xe, xe, s1);
+        s2 = fmaf(ge * we, xe, s2);
       }
     }
     s1 = wave_sum(s1);
@@ -135,7 +169,20 @@ rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
         out.e[e] = from_f32<T>(d);
         dwacc[k][e] = fmaf(gf[k][e], nrm, dwacc[k][e]);
       }
-      if (live && v < nvec) store16_nt(dx + row * ld_dx + (int64_t)v * VE, out);
+      if (live && v < nvec) {
+        T* const d = dx + row * ld_dx + (int64_t)v * VE;
+        if constexpr (RAG) store16_any_nt(d, out);
+        else store16_nt(d, out);
+      }
+    }
+    if constexpr (RAG) {
+      if (live && ce >= 0) {
+        const float nrm = xe * r;
+        float d = r * (ge * we - nrm * cg);
+        if constexpr (ADD_DH) d += to_f32(cur.he);
+        dx[row * ld_dx + ce] = from_f32<T>(d);
+        dwe = fmaf(ge, nrm, dwe);
+      }
     }
     cur = nxt;
   }
@@ -152,14 +199,19 @@ rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
                            __builtin_bit_cast(uint32_t, dwacc[k][e + 1]),
                            __builtin_bit_cast(uint32_t, dwacc[k][e + 2]),
                            __builtin_bit_cast(uint32_t, dwacc[k][e + 3])};
-          *reinterpret_cast<u32x4*>(prow + (int64_t)v * VE + e) = q;
+          // (a partial row's pitch is cols floats, so an odd width leaves it element-aligned)
+          if constexpr (RAG) *reinterpret_cast<u32x4_any*>(prow + (int64_t)v * VE + e) = q;
+          else *reinterpret_cast<u32x4*>(prow + (int64_t)v * VE + e) = q;
         }
       }
+    }
+    if constexpr (RAG) {
+      if (ce >= 0) prow[ce] = dwe;
     }
   }
 }
 
-// Any width or alignment: 256 threads per row with scalar accesses. The row
+// Very wide rows (plan_bwd): 256 threads per row with scalar accesses. The row
 // is read twice (sums, then gradients); the workgroup's partial dw row lives
 // in the workspace and is updated by the thread that owns each column.
 template <typename T, bool ADD_DH>
@@ -211,8 +263,9 @@ rownorm_bwd_generic_kernel(const T* __restrict__ x, const T* __restrict__ w,
 // trip), folded pairwise; the 16 wave sums are then added in wave order.
 constexpr int kColWaves = 16;
 constexpr int kColBatch = 32;
+template <typename G>
 __global__ void __launch_bounds__(64 * kColWaves)
-colsum_kernel(const float* __restrict__ part, float* __restrict__ dw, int nparts, int cols) {
+colsum_kernel(const float* __restrict__ part, G* __restrict__ dw, int nparts, int cols) {
   __shared__ float acc[kColWaves][64];
   const int cl = threadIdx.x % 64, q = threadIdx.x / 64;
   const int c = blockIdx.x * 64 + cl;
@@ -240,7 +293,7 @@ colsum_kernel(const float* __restrict__ part, float* __restrict__ dw, int nparts
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < kColWaves; ++i) s += acc[i][cl];
-    dw[c] = s;
+    dw[c] = from_f32<G>(s);
   }
 }
 
@@ -252,12 +305,28 @@ size_t bwd_ws_bytes(int64_t rows, int64_t cols) {
   return align256((size_t)parts * (size_t)cols * sizeof(float));
 }
 
+// Most workgroups of the row pass (kBwdMaxGrid = one a CU at 64 and at 512 and
+// more threads a row, where more of them measured slower). At 128 and 256
+// threads one workgroup a CU leaves too few waves to hide a row's loads and
+// barrier: two a CU, four where a row fills at most three of the four waves;
+// fewer when a row slot would get less than 8 rows, since every slot's partial
+// row is written and summed. Forward and backward of [8192, 2048] bf16 61.7 ->
+// 55.4 us, [11317, 1088] 76.4 -> 51.3, [16384, 768] 54.3 -> 48.4.
+int64_t bwd_grid(int64_t rows, int tpr, int64_t nvec) {
+  int64_t g = kBwdMaxGrid;
+  if (tpr == 128) g *= 2;
+  if (tpr == 256) g *= nvec <= 192 ? 4 : 2;
+  const int rpw = tpr >= 256 ? 1 : 256 / tpr;
+  while (g > kBwdMaxGrid && rows < 8 * g * rpw) g /= 2;
+  return g;
+}
+
 // Launch plan of the backward's row pass: the kernel (the generic one, or a
 // vector kernel with VPT vectors per thread and TPR threads per row), its
 // grid, and the number of partial weight-gradient rows it writes (one per
 // workgroup row slot), which colsum_kernel then sums.
 struct BwdPlan {
-  bool generic;
+  bool generic, aligned;
   int vpt, tpr, grid, nparts;
 };
 
@@ -266,12 +335,14 @@ BwdPlan plan_bwd(const void* x, const void* w, const void* dy, const void* dh, c
                  int64_t rows, int64_t cols, int64_t ld_x, int64_t ld_dy, int64_t ld_dh,
                  int64_t ld_dx) {
   constexpr int VE = Vec16<T>::VE;
-  bool vec_ok = cols % VE == 0 && ld_x % VE == 0 && ld_dy % VE == 0 && ld_dx % VE == 0 &&
-                aligned16(x) && aligned16(w) && aligned16(dy) && aligned16(dx);
-  if (dh) vec_ok = vec_ok && ld_dh % VE == 0 && aligned16(dh);
-  const int64_t nvec = cols / VE;
   BwdPlan p{};
-  if (!vec_ok || nvec > 8192) {
+  p.aligned = cols % VE == 0 && ld_x % VE == 0 && ld_dy % VE == 0 && ld_dx % VE == 0 &&
+                aligned16(x) && aligned16(w) && aligned16(dy) && aligned16(dx);
+  if (dh) p.aligned = p.aligned && ld_dh % VE == 0 && aligned16(dh);
+  const int64_t nvec = cols / VE;
+  // (ragged 16-bit rows past 4096 vectors spill in the vector kernel: [1000, 40001]
+  // bf16 forward and backward 1036 us with it, 911 with the generic one)
+  if (nvec > 8192 || (!p.aligned && VE == 8 && nvec > 4096)) {
     p.generic = true;
     p.grid = (int)(rows < kBwdMaxGrid ? rows : kBwdMaxGrid);
     p.nparts = p.grid;
@@ -281,7 +352,8 @@ BwdPlan plan_bwd(const void* x, const void* w, const void* dy, const void* dh, c
   p.tpr = nvec <= 64 ? 64 : nvec <= 128 ? 128 : nvec <= 256 ? 256 : nvec <= 512 ? 512 : 1024;
   const int rpw = p.tpr >= 256 ? 1 : 256 / p.tpr;
   const int64_t blocks = (rows + rpw - 1) / rpw;
-  p.grid = (int)(blocks < kBwdMaxGrid ? blocks : kBwdMaxGrid);
+  const int64_t most = bwd_grid(rows, p.tpr, nvec);
+  p.grid = (int)(blocks < most ? blocks : most);
   p.nparts = p.grid * rpw;
   return p;
 }
@@ -291,9 +363,19 @@ size_t plan_ws_bytes(const BwdPlan& p, int64_t cols) {
   return align256((size_t)p.nparts * (size_t)cols * sizeof(float));
 }
 
+// The sum of the partial rows into dw, of the element type or fp32.
+void launch_colsum(const float* part, void* dw, int gw_dtype, int nparts, int cols, hipStream_t s) {
+  const dim3 grid((cols + 63) / 64), block(64 * kColWaves);
+  switch (gw_dtype) {
+    case AK_DTYPE_F32: colsum_kernel<<<grid, block, 0, s>>>(part, static_cast<float*>(dw), nparts, cols); break;
+    case AK_DTYPE_F16: colsum_kernel<<<grid, block, 0, s>>>(part, static_cast<f16*>(dw), nparts, cols); break;
+    default: colsum_kernel<<<grid, block, 0, s>>>(part, static_cast<bf16*>(dw), nparts, cols); break;
+  }
+}
+
 template <typename T, bool ADD_DH>
 void run_bwd(const BwdPlan& plan, const void* xv, const void* wv, const void* dyv,
-             const void* dhv, void* dxv, float* dw, float* part, int64_t rows, int64_t cols,
+             const void* dhv, void* dxv, void* dw, int gw_dtype, float* part, int64_t rows, int64_t cols,
              int64_t ld_x, int64_t ld_dy, int64_t ld_dh, int64_t ld_dx, float eps,
              hipStream_t s) {
   const T* x = static_cast<const T*>(xv);
@@ -304,9 +386,10 @@ void run_bwd(const BwdPlan& plan, const void* xv, const void* wv, const void* dy
   if (!dw) part = nullptr;
   const int c = (int)cols;
   const dim3 grid(plan.grid);
-#define AK_VEC(VPT, TPR)                                                                       \
-  rownorm_bwd_vec_kernel<T, ADD_DH, VPT, TPR><<<grid, dim3(TPR >= 256 ? TPR : 256), 0, s>>>( \
+#define AK_VEC1(VPT, TPR, RAG)                                                                       \
+  rownorm_bwd_vec_kernel<T, ADD_DH, VPT, TPR, RAG><<<grid, dim3(TPR >= 256 ? TPR : 256), 0, s>>>( \
       x, w, dy, dh, dx, part, rows, c, ld_x, ld_dy, ld_dh, ld_dx, eps)
+#define AK_VEC(VPT, TPR) (plan.aligned ? AK_VEC1(VPT, TPR, false) : AK_VEC1(VPT, TPR, true))
   if (plan.generic) {
     rownorm_bwd_generic_kernel<T, ADD_DH><<<grid, dim3(256), 0, s>>>(
         x, w, dy, dh, dx, part, rows, c, ld_x, ld_dy, ld_dh, ld_dx, eps);
@@ -319,7 +402,8 @@ void run_bwd(const BwdPlan& plan, const void* xv, const void* wv, const void* dy
   else if (plan.vpt == 4) AK_VEC(4, 1024);
   else AK_VEC(8, 1024);
 #undef AK_VEC
-  if (dw) colsum_kernel<<<dim3((c + 63) / 64), dim3(64 * kColWaves), 0, s>>>(part, dw, plan.nparts, c);
+#undef AK_VEC1
+  if (dw) launch_colsum(part, dw, gw_dtype, plan.nparts, c, s);
 }
 
 BwdPlan plan_for(const void* x, const void* w, const void* dy, const void* dh, const void* dx,
@@ -352,17 +436,17 @@ int check_bwd_args(const char* name, int64_t rows, int64_t cols, int64_t ld_x, i
 
 // Enqueues the backward with the partial rows in `part` (checked by the caller).
 int enqueue_bwd(const char* name, const BwdPlan& plan, const void* x, const void* w,
-                const void* dy, const void* dh, void* dx, float* dw, float* part, int64_t rows,
+                const void* dy, const void* dh, void* dx, void* dw, int gw_dtype, float* part, int64_t rows,
                 int64_t cols, int64_t ld_x, int64_t ld_dy, int64_t ld_dh, int64_t ld_dx,
                 float eps, int dtype, hipStream_t s) {
   if (rows == 0) {
     // no rows: dw is all zeros (a fixed-order sum over no partial rows)
-    if (dw) colsum_kernel<<<dim3((unsigned)((cols + 63) / 64)), dim3(64 * kColWaves), 0, s>>>(nullptr, dw, 0, (int)cols);
+    if (dw) launch_colsum(nullptr, dw, gw_dtype, 0, (int)cols, s);
     return ak_check_launch(name);
   }
 #define AK_BWD(TT)                                                                              \
-  (dh ? run_bwd<TT, true>(plan, x, w, dy, dh, dx, dw, part, rows, cols, ld_x, ld_dy, ld_dh, ld_dx, eps, s) \
-      : run_bwd<TT, false>(plan, x, w, dy, dh, dx, dw, part, rows, cols, ld_x, ld_dy, ld_dh, ld_dx, eps, s))
+  (dh ? run_bwd<TT, true>(plan, x, w, dy, dh, dx, dw, gw_dtype, part, rows, cols, ld_x, ld_dy, ld_dh, ld_dx, eps, s) \
+      : run_bwd<TT, false>(plan, x, w, dy, dh, dx, dw, gw_dtype, part, rows, cols, ld_x, ld_dy, ld_dh, ld_dx, eps, s))
   switch (dtype) {
     case AK_DTYPE_F32: AK_BWD(float); break;
     case AK_DTYPE_F16: AK_BWD(f16); break;
@@ -373,7 +457,7 @@ int enqueue_bwd(const char* name, const BwdPlan& plan, const void* x, const void
 }
 
 int bwd_entry(const char* name, const void* x, const void* w, const void* dy, const void* dh,
-              void* dx, float* dw, void* ws, size_t ws_bytes, int64_t rows, int64_t cols,
+              void* dx, void* dw, int gw_dtype, void* ws, size_t ws_bytes, int64_t rows, int64_t cols,
               int64_t ld_x, int64_t ld_dy, int64_t ld_dh, int64_t ld_dx, float eps, int dtype,
               void* stream) {
   int rc = check_bwd_args(name, rows, cols, ld_x, ld_dy, ld_dh, ld_dx, dh != nullptr, dtype);
@@ -388,7 +472,7 @@ int bwd_entry(const char* name, const void* x, const void* w, const void* dy, co
                           ws_bytes, bwd_ws_bytes(rows, cols));
   }
   const BwdPlan plan = plan_for(x, w, dy, dh, dx, rows, cols, ld_x, ld_dy, ld_dh, ld_dx, dtype);
-  return enqueue_bwd(name, plan, x, w, dy, dh, dx, dw, static_cast<float*>(ws), rows, cols, ld_x,
+  return enqueue_bwd(name, plan, x, w, dy, dh, dx, dw, gw_dtype, static_cast<float*>(ws), rows, cols, ld_x,
                      ld_dy, ld_dh, ld_dx, eps, dtype, ak_stream(stream));
 }
 
@@ -476,7 +560,7 @@ extern "C" int ak_rmsnorm_bwd(const void* x, const void* weight, const void* gra
                               void* grad_x, float* grad_weight, void* workspace,
                               size_t workspace_bytes, int64_t rows, int64_t cols, int64_t ld_x,
                               int64_t ld_g, int64_t ld_gx, float eps, int dtype, void* stream) {
-  return ak::bwd_entry("ak_rmsnorm_bwd", x, weight, grad_out, nullptr, grad_x, grad_weight,
+  return ak::bwd_entry("ak_rmsnorm_bwd", x, weight, grad_out, nullptr, grad_x, grad_weight, AK_DTYPE_F32,
                        workspace, workspace_bytes, rows, cols, ld_x, ld_g, 0, ld_gx, eps, dtype,
                        stream);
 }
@@ -488,7 +572,18 @@ extern "C" int ak_fused_add_rmsnorm_bwd(const void* hidden, const void* weight,
                                         int64_t ld_h, int64_t ld_gh, int64_t ld_gn,
                                         int64_t ld_gx, float eps, int dtype, void* stream) {
   return ak::bwd_entry("ak_fused_add_rmsnorm_bwd", hidden, weight, grad_normed, grad_hidden,
-                       grad_x, grad_weight, workspace, workspace_bytes, rows, cols, ld_h, ld_gn,
+                       grad_x, grad_weight, AK_DTYPE_F32, workspace, workspace_bytes, rows, cols, ld_h, ld_gn,
+                       ld_gh, ld_gx, eps, dtype, stream);
+}
+
+extern "C" int ak_fused_add_rmsnorm_bwd_gw(const void* hidden, const void* weight,
+                                           const void* grad_hidden, const void* grad_normed,
+                                           void* grad_x, void* grad_weight, void* workspace,
+                                           size_t workspace_bytes, int64_t rows, int64_t cols,
+                                           int64_t ld_h, int64_t ld_gh, int64_t ld_gn,
+                                           int64_t ld_gx, float eps, int dtype, void* stream) {
+  return ak::bwd_entry("ak_fused_add_rmsnorm_bwd_gw", hidden, weight, grad_normed, grad_hidden,
+                       grad_x, grad_weight, dtype, workspace, workspace_bytes, rows, cols, ld_h, ld_gn,
                        ld_gh, ld_gx, eps, dtype, stream);
 }
 
@@ -524,5 +619,5 @@ extern "C" int ak_fused_add_rmsnorm_bwd_noalloc(const void* hidden, const void* 
     part += (size_t)slot * (ak::kNoAllocSlotBytes / sizeof(float));
   }
   return ak::enqueue_bwd(name, plan, hidden, weight, grad_normed, grad_hidden, grad_x,
-                         grad_weight, part, rows, cols, ld_h, ld_gn, ld_gh, ld_gx, eps, dtype, s);
+                         grad_weight, AK_DTYPE_F32, part, rows, cols, ld_h, ld_gn, ld_gh, ld_gx, eps, dtype, s);
 }

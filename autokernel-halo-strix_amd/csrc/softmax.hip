@@ -4,7 +4,7 @@
 // for sum(exp(x - max)) in fp32 with wave64 DPP reductions, then normalised
 // and written once, with nontemporal accesses. Rows of up to 128 16-byte
 // vectors are owned by one wave (no barriers), wider rows by up to 1024
-// threads holding one vector each (up to 16 past 1024 vectors). Rows are
+// threads holding two to four vectors each (up to 16 past 4096 vectors). Rows are
 // indexed with 64-bit arithmetic and walked by grid stride on a capped grid,
 // so every row is written whatever the row count.
 //
@@ -25,7 +25,7 @@ namespace {
 // few elements before the first and behind the last one go one to a thread,
 // so the row still crosses HBM once, in whole vectors. [4096, 50257] fp16:
 // 152 us, 5.4 TB/s, as a copy runs here (523 us with element accesses and two
-// passes); [9324, 777] fp16 24.4 -> 11.1 us.
+// passes); [98304, 777] fp16 56.7 us, 5.4 TB/s.
 //
 // From 4 vectors a thread of 16-bit elements on, the row stays packed between
 // the passes and exp(x - max) is formed twice: 32 registers for 8 vectors
@@ -55,6 +55,7 @@ softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int
       nvec = sp.nvec;
       if (live && t < sp.nx) ex = sp.extra(t);
     }
+    if (!live) nvec = 0;  // a row slot past the last row touches nothing
     Vec16<T> raw[PACKED ? VPT : 1];
     float v[PACKED ? 1 : VPT][VE];
     float xe = -INFINITY;
@@ -74,7 +75,7 @@ softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int
     } else {
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
-        if (live && t + k * TPR < nvec) {
+        if (t + k * TPR < nvec) {
           const Vec16<T> xv = ld(k);
 #pragma unroll
           for (int e = 0; e < VE; ++e) {
@@ -113,7 +114,7 @@ softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int
 #pragma unroll
         for (int e = 0; e < VE; ++e) s += fast_exp(to_f32(raw[k].e[e]) - m);
         keep_packed(raw[k]);
-      } else if (live && t + k * TPR < nvec) {
+      } else if (t + k * TPR < nvec) {
 #pragma unroll
         for (int e = 0; e < VE; ++e) {
           v[k][e] = fast_exp(v[k][e] - m);
@@ -139,7 +140,7 @@ softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       const int c = t + k * TPR;
-      if (live && c < nvec) {
+      if (c < nvec) {
         Vec16<T> o;
 #pragma unroll
         for (int e = 0; e < VE; ++e) {
@@ -239,12 +240,22 @@ int dispatch(const void* xv, void* yv, int64_t rows, int64_t cols, int64_t ld_x,
   const int64_t nvec = cols / VE;
   const int c = (int)cols;
 #define AK_LAUNCH(VPT, TPR) launch_vec<T, VPT, TPR>(aligned, x, y, rows, c, ld_x, ld_y, s)
+  // Two 16-byte vectors a thread (four in rows off the 16-byte grid and in narrow
+  // fp32 rows) past one wave's 128: with one a thread, half of a workgroup's time
+  // went to its reductions. [16384, 8192] bf16 103 -> 84 us, [24000, 3001] fp16
+  // 68.9 -> 49.4, [32768, 777] fp32 47.8 -> 36.8, [8192, 4097] fp32 59.6 -> 46.4.
   if (nvec <= 64) AK_LAUNCH(1, 64);
   else if (nvec <= 128) AK_LAUNCH(2, 64);
-  else if (nvec <= 256) AK_LAUNCH(1, 256);
-  else if (nvec <= 512) AK_LAUNCH(1, 512);
-  else if (nvec <= 1024) AK_LAUNCH(1, 1024);
-  else if (nvec <= 2048) AK_LAUNCH(2, 1024);
+  else if (nvec <= 256) {
+    if (VE == 4) AK_LAUNCH(4, 64);
+    else AK_LAUNCH(2, 128);
+  } else if (nvec <= 512) {
+    if (aligned) AK_LAUNCH(2, 256);
+    else AK_LAUNCH(4, 128);
+  } else if (nvec <= 1024) {
+    if (aligned) AK_LAUNCH(2, 512);
+    else AK_LAUNCH(4, 256);
+  } else if (nvec <= 2048) AK_LAUNCH(4, 512);
   else if (nvec <= 4096) AK_LAUNCH(4, 1024);
   else if (nvec <= 8192) AK_LAUNCH(8, 1024);
   else if (nvec <= 16384) AK_LAUNCH(16, 1024);

@@ -55,6 +55,7 @@ _SIGNATURES = {
     "ak_fused_add_rmsnorm_bwd": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                  _c_void_p, ctypes.c_size_t, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _f32, _int, _c_void_p],
+    "ak_fused_add_rmsnorm_bwd_gw": [_c_void_p] * 7 + [ctypes.c_size_t] + [_i64] * 6 + [_f32, _int, _c_void_p],
     "ak_fused_add_rmsnorm_bwd_noalloc": [_c_void_p] * 6 + [_i64] * 6 + [_f32, _int, _c_void_p],
     "ak_softmax_fwd": [_c_void_p, _c_void_p, _i64, _i64, _i64, _i64, _int, _c_void_p],
     "ak_ce_fwd": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,

@@ -119,6 +119,18 @@ int ak_fused_add_rmsnorm_bwd(const void* hidden, const void* weight,
                              float eps, int dtype, void* stream);
 
 /*
+ * ak_fused_add_rmsnorm_bwd with grad_weight in the element type dtype (the
+ * fp32 sum rounded once), as a parameter of that type takes it.
+ */
+int ak_fused_add_rmsnorm_bwd_gw(const void* hidden, const void* weight,
+                                const void* grad_hidden, const void* grad_normed,
+                                void* grad_x, void* grad_weight,
+                                void* workspace, size_t workspace_bytes,
+                                int64_t rows, int64_t cols,
+                                int64_t ld_h, int64_t ld_gh, int64_t ld_gn, int64_t ld_gx,
+                                float eps, int dtype, void* stream);
+
+/*
  * ak_fused_add_rmsnorm_bwd without a workspace: the same kernels and results
  * (bitwise), with the partial weight-gradient rows in a fixed 64 MiB device
  * array inside the library (one per GPU, held until the process ends) instead

@@ -155,3 +155,39 @@ def test_rownorm_expanded_views_and_grid_stride():
         ws = 1 + 0.1 * torch.randn(cols, generator=g)
         ys = rmsnorm.kernel_fn(xs.to(DEV), ws.to(DEV)).cpu()
         assert _rel_ok_f32(ys, ops.rmsnorm_f32_ref(xs, ws))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vecs,over", [(0, 3), (1, 1), (64, 3), (65, 0), (128, 1), (129, 2), (256, 3), (513, 1),
+                                       (1024, 3), (1025, 2), (4097, 1)])
+@pytest.mark.parametrize("rows", [5, 1027])
+def test_rownorm_rows_at_any_address(dtype, vecs, over, rows):
+    """Ragged rows at the edges of every vectors-per-thread variant (``vecs``
+    16-byte vectors plus ``over`` elements; 1024 and more rows choose others),
+    all operands in pitched views that start off the 16-byte grid, each its own
+    way; the elements around the output rows keep their values."""
+    need_gpu()
+    from kernels.hip import _lib
+    ve = 16 // torch.empty((), dtype=dtype).element_size()
+    cols = max(1, vecs * ve + over)
+    rows = rows if cols < 9000 else 5
+    g = torch.Generator().manual_seed(cols)
+    say("rownorm any address", dtype, rows, cols)
+
+    def view(off, fill=None):
+        b = torch.full((rows, cols + 5), 7.0) if fill is None else torch.randn(rows, cols + 5, generator=g)
+        return b.to(dtype).to(DEV), slice(off, off + cols)
+
+    (xb, xs), (rb, rs), (hb, hs), (yb, ys), (pb, ps) = view(1, 0), view(2, 0), view(3), view(1), view(0)
+    w = (1 + 0.1 * torch.randn(cols + 1, generator=g)).to(dtype).to(DEV)[1:]
+    _lib.fused_add_rmsnorm(xb[:, xs], rb[:, rs], w, hb[:, hs], yb[:, ys], 1e-5)
+    _lib.rmsnorm(xb[:, xs], w, pb[:, ps], 1e-5)
+    x, r, wc = xb[:, xs].cpu(), rb[:, rs].cpu(), w.cpu()
+    hr, yr = ops.fused_residual_add_rmsnorm_ref(x, r, wc, 1e-5)
+    pr = ops.rmsnorm_f32_ref(x, wc, 1e-5)
+    assert torch.equal(hb[:, hs].cpu(), hr)
+    for b, s, want in ((yb, ys, yr), (pb, ps, pr)):
+        got = b[:, s].cpu()
+        assert _rel_ok_f32(got, want) if dtype == torch.float32 else max_ulp(got, want) <= 1
+    for b, s in ((hb, hs), (yb, ys), (pb, ps)):
+        assert bool((b[:, :s.start] == 7).all()) and bool((b[:, s.stop:] == 7).all())

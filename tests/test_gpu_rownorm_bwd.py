@@ -224,3 +224,40 @@ def test_backward_of_broadcast_upstream_gradient():
     ops.rmsnorm_ref(x64, w64, 1e-6).sum(0).backward(up.double())
     assert torch.allclose(xd.grad.double().cpu(), x64.grad, rtol=1e-4, atol=1e-5)
     assert torch.allclose(wd.grad.double().cpu(), w64.grad, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,vecs,over", [(5, 0, 3), (2100, 1, 1), (2100, 64, 3), (8300, 65, 1), (2100, 128, 3),
+                                            (4200, 130, 1), (2100, 193, 0), (4200, 256, 2), (700, 257, 3), (300, 513, 1),
+                                            (40, 1025, 3), (7, 2049, 1)])
+def test_bwd_rows_at_any_address(dtype, rows, vecs, over):
+    """Ragged rows at the edges of every vectors-per-thread variant and of the
+    grid's rule (``vecs`` 16-byte vectors plus ``over`` elements), every operand
+    in a pitched view that starts off the 16-byte grid; the weight gradient in
+    fp32 and, through the element-type entry, that value rounded once; the
+    elements around grad_x keep their values."""
+    need_gpu()
+    from kernels.hip import _lib
+    cols = max(1, vecs * (16 // torch.empty((), dtype=dtype).element_size()) + over)
+    x, w, dy, dh = _inputs(rows, cols, dtype, cols)
+
+    def view(t, off):
+        b = torch.full((rows, cols + 4), 7.0, dtype=dtype, device=DEV)
+        b[:, off:off + cols] = t.to(DEV)
+        return b, b[:, off:off + cols]
+
+    (_, xv), (_, gv), (_, hv), (ob, ov) = view(x, 1), view(dy, 2), view(dh, 3), view(x, 1)
+    wd = torch.cat([w[:1], w]).to(DEV)[1:]
+    ws = torch.empty(_lib.rmsnorm_bwd_workspace_bytes(rows, cols), dtype=torch.uint8, device=DEV)
+    for h in (None, hv):
+        say("rownorm bwd any address", dtype, rows, cols, h is not None)
+        gw = torch.full((cols,), 7.0, device=DEV)
+        _lib.fused_add_rmsnorm_bwd(xv, wd, h, gv, ov, gw, ws, 1e-5)
+        _check_gx(ov, x, w, dy, dh if h is not None else None, 1e-5)
+        _check_gw(gw, x, w, dy, 1e-5)
+        assert bool((ob[:, :1] == 7).all()) and bool((ob[:, 1 + cols:] == 7).all())
+    gt = torch.empty(cols, dtype=dtype, device=DEV)
+    rc = _lib.load().ak_fused_add_rmsnorm_bwd_gw(
+        xv.data_ptr(), wd.data_ptr(), None, gv.data_ptr(), ov.data_ptr(), gt.data_ptr(), ws.data_ptr(), ws.numel(),
+        rows, cols, cols + 4, cols, cols + 4, cols + 4, 1e-5, _lib.dtype_code(dtype), _lib._stream(xv))
+    assert rc == 0 and torch.equal(gt, gw.to(dtype))
