@@ -32,7 +32,7 @@ using Maybe = std::optional<Tensor>;
   X(ak_last_error) X(ak_rmsnorm_fwd) X(ak_fused_add_rmsnorm_fwd) X(ak_rmsnorm_bwd_workspace_bytes) \
   X(ak_fused_add_rmsnorm_bwd_gw) X(ak_softmax_fwd) X(ak_ce_fwd) X(ak_ce_bwd_tiny)   \
   X(ak_ce_count_valid) X(ak_ce_mean) X(ak_scale_inplace) X(ak_diag_scan_fwd)                       \
-  X(ak_diag_scan_bwd_workspace_bytes) X(ak_diag_scan_bwd) X(ak_selective_scan_fwd)                 \
+  X(ak_diag_scan_bwd_workspace_bytes) X(ak_diag_scan_bwd) X(ak_selective_scan_fwd_ws) X(ak_selective_scan_fwd_workspace_bytes)                 \
   X(ak_selective_scan_bwd_workspace_bytes) X(ak_selective_scan_bwd)                                \
   X(ak_lmhead_ce_workspace_bytes) X(ak_lmhead_ce_fwd) X(ak_lmhead_ce_bwd_range)                    \
   X(ak_lmhead_grad_workspace_bytes) X(ak_lmhead_grad_hidden) X(ak_lmhead_grad_weight)
@@ -440,12 +440,14 @@ void run_scan(const Tensor& u, const Tensor& delta, const Tensor& A, const Tenso
               const Tensor& z, const Tensor& bias, bool softplus, const ScanDims& k, const Tensor& out, const Tensor& last,
               const Tensor& prez, const Tensor& ckpt) {
   const BcStride sb = bc_stride(B), sc = bc_stride(C);
-  check(api.ak_selective_scan_fwd(
+  const size_t bytes = api.ak_selective_scan_fwd_workspace_bytes(k.b, k.d, k.l, k.n, k.g, 0);
+  const Tensor ws = bytes ? bytes_like(u, bytes) : Tensor();
+  check(api.ak_selective_scan_fwd_ws(
             u.data_ptr(), delta.data_ptr(), f32p(A), B.data_ptr(), C.data_ptr(), f32p(D), ptr(z), f32p(bias), out.data_ptr(),
             f32p(last), ptr(prez), nullptr, f32p(ckpt), k.b, k.d, k.l, k.n, k.g, u.stride(0), u.stride(1), delta.stride(0),
             delta.stride(1), A.stride(0), sb.b, sb.g, sb.n, sc.b, sc.g, sc.n, z.defined() ? z.stride(0) : 0,
             z.defined() ? z.stride(1) : 0, out.stride(0), out.stride(1), softplus, 0, code_of(u.scalar_type()),
-            code_of(delta.scalar_type()), code_of(B.scalar_type()), AK_DTYPE_F32, stream_of(u)), "ak_selective_scan_fwd");
+            code_of(delta.scalar_type()), code_of(B.scalar_type()), AK_DTYPE_F32, ptr(ws), bytes, stream_of(u)), "ak_selective_scan_fwd");
 }
 
 struct SelectiveScan : torch::autograd::Function<SelectiveScan> {

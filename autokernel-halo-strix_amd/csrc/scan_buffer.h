@@ -34,6 +34,29 @@ __device__ __forceinline__ Raw4<T> bload4(Rsrc r, uint32_t voff, uint32_t soff) 
     return __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0);
 }
 
+// Four consecutive elements at any element address: a wave-uniform base and a
+// lane's byte offset.
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+template <typename T>
+__device__ __forceinline__ Raw4<T> gload4_any(const void* base, uint32_t off) {
+  const char* q = static_cast<const char*>(base) + off;
+  if constexpr (sizeof(T) == 4) return *reinterpret_cast<const u32x4_any*>(q);
+  else return *reinterpret_cast<const u32x2_any*>(q);
+}
+
+// The elements of v from s on (s in 0 .. 4), zeros behind them.
+template <typename T>
+__device__ __forceinline__ void raw4_drop(Raw4<T>& v, int s) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s > i) v = u32x4{v[1], v[2], v[3], 0u};
+  } else {
+    const uint64_t w = __builtin_bit_cast(uint64_t, v);
+    v = __builtin_bit_cast(u32x2, s < 4 ? w >> (16 * s) : (uint64_t)0);
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ Raw1<T> bload1(Rsrc r, uint32_t voff, uint32_t soff) {
   if constexpr (sizeof(T) == 4)

@@ -55,9 +55,58 @@ struct ScanParams {
   // [batch, dim, dstate] of their gradients
   int b_const, c_const;
   int64_t B_ds, C_ds;
+  // sequence segments (scan_segments): segs segments of seg_tiles 64-step tiles,
+  // and what the segment pass leaves: per segment the state from zero (the
+  // adjoint, in the backward) and the sum of delta' over it
+  int segs, seg_tiles;
+  float* seg_state;            // [batch, segs, dim, dstate]
+  float* seg_dsum;             // [batch, segs, dim]
   float* dBc_part;
   float* dCc_part;
 };
+
+// A scan whose (channel, state) lanes leave most of the GPU empty is cut into
+// segments of the sequence, a workgroup each. A segment pass first forms each
+// segment's state from zero and its sum of delta' (all of its decay: the
+// product of exp(delta' A) is exp(A sum delta')); the scan's workgroups then
+// fold the segments before theirs into their entering state. The recurrence's
+// exponentials are paid twice and a launch is added, so: up to 128 workgroups
+// of 16 channels, about 512 segments in all (two workgroups a CU) from 4 tiles
+// on; up to 192 workgroups, about 1024 from 24 tiles on. Measured (us, one
+// segment -> cut): training [1, 384, 4096] 422 -> 85, [1, 2048, 1024] 124 -> 82,
+// [1, 768, 671] 113 -> 46, [2, 1536, 2048] (192) 237 -> 203; inference [1, 2048,
+// 1777] 88 -> 52, [1, 768, 4096] 100 -> 43, [1, 384, 512] 15.1 -> 10.6. Cut,
+// training [4, 768, 512] (192) would go 69 -> 72, [1, 1536, 128] 27.6 -> 29.7,
+// inference [2, 2048, 1024] (256) 30 -> 40. A function of the shape alone: the
+// bits of a result depend on it.
+struct ScanSegs {
+  int n, tiles;
+};
+inline ScanSegs scan_segments(int64_t batch, int64_t dim, int64_t seqlen, int64_t dstate,
+                              int64_t ngroups, int bc_flags) {
+  const int64_t tiles = (seqlen + kScanT - 1) / kScanT;
+  const int64_t groups = batch * ngroups * ((dim / ngroups + kScanCh - 1) / kScanCh);
+  int64_t n = 1;
+  if (dstate <= 16 && !(bc_flags & (AK_SCAN_B_CONST | AK_SCAN_C_CONST)) && groups > 0) {
+    if (groups <= 128 && tiles >= 4) n = (512 + groups / 2) / groups;
+    else if (groups <= 192 && tiles >= 24) n = 1024 / groups;
+    if (n > 32) n = 32;
+    if (n > tiles) n = tiles;
+    if (n < 1) n = 1;
+  }
+  const int64_t per = (tiles + n - 1) / n;
+  return {per > 0 ? (int)((tiles + per - 1) / per) : 1, per > 0 ? (int)per : 1};
+}
+
+// Bytes of the segment pass's states and sums, each region 256-byte aligned.
+struct ScanSegWs {
+  size_t state, dsum;
+};
+inline ScanSegWs scan_seg_ws(const ScanSegs& sg, int64_t batch, int64_t dim, int64_t dstate) {
+  if (sg.n <= 1) return {0, 0};
+  auto a256 = [](int64_t v) { return (size_t)((v + 255) & ~(int64_t)255); };
+  return {a256(batch * sg.n * dim * dstate * 4), a256(batch * sg.n * dim * 4)};
+}
 
 // v * m, with v taken from lane K of each 16-lane row (DPP row_newbcast:K
 // fused into the multiply). The DPP source must not have been written by a
@@ -131,12 +180,43 @@ __device__ __forceinline__ float sigmoid_f32(float x) {
 }
 
 
+// The workgroup's batch, segment and tiles [first, end) of the sequence.
+struct ScanSeg {
+  int b, seg, first, end;
+  bool last;
+  __device__ __forceinline__ ScanSeg(const ScanParams& p, int bk) {
+    b = bk / p.segs;
+    seg = bk - b * p.segs;
+    const int all = (p.seqlen + kScanT - 1) / kScanT;
+    first = seg * p.seg_tiles;
+    end = min(first + p.seg_tiles, all);
+    last = end == all;
+  }
+};
+
+// The state that enters the segment: the segments before it (kBwd: the adjoint
+// that enters it from those behind it), folded in order.
+template <bool kBwd>
+__device__ __forceinline__ float seg_enter(const ScanParams& p, const ScanSeg& sg, int d, int n, float a_scaled) {
+  float h = 0.0f;
+  const int count = kBwd ? p.segs - 1 - sg.seg : sg.seg;
+#pragma unroll 4
+  for (int i = 0; i < count; ++i) {
+    const int64_t at = ((int64_t)sg.b * p.segs + (kBwd ? p.segs - 1 - i : i)) * p.dim + d;
+    // (a zero state stays out of the product: a growing decay, A > 0, may overflow)
+    const float in = p.seg_state[at * p.dstate + n], decay = __builtin_amdgcn_exp2f(a_scaled * p.seg_dsum[at]);
+    h = h == 0.0f ? in : fmaf(decay, h, in);
+  }
+  return h;
+}
+
 // Workspace of the Mamba-1 backward, each region 256-byte aligned: the states
 // before every 16-step block, the per-channel-tile partial rows of a
 // variable dB / dC, the per-batch partials of dA / dD / ddelta_bias and of a
 // constant dB / dC.
 struct ScanBwdWs {
   size_t ck, partB, partC, dA, dD, dBc, dCc, total;
+  ScanSegWs seg;
 };
 
 inline ScanBwdWs scan_bwd_ws(int64_t batch, int64_t dim, int64_t seqlen, int64_t dstate,
@@ -149,11 +229,13 @@ inline ScanBwdWs scan_bwd_ws(int64_t batch, int64_t dim, int64_t seqlen, int64_t
   w.ck = a256(batch * nck * dim * dstate * 4);
   w.partB = bc ? 0 : a256(tiles * batch * ngroups * dstate * seqlen * 4);
   w.partC = cc ? 0 : a256(tiles * batch * ngroups * dstate * seqlen * 4);
-  w.dA = a256(batch * dim * dstate * 4);
-  w.dD = a256(batch * dim * 4);
+  const ScanSegs sg = scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags);
+  w.seg = scan_seg_ws(sg, batch, dim, dstate);
+  w.dA = a256(batch * sg.n * dim * dstate * 4);  // a partial per batch and segment
+  w.dD = a256(batch * sg.n * dim * 4);
   w.dBc = bc ? a256(batch * dim * dstate * 4) : 0;
   w.dCc = cc ? a256(batch * dim * dstate * 4) : 0;
-  w.total = w.ck + w.partB + w.partC + w.dA + 2 * w.dD + w.dBc + w.dCc;
+  w.total = w.ck + w.partB + w.partC + w.dA + 2 * w.dD + w.dBc + w.dCc + w.seg.state + w.seg.dsum;
   return w;
 }
 

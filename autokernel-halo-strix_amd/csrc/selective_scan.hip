@@ -48,7 +48,8 @@ mamba_scan_fwd_kernel(ScanParams p) {
   const int n = lane % 16;  // state owned by this lane
 
   const int per_batch = p.ngroups * p.tiles_per_group;
-  const int b = blockIdx.x / per_batch;
+  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
   const int tile = blockIdx.x % p.tiles_per_group;
   const int ch_local = tile * kScanCh + wave * 4 + c;  // channel index inside the group
@@ -68,7 +69,7 @@ mamba_scan_fwd_kernel(ScanParams p) {
   const int64_t B_base = (int64_t)b * p.B_bs + (int64_t)g * p.B_gs;
   const int64_t C_base = (int64_t)b * p.C_bs + (int64_t)g * p.C_gs;
 
-  float h = 0.0f;
+  float h = (ch_ok && n_ok) ? seg_enter<false>(p, sg, d, n, a_scaled) : 0.0f;
   float* hb = hbuf[wave];
 
   // Global loads for one 64-step tile, issued one tile ahead of their use so
@@ -140,9 +141,12 @@ mamba_scan_fwd_kernel(ScanParams p) {
   };
 
   float dsum = 0.0f;  // sum of delta' since step 0 (chunk states)
+  if (!kPrep && p.chunk_states)
+    for (int i = 0; i < sg.seg; ++i) dsum += p.seg_dsum[((int64_t)b * p.segs + i) * p.dim + d];
   TileRegs cur, nxt{};
-  load_tile(0, cur);
-  for (int l0 = 0; l0 < p.seqlen; l0 += kScanT) {
+  load_tile(sg.first * kScanT, cur);
+  const int l_end = min(sg.end * kScanT, p.seqlen);
+  for (int l0 = sg.first * kScanT; l0 < l_end; l0 += kScanT) {
     __syncthreads();  // previous tile's readers of Bs / Cs are done
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -163,7 +167,7 @@ mamba_scan_fwd_kernel(ScanParams p) {
     asm volatile("s_nop 1"
                  : "+v"(dl[0]), "+v"(dl[1]), "+v"(dl[2]), "+v"(dl[3]), "+v"(du[0]), "+v"(du[1]),
                    "+v"(du[2]), "+v"(du[3]));
-    if (l0 + kScanT < p.seqlen) load_tile(l0 + kScanT, nxt);
+    if (l0 + kScanT < l_end) load_tile(l0 + kScanT, nxt);
     // keep the compiler from sinking the prefetch towards its use
     asm volatile("" ::: "memory");
     __syncthreads();
@@ -257,7 +261,7 @@ mamba_scan_fwd_kernel(ScanParams p) {
     cur = nxt;
   }
   finish_pending();
-  if (!kPrep && p.last_state && ch_ok && n_ok) {
+  if (!kPrep && p.last_state && sg.last && ch_ok && n_ok) {
     p.last_state[((int64_t)b * p.dim + d) * p.dstate + n] = h;
   }
 }
@@ -669,9 +673,17 @@ mamba_scan_fast_kernel(ScanParams p) {
 // the chunk states); or kPrepGated: the backward's preparation pass with a
 // gate (checkpoints by the producers, dz = dout y sigma(z) (1 + z (1 -
 // sigma(z))) by the consumers).
+//
+// kRag: any sequence length from 4 on and any row alignment. The four-element
+// loads then take any address, in the sequence's last, partial tile from the
+// last four elements on (shifted into place), steps past the end get delta' = 0
+// (which leaves the state as it is) and store nothing. Against
+// mamba_scan_fwd_kernel, which took these lengths before: [1, 2048, 1777] bf16
+// (four segments, both passes) 52.0 -> 42.5 us, [2, 1536, 300] fp16 18.4 -> 12.1,
+// [4, 1536, 300] bf16 23.8 -> 16.8.
 enum { kPrepGated = 3 };
 
-template <typename TU, typename TD, typename TBC, bool kSoftplus, int kMode>
+template <typename TU, typename TD, typename TBC, bool kSoftplus, int kMode, bool kRag>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 mamba_scan_split_kernel(ScanParams p) {
   constexpr bool kPrep = kMode == kPrepGated;
@@ -691,7 +703,8 @@ mamba_scan_split_kernel(ScanParams p) {
   const int c = lane / 16;
   const int n = lane % 16;
   const int per_batch = p.ngroups * p.tiles_per_group;
-  const int b = blockIdx.x / per_batch;
+  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
   const int tile = blockIdx.x % p.tiles_per_group;
   const int d0 = g * p.ch_per_group + tile * kScanCh;
@@ -699,7 +712,7 @@ mamba_scan_split_kernel(ScanParams p) {
   const int d = d0 + wc;
   const bool n_ok = n < p.dstate;
   const uint32_t L = (uint32_t)p.seqlen;
-  const int nt = p.seqlen / kScanT;
+  const int t0 = sg.first, nt = sg.end - sg.first;  // tiles t0 .. t0 + nt - 1; t below counts from t0
   auto row_rsrc = [&](const void* base, int64_t bs, int64_t ds, int esz) {
     const char* q = static_cast<const char*>(base) + ((int64_t)b * bs + (int64_t)d0 * ds) * esz;
     return make_rsrc(q, (uint32_t)(((kScanCh - 1) * ds + L) * esz));
@@ -710,6 +723,18 @@ mamba_scan_split_kernel(ScanParams p) {
   const int sn = r % 16, q = r / 16;
   const int sn_c = min(sn, p.dstate - 1);
   const bool s_ok = sn < p.dstate;
+  // the sequence's partial tile (kRag), or -1; how far the four steps from
+  // `step` on of that tile start behind the last four of the sequence
+  const int tail = kRag && p.seqlen % kScanT ? p.seqlen / kScanT : -1;
+  auto past = [&](int step) { return max(tail * kScanT + step - (p.seqlen - 4), 0); };
+  // four elements of tile T (counted from the sequence's start): vo the lane's
+  // offset of step `step` in tile 0
+  auto ld4 = [&](auto tag, const Rsrc& rs, const void* base, uint32_t vo, int step, int T) {
+    using E = decltype(tag);
+    const uint32_t l0 = (uint32_t)T * kScanT * sizeof(E);
+    if constexpr (!kRag) return bload4<E>(rs, vo, l0);
+    else return gload4_any<E>(base, vo + l0 - (T == tail ? (uint32_t)past(step) * sizeof(E) : 0u));
+  };
 
   if (producer) {
     __builtin_amdgcn_s_setprio(2);
@@ -718,7 +743,10 @@ mamba_scan_split_kernel(ScanParams p) {
     const Rsrc rs_u = row_rsrc(p.u, p.u_bs, p.u_ds, sizeof(TU));
     const Rsrc rs_d = row_rsrc(p.delta, p.d_bs, p.d_ds, sizeof(TD));
     const uint32_t bc_bytes_B = (uint32_t)(((p.dstate - 1) * p.B_ns + L) * sizeof(TBC));
-    const Rsrc rs_B = make_rsrc(static_cast<const TBC*>(p.B) + (int64_t)b * p.B_bs + (int64_t)g * p.B_gs, bc_bytes_B);
+    const TBC* const base_B = static_cast<const TBC*>(p.B) + (int64_t)b * p.B_bs + (int64_t)g * p.B_gs;
+    const TU* const base_u = static_cast<const TU*>(p.u) + (int64_t)b * p.u_bs + (int64_t)d0 * p.u_ds;
+    const TD* const base_d = static_cast<const TD*>(p.delta) + (int64_t)b * p.d_bs + (int64_t)d0 * p.d_ds;
+    const Rsrc rs_B = make_rsrc(base_B, bc_bytes_B);
     const uint32_t vo_d4 = (uint32_t)(wc * p.d_ds + 4 * n) * sizeof(TD);  // delta, steps 4n..4n+3
     const uint32_t vo_u4 = (uint32_t)(wc * p.u_ds + 4 * n) * sizeof(TU);
     const uint32_t vo_B = (uint32_t)(sn_c * p.B_ns + 4 * q) * sizeof(TBC);
@@ -732,29 +760,36 @@ mamba_scan_split_kernel(ScanParams p) {
       Raw4<TU> uv;
     };
     auto load_regs = [&](int t, Regs& rr) {
-      const uint32_t l0 = (uint32_t)t * kScanT;
-      rr.dv = bload4<TD>(rs_d, vo_d4, l0 * sizeof(TD));
-      rr.uv = bload4<TU>(rs_u, vo_u4, l0 * sizeof(TU));
+      rr.dv = ld4(TD{}, rs_d, base_d, vo_d4, 4 * n, t0 + t);
+      rr.uv = ld4(TU{}, rs_u, base_u, vo_u4, 4 * n, t0 + t);
     };
-    auto write_B = [&](const Raw4<TBC>& v, int buf) {
+    auto write_B = [&](Raw4<TBC> v, int t) {
+      const int buf = t & 1;
+      if (kRag && t0 + t == tail) raw4_drop<TBC>(v, min(past(4 * q), 4));
 #pragma unroll
       for (int k = 0; k < 4; ++k) Bs[buf][sn * kBStride + 4 * q + k] = s_ok ? raw4_f32<TBC>(v, k) : 0.0f;
     };
-    Raw4<TBC> sv = bload4<TBC>(rs_B, vo_B, 0u);
+    Raw4<TBC> sv = ld4(TBC{}, rs_B, base_B, vo_B, 4 * q, t0);
     Regs ra, rb;
     load_regs(0, ra);
     write_B(sv, 0);
-    sv = bload4<TBC>(rs_B, vo_B, (uint32_t)min(1, nt - 1) * kScanT * sizeof(TBC));
+    sv = ld4(TBC{}, rs_B, base_B, vo_B, 4 * q, t0 + min(1, nt - 1));
     __syncthreads();
-    float h = 0.0f;
+    float h = n_ok ? seg_enter<false>(p, sg, d, n, a_scaled) : 0.0f;
     float dsum = 0.0f;  // sum of delta' since step 0 (chunk states)
+    if (xs_out)
+      for (int i = 0; i < sg.seg; ++i) dsum += p.seg_dsum[((int64_t)b * p.segs + i) * p.dim + d];
     // Tile t: stage tile t + 1's B (its buffer was last read in tile t - 1,
     // before the barrier that ended it), issue the loads of tile t + 2's B
     // and tile t + 1's delta / u (clamped to the last tile), then the four
     // blocks, each ending with the states written and a barrier.
-    auto tile_body = [&](int t, const Regs& cur, Regs& nxt) {
-      write_B(sv, (t + 1) & 1);
-      sv = bload4<TBC>(rs_B, vo_B, (uint32_t)min(t + 2, nt - 1) * kScanT * sizeof(TBC));
+    auto tile_body = [&](int t, Regs& cur, Regs& nxt) {
+      if (kRag && t0 + t == tail) {
+        raw4_drop<TD>(cur.dv, min(past(4 * n), 4));
+        raw4_drop<TU>(cur.uv, min(past(4 * n), 4));
+      }
+      write_B(sv, t + 1);
+      sv = ld4(TBC{}, rs_B, base_B, vo_B, 4 * q, t0 + min(t + 2, nt - 1));
       load_regs(min(t + 1, nt - 1), nxt);
       asm volatile("" ::: "memory");
       const int buf = t & 1;
@@ -764,6 +799,7 @@ mamba_scan_split_kernel(ScanParams p) {
       for (int k = 0; k < 4; ++k) {
         float dv = raw4_f32<TD>(cur.dv, k) + dbias;
         if constexpr (kSoftplus) dv = softplus_f32(dv);
+        if (kRag && (t0 + t) * kScanT + 4 * n + k >= p.seqlen) dv = 0.0f;
         dl[k] = dv;
         du[k] = dv * raw4_f32<TU>(cur.uv, k);
       }
@@ -819,14 +855,15 @@ mamba_scan_split_kernel(ScanParams p) {
       if (has_ck && n_ok) {
 #pragma unroll
         for (int blk = 0; blk < kScanT / 16; ++blk)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, hck[blk]), rs_ck, (int)vo_ck,
-                                                (int)((uint32_t)((t * kScanT + 16 * blk) / kCk) * ck_chunk_bytes), 0);
+          if (!kRag || (t0 + t) * kScanT + 16 * blk < p.seqlen)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, hck[blk]), rs_ck, (int)vo_ck,
+                                                  (int)((uint32_t)(((t0 + t) * kScanT + 16 * blk) / kCk) * ck_chunk_bytes), 0);
       }
       if (xs_out) {
         // the channel's delta' over the tile, then (decay product, state) at
         // each 2048-step chunk end
         dsum += row16_sum((dl[0] + dl[1]) + (dl[2] + dl[3]));
-        const int l1 = (t + 1) * kScanT;
+        const int l1 = (t0 + t + 1) * kScanT;
         if ((l1 % kXChunk == 0 || l1 >= p.seqlen) && n_ok) {
           float* xs = xs_out + ((((int64_t)b * p.dim + d) * p.xchunks + (l1 - 1) / kXChunk) * p.dstate + n) * 2;
           xs[0] = __builtin_amdgcn_exp2f(a_scaled * dsum);
@@ -838,7 +875,7 @@ mamba_scan_split_kernel(ScanParams p) {
       tile_body(t, ra, rb);
       if (t + 1 < nt) tile_body(t + 1, rb, ra);
     }
-    if (!kPrep && p.last_state && n_ok) p.last_state[((int64_t)b * p.dim + d) * p.dstate + n] = h;
+    if (!kPrep && p.last_state && sg.last && n_ok) p.last_state[((int64_t)b * p.dim + d) * p.dstate + n] = h;
   } else {
     const float dskip = p.D ? p.D[d] : 0.0f;
     const Rsrc rs_u = row_rsrc(p.u, p.u_bs, p.u_ds, sizeof(TU));
@@ -850,7 +887,8 @@ mamba_scan_split_kernel(ScanParams p) {
     const Rsrc rs_oz = has_prez ? row_rsrc(p.out_prez, p.o_bs, p.o_ds, sizeof(TU)) : rs_o;
     const Rsrc rs_go = kPrep ? row_rsrc(p.dout, p.go_bs, p.go_ds, sizeof(TU)) : rs_u;
     const uint32_t bc_bytes_C = (uint32_t)(((p.dstate - 1) * p.C_ns + L) * sizeof(TBC));
-    const Rsrc rs_C = make_rsrc(static_cast<const TBC*>(p.C) + (int64_t)b * p.C_bs + (int64_t)g * p.C_gs, bc_bytes_C);
+    const TBC* const base_C = static_cast<const TBC*>(p.C) + (int64_t)b * p.C_bs + (int64_t)g * p.C_gs;
+    const Rsrc rs_C = make_rsrc(base_C, bc_bytes_C);
     // lane (c, n) forms step 16 blk + n of channel wc
     const uint32_t vo_u1 = (uint32_t)(wc * p.u_ds + n) * sizeof(TU);
     const uint32_t vo_z1 = (uint32_t)(wc * zds + n) * sizeof(TU);
@@ -862,7 +900,7 @@ mamba_scan_split_kernel(ScanParams p) {
       Raw1<TU> go[kPrep ? 4 : 1];
     };
     auto load_regs = [&](int t, Regs& rr) {
-      const uint32_t l0 = (uint32_t)t * kScanT;
+      const uint32_t l0 = (uint32_t)(t0 + t) * kScanT;
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk) {
         rr.uo[blk] = bload1<TU>(rs_u, vo_u1 + 16 * blk * sizeof(TU), l0 * sizeof(TU));
@@ -870,15 +908,17 @@ mamba_scan_split_kernel(ScanParams p) {
         if constexpr (kPrep) rr.go[blk] = bload1<TU>(rs_go, vo_go1 + 16 * blk * sizeof(TU), l0 * sizeof(TU));
       }
     };
-    auto write_C = [&](const Raw4<TBC>& v, int buf) {
+    auto write_C = [&](Raw4<TBC> v, int t) {
+      const int buf = t & 1;
+      if (kRag && t0 + t == tail) raw4_drop<TBC>(v, min(past(4 * q), 4));
 #pragma unroll
       for (int k = 0; k < 4; ++k) Cs[buf][(4 * q + k) * kCStride + sn] = s_ok ? raw4_f32<TBC>(v, k) : 0.0f;
     };
-    Raw4<TBC> sv = bload4<TBC>(rs_C, vo_C, 0u);
+    Raw4<TBC> sv = ld4(TBC{}, rs_C, base_C, vo_C, 4 * q, t0);
     Regs ra, rb;
     load_regs(0, ra);
     write_C(sv, 0);
-    sv = bload4<TBC>(rs_C, vo_C, (uint32_t)min(1, nt - 1) * kScanT * sizeof(TBC));
+    sv = ld4(TBC{}, rs_C, base_C, vo_C, 4 * q, t0 + min(1, nt - 1));
     __syncthreads();
     // Tile t: after each block's barrier, that block's states are complete;
     // after the first, stage tile t + 1's C (its buffer was last read for
@@ -889,8 +929,8 @@ mamba_scan_split_kernel(ScanParams p) {
       for (int blk = 0; blk < kScanT / 16; ++blk) {
         __syncthreads();
         if (blk == 0) {
-          write_C(sv, (t + 1) & 1);
-          sv = bload4<TBC>(rs_C, vo_C, (uint32_t)min(t + 2, nt - 1) * kScanT * sizeof(TBC));
+          write_C(sv, t + 1);
+          sv = ld4(TBC{}, rs_C, base_C, vo_C, 4 * q, t0 + min(t + 2, nt - 1));
           load_regs(min(t + 1, nt - 1), nxt);
           asm volatile("" ::: "memory");
         }
@@ -912,17 +952,18 @@ mamba_scan_split_kernel(ScanParams p) {
         float o = fmaf(dskip, raw_f32<TU>(cur.uo[blk]), ysum);
         asm("" : "+v"(o));
         const float zv = raw_f32<TU>(cur.zo[blk]);
-        const uint32_t off = vo_o1 + ((uint32_t)t * kScanT + 16 * blk) * sizeof(TU);
+        const uint32_t off = vo_o1 + ((uint32_t)(t0 + t) * kScanT + 16 * blk) * sizeof(TU);
+        const bool live = !kRag || (t0 + t) * kScanT + 16 * blk + n < p.seqlen;
         float v;
         if constexpr (kPrep) {
           const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-zv * kLog2e));
           v = raw_f32<TU>(cur.go[blk]) * o * sg * fmaf(zv, 1.0f - sg, 1.0f);
         } else {
-          if (has_prez) bstore1<TU>(rs_oz, off, o);
+          if (has_prez && live) bstore1<TU>(rs_oz, off, o);
           v = has_z ? o * silu_fast(zv) : o;
         }
         asm("" : "+v"(v));
-        bstore1<TU>(rs_o, off, v);
+        if (live) bstore1<TU>(rs_o, off, v);
       }
     };
     for (int t = 0; t < nt; t += 2) {
@@ -1656,6 +1697,145 @@ diag_bwd_chunk_kernel(const float* __restrict__ dA, const float* __restrict__ dB
 }
 
 // ---------------------------------------------------------------------------
+// The segment pass (scan_segments): the lanes and tiles of
+// mamba_scan_fwd_kernel without its outputs, VALU-bound (two DPP multiplies, an
+// exp2 and an FMA a step and state: [1, 2048, 1777] 18 us for 3 of 4 segments).
+// kBwd = false: every segment's state from zero and sum of delta', for all
+// segments but the last. kBwd: the adjoint that a segment passes to the step
+// before it, c_{l-1} = a_l (c_l + dy_l C_l) from c = 0, for all but the first.
+// ---------------------------------------------------------------------------
+template <typename TU, typename TD, typename TBC, bool kBwd>
+__global__ void __launch_bounds__(256)
+mamba_scan_seg_kernel(ScanParams p) {
+  __shared__ float Bs[2][16 * kBStride];  // B (kBwd: C) of a tile, double-buffered
+  const int tid = threadIdx.x;
+  const int wave = tid / 64, lane = tid % 64;
+  const int c = lane / 16, n = lane % 16;
+  const int per_batch = p.ngroups * p.tiles_per_group;
+  const int bs = blockIdx.x / per_batch;
+  const int b = bs / (p.segs - 1), seg = bs % (p.segs - 1) + (kBwd ? 1 : 0);
+  const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
+  const int ch_local = (blockIdx.x % p.tiles_per_group) * kScanCh + wave * 4 + c;
+  const bool ch_ok = ch_local < p.ch_per_group;
+  const int d = g * p.ch_per_group + (ch_ok ? ch_local : 0);
+  const bool n_ok = n < p.dstate;
+  const float a_scaled = (ch_ok && n_ok) ? p.A[(int64_t)d * p.A_ds + n] * kLog2e : 0.0f;
+  const float dbias = p.delta_bias ? p.delta_bias[d] : 0.0f;
+
+  const TD* const drow = static_cast<const TD*>(p.delta) + (int64_t)b * p.d_bs + (int64_t)d * p.d_ds;
+  const TU* const xrow = kBwd ? static_cast<const TU*>(p.dout) + (int64_t)b * p.go_bs + (int64_t)d * p.go_ds
+                              : static_cast<const TU*>(p.u) + (int64_t)b * p.u_bs + (int64_t)d * p.u_ds;
+  const TU* const zrow = kBwd && p.z ? static_cast<const TU*>(p.z) + (int64_t)b * p.z_bs + (int64_t)d * p.z_ds : xrow;
+  const int sn = tid / 16, q = tid % 16;
+  const int sn_c = min(sn, p.dstate - 1);
+  const TBC* const brow = kBwd ? static_cast<const TBC*>(p.C) + (int64_t)b * p.C_bs + (int64_t)g * p.C_gs + (int64_t)sn_c * p.C_ns
+                               : static_cast<const TBC*>(p.B) + (int64_t)b * p.B_bs + (int64_t)g * p.B_gs + (int64_t)sn_c * p.B_ns;
+
+  const int first = seg * p.seg_tiles;
+  const int end = min(first + p.seg_tiles, (p.seqlen + kScanT - 1) / kScanT);
+  const int nt = end - first;
+  // the i-th tile that is walked, in steps
+  auto step0 = [&](int i) { return (kBwd ? end - 1 - i : first + i) * kScanT; };
+
+  // loads from clamped, always-valid addresses, masked and converted at the
+  // use; the inputs come two tiles ahead
+  const int last_l = p.seqlen - 1;
+  TBC bv[4];
+  struct In {
+    TD d[4];
+    TU x[4], z[4];
+  };
+  auto load_B = [&](int i) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bv[k] = brow[min(step0(i) + 4 * q + k, last_l)];
+  };
+  auto load_x = [&](int i, In& r) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int l = min(step0(i) + 4 * n + k, last_l);
+      r.d[k] = drow[l];
+      r.x[k] = xrow[l];
+      if constexpr (kBwd) r.z[k] = zrow[l];
+    }
+  };
+  auto write_B = [&](int i) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      Bs[i & 1][sn * kBStride + 4 * q + k] = sn < p.dstate && step0(i) + 4 * q + k < p.seqlen ? to_f32(bv[k]) : 0.0f;
+  };
+
+  float h = 0.0f, dsum = 0.0f;
+  In xa, xb;
+  load_B(0);
+  load_x(0, xa);
+  load_x(min(1, nt - 1), xb);
+  write_B(0);
+  if (nt > 1) load_B(1);
+  auto tile = [&](int i, In& cur) {
+    __syncthreads();  // tile i is staged, and nobody reads tile i - 1's buffer any more
+    float dl[4], xi[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool ok = ch_ok && step0(i) + 4 * n + k < p.seqlen;
+      float dvv = to_f32(cur.d[k]) + dbias;
+      if (p.softplus) dvv = softplus_f32(dvv);
+      dl[k] = ok ? dvv : 0.0f;
+      const float x = to_f32(cur.x[k]);
+      if constexpr (kBwd) {
+        const float z = to_f32(cur.z[k]);
+        xi[k] = ok ? (p.z ? x * z * sigmoid_f32(z) : x) : 0.0f;
+      } else {
+        xi[k] = dl[k] * x;
+      }
+    }
+    // wait states between the last VALU write of dl / xi and their DPP reads
+    asm volatile("s_nop 1"
+                 : "+v"(dl[0]), "+v"(dl[1]), "+v"(dl[2]), "+v"(dl[3]), "+v"(xi[0]), "+v"(xi[1]),
+                   "+v"(xi[2]), "+v"(xi[3]));
+    if (i + 1 < nt) {
+      write_B(i + 1);
+      load_x(min(i + 2, nt - 1), cur);
+      if (i + 2 < nt) load_B(i + 2);
+    }
+    asm volatile("" ::: "memory");
+    auto block = [&](auto blk_c) {
+      constexpr int BLK = decltype(blk_c)::value;
+      float bt[16], av[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) bt[j] = Bs[i & 1][n * kBStride + 16 * BLK + j];
+      static_for<0, 16>([&](auto j_c) {
+        constexpr int J = decltype(j_c)::value;
+        av[J] = mul_bcast<4 * BLK + J / 4>(dl[J % 4], a_scaled);
+        if constexpr (!kBwd) bt[J] = mul_bcast<4 * BLK + J / 4>(xi[J % 4], bt[J]);
+      });
+#pragma unroll
+      for (int j = 0; j < 16; ++j) av[j] = __builtin_amdgcn_exp2f(av[j]);
+      static_for<0, 16>([&](auto j_c) {
+        if constexpr (kBwd) {
+          constexpr int J = 15 - decltype(j_c)::value;
+          h = av[J] * fma_bcast<4 * BLK + J / 4>(xi[J % 4], bt[J], h);
+        } else {
+          constexpr int J = decltype(j_c)::value;
+          h = fmaf(av[J], h, bt[J]);
+        }
+      });
+    };
+    static_for<0, 4>([&](auto i_c) {
+      constexpr int I = decltype(i_c)::value;
+      block(std::integral_constant<int, kBwd ? 3 - I : I>{});
+    });
+    dsum += row16_sum((dl[0] + dl[1]) + (dl[2] + dl[3]));
+  };
+  for (int i = 0; i < nt; i += 2) {
+    tile(i, xa);
+    if (i + 1 < nt) tile(i + 1, xb);
+  }
+  const int64_t at = ((int64_t)b * p.segs + seg) * p.dim + d;
+  if (ch_ok && n_ok) p.seg_state[at * p.dstate + n] = h;
+  if (ch_ok && n == 0) p.seg_dsum[at] = dsum;
+}
+
+// ---------------------------------------------------------------------------
 // Mamba-1 backward (the gradient of selective_scan_ref; the reference's
 // kernel is external/mamba/csrc/selective_scan/selective_scan_bwd_kernel.cuh,
 // entry point selective_scan.cpp:339-490). With delta' = softplus?(delta +
@@ -1697,7 +1877,8 @@ mamba_scan_bwd_kernel(ScanParams p) {
   const int n = lane % 16;
 
   const int per_batch = p.ngroups * p.tiles_per_group;
-  const int b = blockIdx.x / per_batch;
+  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
   const int tile = blockIdx.x % p.tiles_per_group;
   const int ch_local = tile * kScanCh + wave * 4 + c;
@@ -1771,14 +1952,16 @@ mamba_scan_bwd_kernel(ScanParams p) {
   // dy = dout * silu(z) (dout without a gate)
   auto gated = [&](float go, float zv) { return p.z ? go * zv * sigmoid_f32(zv) : go; };
 
-  float gs = 0.0f;       // gradient of the state after the step being processed
-  float a_next = 0.0f;   // decay of the step after it
+  // gradient of the state after the step being processed, decay of the step
+  // after it; they start from the adjoint of the segments behind this one
+  float gs = (ch_ok && n_ok) ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f;
+  float a_next = 1.0f;
   float dA_acc = 0.0f;
   float dD_acc = 0.0f, dbias_acc = 0.0f;  // reducer role: channel c, steps 16 blk + n
 
   TileRegs cur, nxt{};
-  load_tile((last_l / kScanT) * kScanT, cur);
-  for (int l0 = (last_l / kScanT) * kScanT; l0 >= 0; l0 -= kScanT) {
+  load_tile((sg.end - 1) * kScanT, cur);
+  for (int l0 = (sg.end - 1) * kScanT; l0 >= sg.first * kScanT; l0 -= kScanT) {
     __syncthreads();  // the previous tile's readers of Bs / Cs / wbuf are done
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1800,7 +1983,7 @@ mamba_scan_bwd_kernel(ScanParams p) {
     asm volatile("s_nop 1"
                  : "+v"(bd[0]), "+v"(bd[1]), "+v"(bd[2]), "+v"(bd[3]), "+v"(bdu[0]), "+v"(bdu[1]),
                    "+v"(bdu[2]), "+v"(bdu[3]), "+v"(bdy[0]), "+v"(bdy[1]), "+v"(bdy[2]), "+v"(bdy[3]));
-    if (l0 > 0) load_tile(l0 - kScanT, nxt);
+    if (l0 > sg.first * kScanT) load_tile(l0 - kScanT, nxt);
     // keep the compiler from sinking the prefetch towards its use
     asm volatile("" ::: "memory");
     __syncthreads();
@@ -1923,12 +2106,13 @@ mamba_scan_bwd_kernel(ScanParams p) {
     }
     cur = nxt;
   }
-  if (ch_ok && n_ok) p.dA_part[((int64_t)b * p.dim + d) * p.dstate + n] = dA_acc;
+  const int64_t bd_row = (int64_t)(blockIdx.x / per_batch) * p.dim + d;  // partials per batch and segment
+  if (ch_ok && n_ok) p.dA_part[bd_row * p.dstate + n] = dA_acc;
   dD_acc = row16_sum(dD_acc);
   dbias_acc = row16_sum(dbias_acc);
   if (ch_ok && n == 0) {
-    p.dD_part[(int64_t)b * p.dim + d] = dD_acc;
-    p.dbias_part[(int64_t)b * p.dim + d] = dbias_acc;
+    p.dD_part[bd_row] = dD_acc;
+    p.dbias_part[bd_row] = dbias_acc;
   }
 }
 
@@ -2068,9 +2252,10 @@ __global__ void __launch_bounds__(256) scan_bwd_finalize_kernel(FinArgs<TBC> a) 
 // Whether the fast kernel's layout assumptions hold: whole 64-step tiles,
 // whole 16-channel workgroups, 4-element aligned rows for the vector loads,
 // and every buffer resource's extent (16 channel rows, or dstate B / C rows)
-// below 2 GiB.
+// below 2 GiB. rag: those of the split kernel's kRag form, which takes any
+// length from 4 steps on and any alignment.
 template <typename TU, typename TD, typename TBC>
-bool scan_fast_ok(const ScanParams& p, bool prep = false, int wgc = kScanCh) {
+bool scan_fast_ok(const ScanParams& p, bool prep = false, int wgc = kScanCh, bool rag = false) {
   auto al4 = [](const void* ptr, int64_t s0, int64_t s1, int64_t s2, size_t esz) {
     return (reinterpret_cast<uintptr_t>(ptr) % (4 * esz)) == 0 && s0 % 4 == 0 && s1 % 4 == 0 &&
            s2 % 4 == 0;
@@ -2078,10 +2263,9 @@ bool scan_fast_ok(const ScanParams& p, bool prep = false, int wgc = kScanCh) {
   auto fits = [&](int64_t rows, int64_t pitch, size_t esz) {
     return pitch >= 0 && ((rows - 1) * pitch + p.seqlen) * (int64_t)esz < ((int64_t)1 << 31);
   };
-  if (p.seqlen % kScanT != 0 || p.ch_per_group % wgc != 0) return false;
-  if (!al4(p.u, p.u_bs, p.u_ds, 0, sizeof(TU)) || !al4(p.delta, p.d_bs, p.d_ds, 0, sizeof(TD)))
-    return false;
-  if (!al4(p.B, p.B_bs, p.B_gs, p.B_ns, sizeof(TBC)) || !al4(p.C, p.C_bs, p.C_gs, p.C_ns, sizeof(TBC)))
+  if (p.ch_per_group % wgc != 0 || (rag ? p.seqlen < 4 : p.seqlen % kScanT != 0)) return false;
+  if (!rag && (!al4(p.u, p.u_bs, p.u_ds, 0, sizeof(TU)) || !al4(p.delta, p.d_bs, p.d_ds, 0, sizeof(TD)) ||
+               !al4(p.B, p.B_bs, p.B_gs, p.B_ns, sizeof(TBC)) || !al4(p.C, p.C_bs, p.C_gs, p.C_ns, sizeof(TBC))))
     return false;
   if (p.u_bs < 0 || p.d_bs < 0 || p.o_bs < 0 || p.z_bs < 0 || p.B_bs < 0 || p.C_bs < 0 ||
       p.B_gs < 0 || p.C_gs < 0)
@@ -2093,27 +2277,35 @@ bool scan_fast_ok(const ScanParams& p, bool prep = false, int wgc = kScanCh) {
          fits(p.dstate, p.B_ns, sizeof(TBC)) && fits(p.dstate, p.C_ns, sizeof(TBC));
 }
 
+// Producer / consumer waves for whole tiles, and in their kRag form for other
+// lengths and alignments. Returns whether they take the call.
+template <typename TU, typename TD, typename TBC, int kMode>
+bool launch_split(const ScanParams& p, int grid, hipStream_t s) {
+  constexpr bool kPrep = kMode == kPrepGated;
+  const bool whole = scan_fast_ok<TU, TD, TBC>(p, kPrep);
+  if (!whole && !scan_fast_ok<TU, TD, TBC>(p, kPrep, kScanCh, true)) return false;
+  const dim3 g(grid), t(512);
+  if (whole && p.softplus) mamba_scan_split_kernel<TU, TD, TBC, true, kMode, false><<<g, t, 0, s>>>(p);
+  else if (whole) mamba_scan_split_kernel<TU, TD, TBC, false, kMode, false><<<g, t, 0, s>>>(p);
+  else if (p.softplus) mamba_scan_split_kernel<TU, TD, TBC, true, kMode, true><<<g, t, 0, s>>>(p);
+  else mamba_scan_split_kernel<TU, TD, TBC, false, kMode, true><<<g, t, 0, s>>>(p);
+  return true;
+}
+
 template <typename TU, typename TD, typename TBC>
 void launch_scan(const ScanParams& p, hipStream_t s) {
-  const int grid = p.batch * p.ngroups * p.tiles_per_group;
+  const int groups = p.batch * p.ngroups * p.tiles_per_group;
+  const int grid = groups * p.segs;
+  if (p.segs > 1)
+    mamba_scan_seg_kernel<TU, TD, TBC, false><<<dim3(groups * (p.segs - 1)), dim3(256), 0, s>>>(p);
+  // inference and training variants fixed at compile time, any other
+  // combination of outputs at run time
   const bool lean = p.z && !p.out_prez && !p.ck && !p.chunk_states;
   const bool train = p.z && p.out_prez && p.ck && !p.chunk_states;
-  // whole tiles: producer / consumer waves (inference and training variants
-  // fixed at compile time, any other combination of outputs at run time)
-  if (scan_fast_ok<TU, TD, TBC>(p) && lean && p.softplus)
-    mamba_scan_split_kernel<TU, TD, TBC, true, kFwdLean><<<dim3(grid), dim3(512), 0, s>>>(p);
-  else if (scan_fast_ok<TU, TD, TBC>(p) && lean)
-    mamba_scan_split_kernel<TU, TD, TBC, false, kFwdLean><<<dim3(grid), dim3(512), 0, s>>>(p);
-  else if (scan_fast_ok<TU, TD, TBC>(p) && train && p.softplus)
-    mamba_scan_split_kernel<TU, TD, TBC, true, kFwdTrain><<<dim3(grid), dim3(512), 0, s>>>(p);
-  else if (scan_fast_ok<TU, TD, TBC>(p) && train)
-    mamba_scan_split_kernel<TU, TD, TBC, false, kFwdTrain><<<dim3(grid), dim3(512), 0, s>>>(p);
-  else if (scan_fast_ok<TU, TD, TBC>(p) && p.softplus)
-    mamba_scan_split_kernel<TU, TD, TBC, true, kFwdAny><<<dim3(grid), dim3(512), 0, s>>>(p);
-  else if (scan_fast_ok<TU, TD, TBC>(p))
-    mamba_scan_split_kernel<TU, TD, TBC, false, kFwdAny><<<dim3(grid), dim3(512), 0, s>>>(p);
-  else
-    mamba_scan_fwd_kernel<TU, TD, TBC><<<dim3(grid), dim3(256), 0, s>>>(p);
+  const bool done = lean ? launch_split<TU, TD, TBC, kFwdLean>(p, grid, s)
+                  : train ? launch_split<TU, TD, TBC, kFwdTrain>(p, grid, s)
+                          : launch_split<TU, TD, TBC, kFwdAny>(p, grid, s);
+  if (!done) mamba_scan_fwd_kernel<TU, TD, TBC><<<dim3(grid), dim3(256), 0, s>>>(p);
 }
 
 // dstate in (16, 64] with variable B / C: the specialised kernel with 2 or 4
@@ -2177,7 +2369,7 @@ void scan_bwd_finish(const ScanParams& p, void* dB, void* dC, float* dA, float* 
   const size_t out4 = 4 * sizeof(TBC);
   auto al4 = [&](const void* q) { return !q || reinterpret_cast<uintptr_t>(q) % out4 == 0; };
   FinArgs<TBC> fa{p.dB_part, p.dC_part, p.dA_part, p.dBc_part, p.dCc_part, p.dD_part, p.dbias_part,
-                  dBv, dCv, dA, dBk, dCk, dD, dbias, nbc, p.tiles_per_group, p.batch, p.dim, p.dstate};
+                  dBv, dCv, dA, dBk, dCk, dD, dbias, nbc, p.tiles_per_group, p.batch * p.segs, p.dim, p.dstate};
   if (nbc > 0 && nbc % 4 == 0 && al4(dBv) && al4(dCv)) {
     // one launch: the vector dB / dC sums, then blocks for the per-batch sums
     const int64_t n4 = nbc / 4;
@@ -2215,19 +2407,24 @@ constexpr int dtype_code_of() {
 template <typename TU, typename TD, typename TBC>
 void launch_scan_bwd(const ScanParams& p, void* dB, void* dC, float* dA, float* dD, float* dbias,
                      bool saved_states, hipStream_t s) {
-  const int grid = p.batch * p.ngroups * p.tiles_per_group;
+  const int groups = p.batch * p.ngroups * p.tiles_per_group;
+  const int grid = groups * p.segs;
+  const dim3 seg_grid(groups * (p.segs - 1));
   if (!saved_states) {  // preparation pass: states every 16 steps and dz
-    if (scan_fast_ok<TU, TD, TBC>(p, true) && p.z && p.softplus)
-      mamba_scan_split_kernel<TU, TD, TBC, true, kPrepGated><<<dim3(grid), dim3(512), 0, s>>>(p);
-    else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.z)
-      mamba_scan_split_kernel<TU, TD, TBC, false, kPrepGated><<<dim3(grid), dim3(512), 0, s>>>(p);
-    else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.softplus)
+    if (p.segs > 1) mamba_scan_seg_kernel<TU, TD, TBC, false><<<seg_grid, dim3(256), 0, s>>>(p);
+    if (p.z && launch_split<TU, TD, TBC, kPrepGated>(p, grid, s)) {
+      // producer / consumer waves
+    } else if (p.z) {
+      mamba_scan_fwd_kernel<TU, TD, TBC, true><<<dim3(grid), dim3(256), 0, s>>>(p);
+    }
+    else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1 && p.softplus)
       mamba_scan_fast_kernel<TU, TD, TBC, true, true><<<dim3(grid), dim3(256), 0, s>>>(p);
-    else if (scan_fast_ok<TU, TD, TBC>(p, true))
+    else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1)
       mamba_scan_fast_kernel<TU, TD, TBC, false, true><<<dim3(grid), dim3(256), 0, s>>>(p);
     else
       mamba_scan_fwd_kernel<TU, TD, TBC, true><<<dim3(grid), dim3(256), 0, s>>>(p);
   }
+  if (p.segs > 1) mamba_scan_seg_kernel<TU, TD, TBC, true><<<seg_grid, dim3(256), 0, s>>>(p);
   ScanParams q = p;  // the whole-tile pass may write fewer, wider dB / dC partial rows
   if (launch_scan_bwd_fast(q, dtype_code_of<TU>(), dtype_code_of<TD>(), dtype_code_of<TBC>(), s)) {
     // whole tiles: the buffer-resource reverse pass
@@ -2285,7 +2482,18 @@ int scan_common_args(const char* name, ScanParams& p, int64_t batch, int64_t dim
   p.c_const = (bc_flags & AK_SCAN_C_CONST) ? 1 : 0;
   p.nchunks = (int)((seqlen + kCk - 1) / kCk);
   p.xchunks = (int)((seqlen + kXChunk - 1) / kXChunk);
+  p.segs = 1;  // the callers that have scratch for segments set them (use_segments)
+  p.seg_tiles = (int)((seqlen + kScanT - 1) / kScanT);
   return AK_OK;
+}
+
+// The scan's segments, with their states and sums in `scratch` (scan_seg_ws).
+void use_segments(ScanParams& p, const ScanSegs& sg, const ScanSegWs& ws, char* scratch) {
+  if (sg.n <= 1) return;
+  p.segs = sg.n;
+  p.seg_tiles = sg.tiles;
+  p.seg_state = reinterpret_cast<float*>(scratch);
+  p.seg_dsum = reinterpret_cast<float*>(scratch + ws.state);
 }
 
 // B / C strides: variable ([batch, ngroups, dstate, seqlen]) or constant
@@ -2301,7 +2509,11 @@ void scan_bc_strides(ScanParams& p, int64_t B_bs, int64_t B_gs, int64_t B_ns, in
 }  // namespace
 }  // namespace ak
 
-extern "C" int ak_selective_scan_fwd(
+namespace ak {
+namespace {
+// The forward entry points; without a workspace the scan runs in one segment.
+int scan_fwd_entry(
+    const char* name, void* workspace, size_t workspace_bytes,
     const void* u, const void* delta, const float* A, const void* B, const void* C,
     const float* D, const void* z, const float* delta_bias, void* out, float* last_state,
     void* out_prez, float* chunk_states, float* checkpoints, int64_t batch, int64_t dim,
@@ -2312,7 +2524,6 @@ extern "C" int ak_selective_scan_fwd(
     int64_t C_group_stride, int64_t C_state_stride, int64_t z_batch_stride, int64_t z_dim_stride,
     int64_t out_batch_stride, int64_t out_dim_stride, int delta_softplus, int bc_flags,
     int u_dtype, int delta_dtype, int bc_dtype, int a_dtype, void* stream) {
-  const char* name = "ak_selective_scan_fwd";
   ak::ScanParams p{};
   int bc_eff = 0;
   int rc = ak::scan_common_args(name, p, batch, dim, seqlen, dstate, ngroups, bc_flags, u_dtype,
@@ -2331,6 +2542,14 @@ extern "C" int ak_selective_scan_fwd(
   p.z_bs = z_batch_stride; p.z_ds = z_dim_stride; p.o_bs = out_batch_stride; p.o_ds = out_dim_stride;
   p.softplus = delta_softplus ? 1 : 0;
   hipStream_t s = ak_stream(stream);
+  if (workspace && a_dtype != AK_DTYPE_C64) {
+    const ak::ScanSegs sg = ak::scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags);
+    const ak::ScanSegWs ws = ak::scan_seg_ws(sg, batch, dim, dstate);
+    if (workspace_bytes < ws.state + ws.dsum)
+      return ak_set_error(AK_ERR_WORKSPACE, "%s: workspace %zu bytes < required %zu", name,
+                          workspace_bytes, ws.state + ws.dsum);
+    ak::use_segments(p, sg, ws, static_cast<char*>(workspace));
+  }
   if (a_dtype == AK_DTYPE_C64) {
     if (ak::launch_scan_complex_fwd(p, u_dtype, delta_dtype, bc_eff, s))
       return ak_set_error(AK_ERR_UNSUPPORTED, "%s: delta and a variable B/C must be fp32 or the dtype of u", name);
@@ -2357,6 +2576,58 @@ extern "C" int ak_selective_scan_fwd(
   }
   if (rc) return ak_set_error(AK_ERR_UNSUPPORTED, "%s: delta and a variable B/C must be fp32 or the dtype of u", name);
   return ak_check_launch(name);
+}
+}  // namespace
+}  // namespace ak
+
+extern "C" int ak_selective_scan_fwd(
+    const void* u, const void* delta, const float* A, const void* B, const void* C,
+    const float* D, const void* z, const float* delta_bias, void* out, float* last_state,
+    void* out_prez, float* chunk_states, float* checkpoints, int64_t batch, int64_t dim,
+    int64_t seqlen, int64_t dstate, int64_t ngroups,
+    int64_t u_batch_stride, int64_t u_dim_stride, int64_t delta_batch_stride,
+    int64_t delta_dim_stride, int64_t A_dim_stride, int64_t B_batch_stride,
+    int64_t B_group_stride, int64_t B_state_stride, int64_t C_batch_stride,
+    int64_t C_group_stride, int64_t C_state_stride, int64_t z_batch_stride, int64_t z_dim_stride,
+    int64_t out_batch_stride, int64_t out_dim_stride, int delta_softplus, int bc_flags,
+    int u_dtype, int delta_dtype, int bc_dtype, int a_dtype, void* stream) {
+  return ak::scan_fwd_entry(
+      "ak_selective_scan_fwd", nullptr, 0,
+      u, delta, A, B, C, D, z, delta_bias, out, last_state, out_prez, chunk_states, checkpoints, batch,
+      dim, seqlen, dstate, ngroups, u_batch_stride, u_dim_stride, delta_batch_stride, delta_dim_stride,
+      A_dim_stride, B_batch_stride, B_group_stride, B_state_stride, C_batch_stride, C_group_stride,
+      C_state_stride, z_batch_stride, z_dim_stride, out_batch_stride, out_dim_stride, delta_softplus,
+      bc_flags, u_dtype, delta_dtype, bc_dtype, a_dtype, stream);
+}
+
+extern "C" size_t ak_selective_scan_fwd_workspace_bytes(int64_t batch, int64_t dim, int64_t seqlen,
+                                                       int64_t dstate, int64_t ngroups, int bc_flags) {
+  if (batch <= 0 || dim <= 0 || seqlen <= 0 || dstate <= 0 || ngroups <= 0 || dim % ngroups) return 0;
+  if (bc_flags & AK_SCAN_A_COMPLEX) return 0;
+  const ak::ScanSegWs ws = ak::scan_seg_ws(
+      ak::scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags), batch, dim, dstate);
+  return ws.state + ws.dsum;
+}
+
+extern "C" int ak_selective_scan_fwd_ws(
+    const void* u, const void* delta, const float* A, const void* B, const void* C,
+    const float* D, const void* z, const float* delta_bias, void* out, float* last_state,
+    void* out_prez, float* chunk_states, float* checkpoints, int64_t batch, int64_t dim,
+    int64_t seqlen, int64_t dstate, int64_t ngroups,
+    int64_t u_batch_stride, int64_t u_dim_stride, int64_t delta_batch_stride,
+    int64_t delta_dim_stride, int64_t A_dim_stride, int64_t B_batch_stride,
+    int64_t B_group_stride, int64_t B_state_stride, int64_t C_batch_stride,
+    int64_t C_group_stride, int64_t C_state_stride, int64_t z_batch_stride, int64_t z_dim_stride,
+    int64_t out_batch_stride, int64_t out_dim_stride, int delta_softplus, int bc_flags,
+    int u_dtype, int delta_dtype, int bc_dtype, int a_dtype, void* workspace, size_t workspace_bytes,
+    void* stream) {
+  return ak::scan_fwd_entry(
+      "ak_selective_scan_fwd_ws", workspace, workspace_bytes,
+      u, delta, A, B, C, D, z, delta_bias, out, last_state, out_prez, chunk_states, checkpoints, batch,
+      dim, seqlen, dstate, ngroups, u_batch_stride, u_dim_stride, delta_batch_stride, delta_dim_stride,
+      A_dim_stride, B_batch_stride, B_group_stride, B_state_stride, C_batch_stride, C_group_stride,
+      C_state_stride, z_batch_stride, z_dim_stride, out_batch_stride, out_dim_stride, delta_softplus,
+      bc_flags, u_dtype, delta_dtype, bc_dtype, a_dtype, stream);
 }
 
 extern "C" int ak_diag_scan_fwd(const float* dA, const float* dBx, const float* C, const float* D,
@@ -2591,6 +2862,7 @@ extern "C" int ak_selective_scan_bwd(
   p.dbias_part = take(ws.dD);
   p.dBc_part = take(ws.dBc);
   p.dCc_part = take(ws.dCc);
+  ak::use_segments(p, ak::scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags), ws.seg, w + off);
   // saved forward states: the reverse pass reads them (and out_prez) in place
   if (checkpoints) {
     p.ck = const_cast<float*>(checkpoints);

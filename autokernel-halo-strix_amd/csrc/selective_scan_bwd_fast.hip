@@ -54,7 +54,8 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
   const int n = lane % 16;
   const int tpg = p.tiles_per_group;  // whole kCh-channel tiles
   const int per_batch = p.ngroups * tpg;
-  const int b = blockIdx.x / per_batch;
+  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / tpg;
   const int tile = blockIdx.x % tpg;
   const int d0 = g * p.ch_per_group + tile * kCh;
@@ -133,8 +134,11 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
     r.ck = __builtin_amdgcn_raw_buffer_load_b32(rs_ck, (int)vo_ck, (int)((l / kCk) * (uint32_t)ck_cs * 4u), 0);
   };
 
-  float gs = 0.0f, a_next = 0.0f, dA_acc = 0.0f, dD_acc = 0.0f, dbias_acc = 0.0f;
-  const int nt = p.seqlen / kScanT;
+  // the adjoint of the segments behind this one, as the product of a step's
+  // state gradient and the decay that follows it
+  float gs = n_ok ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f, a_next = 1.0f;
+  float dA_acc = 0.0f, dD_acc = 0.0f, dbias_acc = 0.0f;
+  const int t_lo = sg.first, nt = sg.end;  // tiles nt - 1 down to t_lo
   Raw4<TBC> bv{}, cv{};
   if (stager) {
     bv = bload4<TBC>(rs_B, vo_B, (uint32_t)(nt - 1) * kScanT * sizeof(TBC));
@@ -152,7 +156,7 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
   float st_du[4], st_dd[4], st_dz[4];
   const uint32_t vo_o4 = (uint32_t)(wc * p.o_ds + 4 * n) * sizeof(TU);
   const uint32_t vo_dd4 = (uint32_t)(wc * p.o_ds + 4 * n) * sizeof(TD);
-  for (int t = nt - 1; t >= 0; --t) {
+  for (int t = nt - 1; t >= t_lo; --t) {
     const int l0 = t * kScanT;
     __syncthreads();
     if (stager) {
@@ -325,12 +329,13 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
       }
     }
   }
-  if (n_ok) p.dA_part[((int64_t)b * p.dim + d) * p.dstate + n] = dA_acc;
+  const int64_t bd_row = (int64_t)(blockIdx.x / per_batch) * p.dim + d;  // partials per batch and segment
+  if (n_ok) p.dA_part[bd_row * p.dstate + n] = dA_acc;
   dD_acc = row16_sum(dD_acc);
   dbias_acc = row16_sum(dbias_acc);
   if (n == 0) {
-    p.dD_part[(int64_t)b * p.dim + d] = dD_acc;
-    p.dbias_part[(int64_t)b * p.dim + d] = dbias_acc;
+    p.dD_part[bd_row] = dD_acc;
+    p.dbias_part[bd_row] = dbias_acc;
   }
 }
 
@@ -370,11 +375,11 @@ bool launch_fast(ScanParams& p, hipStream_t s) {
   // channels, so it depends on the shape alone and the bits of every
   // gradient are the same on any device or partition.
   constexpr int64_t kWideMinGroups = 256;
-  const bool wide = p.ch_per_group % 32 == 0 && scan_bwd_fast_ok<TU, TD, TBC>(p, 32) &&
+  const bool wide = p.segs == 1 && p.ch_per_group % 32 == 0 && scan_bwd_fast_ok<TU, TD, TBC>(p, 32) &&
                     (int64_t)p.batch * p.ngroups * (p.ch_per_group / 32) >= kWideMinGroups;
   if (!wide && !scan_bwd_fast_ok<TU, TD, TBC>(p, kScanCh)) return false;
   if (wide) p.tiles_per_group = p.ch_per_group / 32;
-  const int grid = p.batch * p.ngroups * p.tiles_per_group;
+  const int grid = p.batch * p.segs * p.ngroups * p.tiles_per_group;
   const bool gate = p.z != nullptr, dz = gate && p.out_prez != nullptr;
   auto go = [&](auto sp, auto gt, auto dzt) {
     constexpr bool kSp = decltype(sp)::value, kGt = decltype(gt)::value, kDzt = decltype(dzt)::value;

@@ -78,6 +78,9 @@ _SIGNATURES = {
     "ak_lmhead_grad_weight": [_c_void_p, _i64, _c_void_p, _i64, _c_void_p, _i64, _i64, _i64, _i64,
                               _int, _c_void_p, ctypes.c_size_t, _int, _c_void_p],
     "ak_selective_scan_fwd": [_c_void_p] * 13 + [_i64] * 5 + [_i64] * 15 + [_int] * 6 + [_c_void_p],
+    "ak_selective_scan_fwd_ws": [_c_void_p] * 13 + [_i64] * 5 + [_i64] * 15 + [_int] * 6
+    + [_c_void_p, ctypes.c_size_t, _c_void_p],
+    "ak_selective_scan_fwd_workspace_bytes": [_i64] * 5 + [_int],
     "ak_diag_scan_fwd": [_c_void_p] * 6 + [_i64] * 3 + [_c_void_p],
     "ak_diag_scan_bwd_workspace_bytes": [_i64, _i64],
     "ak_diag_scan_bwd": [_c_void_p] * 12 + [ctypes.c_size_t] + [_i64] * 3 + [_c_void_p],
@@ -93,6 +96,7 @@ _RESTYPES = {
     "ak_rmsnorm_bwd_workspace_bytes": ctypes.c_size_t,
     "ak_diag_scan_bwd_workspace_bytes": ctypes.c_size_t,
     "ak_selective_scan_bwd_workspace_bytes": ctypes.c_size_t,
+    "ak_selective_scan_fwd_workspace_bytes": ctypes.c_size_t,
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
@@ -630,15 +634,19 @@ def selective_scan(u, delta, A, B, C, D, z, delta_bias, out, last_state, delta_s
     dstate = A.shape[1]
     flags, bs, cs, ngroups, bc_dtype = _scan_bc(B, C)
     zs = (z.stride(0), z.stride(1)) if z is not None else (0, 0)
+    lib = load()
+    ws_bytes = int(lib.ak_selective_scan_fwd_workspace_bytes(
+        batch, dim, seqlen, dstate, ngroups, flags | (SCAN_A_COMPLEX if A.is_complex() else 0)))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=u.device) if ws_bytes else None
     with _on_device(u):
-        rc = load().ak_selective_scan_fwd(
+        rc = lib.ak_selective_scan_fwd_ws(
             _ptr(u), _ptr(delta), _ptr(A), _ptr(B), _ptr(C), _ptr(D), _ptr(z), _ptr(delta_bias),
             _ptr(out), _ptr(last_state), _ptr(out_prez), _ptr(chunk_states), _ptr(checkpoints),
             batch, dim, seqlen, dstate, ngroups,
             u.stride(0), u.stride(1), delta.stride(0), delta.stride(1), A.stride(0),
             *bs, *cs, zs[0], zs[1], out.stride(0), out.stride(1),
             int(bool(delta_softplus)), flags, dtype_code(u.dtype), dtype_code(delta.dtype),
-            bc_dtype, _a_code(A), _stream(u))
+            bc_dtype, _a_code(A), _ptr(ws), ws_bytes, _stream(u))
     _check(rc, "ak_selective_scan_fwd")
 
 

@@ -416,6 +416,35 @@ int ak_selective_scan_fwd(const void* u, const void* delta, const float* A,
                           int u_dtype, int delta_dtype, int bc_dtype, int a_dtype, void* stream);
 
 /*
+ * ak_selective_scan_fwd with scratch: a scan with few (channel, state) lanes
+ * (dstate <= 16, variable B / C) is cut into segments of the sequence that run
+ * side by side, after a pass over each segment's own state
+ * (scan_segments in csrc/scan_common.h). workspace must hold
+ * ak_selective_scan_fwd_workspace_bytes() bytes (0 where the shape runs in one
+ * segment; bc_flags as for ak_selective_scan_bwd_workspace_bytes); NULL runs
+ * every shape in one segment.
+ */
+size_t ak_selective_scan_fwd_workspace_bytes(int64_t batch, int64_t dim, int64_t seqlen,
+                                             int64_t dstate, int64_t ngroups, int bc_flags);
+int ak_selective_scan_fwd_ws(const void* u, const void* delta, const float* A,
+                          const void* B, const void* C, const float* D,
+                          const void* z, const float* delta_bias,
+                          void* out, float* last_state, void* out_prez, float* chunk_states,
+                          float* checkpoints,
+                          int64_t batch, int64_t dim, int64_t seqlen,
+                          int64_t dstate, int64_t ngroups,
+                          int64_t u_batch_stride, int64_t u_dim_stride,
+                          int64_t delta_batch_stride, int64_t delta_dim_stride,
+                          int64_t A_dim_stride,
+                          int64_t B_batch_stride, int64_t B_group_stride, int64_t B_state_stride,
+                          int64_t C_batch_stride, int64_t C_group_stride, int64_t C_state_stride,
+                          int64_t z_batch_stride, int64_t z_dim_stride,
+                          int64_t out_batch_stride, int64_t out_dim_stride,
+                          int delta_softplus, int bc_flags,
+                          int u_dtype, int delta_dtype, int bc_dtype, int a_dtype, void* workspace, size_t workspace_bytes,
+    void* stream);
+
+/*
  * Mamba-1 selective scan backward: every input gradient of
  * ak_selective_scan_fwd's output given dout. Replaces selective_scan_cuda.bwd,
  * external/mamba/csrc/selective_scan/selective_scan.cpp:339-490, as called by

@@ -361,3 +361,81 @@ def test_saved_states_c_abi():
         grads.append(g)
     for name, a, b in zip(NAMES, *grads):
         assert (a is None and b is None) or torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("itype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("batch,dim,seqlen,groups,opts", [
+    (1, 16, 4, 1, "Dzb"), (1, 16, 63, 1, "z"), (2, 32, 193, 1, "Dzb"), (1, 16, 255, 1, "Dzb"), (1, 32, 256, 2, "Dzb"),
+    (1, 16, 321, 1, ""), (1, 24, 700, 1, "Dzb"), (1, 16, 2111, 1, "Dzb"), (3, 64, 1025, 2, "zb"), (8, 384, 1537, 1, "Dzb")])
+def test_segments_and_ragged_lengths(itype, batch, dim, seqlen, groups, opts):
+    """Sequences cut into segments (from 4 tiles on, one to several tiles each;
+    (8, 384, 1537) takes the plan of 192 channel groups) and every length's
+    partial tile, from views that start off the alignment grid: outputs, last
+    state, chunk states and gradients against the one-segment call (states and
+    outputs equal to fp32 rounding: |h| times 2e-6 a step boundary, and one
+    rounding of the output type) and the oracle; the saved-states and recomputed
+    backwards bitwise alike; neighbours of the outputs untouched."""
+    need_gpu()
+    from kernels.hip import _lib, selective_scan as ss
+    dt = ITYPES[itype]
+    args = _inputs(batch, dim, 16, seqlen, groups, dt, seqlen + dim)
+    u, delta, A, B, C, D, z, bias, dout = args
+    say("scan segments", itype, batch, dim, seqlen, groups, opts)
+
+    def odd(t):  # the same values, rows one element off the grid
+        if t is None:
+            return None
+        v = torch.zeros(t.shape[:-1] + (t.shape[-1] + 3,), dtype=t.dtype, device=DEV)
+        v[..., 1:1 + t.shape[-1]] = t.to(DEV)
+        return v[..., 1:1 + t.shape[-1]]
+
+    D, z, bias = (t if o in opts else None for t, o in ((D, "D"), (z, "z"), (bias, "b")))
+    dev = [odd(u), odd(delta), A.to(DEV), odd(B), odd(C)] + [None if t is None else t.to(DEV) for t in (D,)] + \
+          [odd(z), None if bias is None else bias.to(DEV)]
+    runs = []
+    for segmented in (True, False):
+        ob = torch.full((batch, dim, seqlen + 2), 7.0, dtype=dt, device=DEV)
+        out, last = ob[..., 1:1 + seqlen], torch.full((batch, dim, 16), 7.0, device=DEV)
+        xs = torch.full((batch, dim, -(-seqlen // 2048), 16, 2), 7.0, device=DEV)
+        ck = torch.full((batch, -(-seqlen // 16), dim, 16), 7.0, device=DEV)
+        with pytest.MonkeyPatch.context() as m:
+            if not segmented:  # no workspace: one segment
+                lib = _lib.load()
+                one = lib.ak_selective_scan_fwd_ws
+
+                class Lib:
+                    def __getattr__(self, name):
+                        return getattr(lib, name)
+
+                    def ak_selective_scan_fwd_workspace_bytes(self, *a):
+                        return 0
+
+                    def ak_selective_scan_fwd_ws(self, *a):
+                        return one(*a)
+
+                m.setattr(_lib, "load", lambda: Lib())
+            _lib.selective_scan(*dev[:5], dev[5], dev[6], dev[7], out, last, True, chunk_states=xs, checkpoints=ck)
+        assert bool((ob[..., 0] == 7).all()) and bool((ob[..., -1] == 7).all())
+        runs.append([t.double().cpu() for t in (out, last, xs, ck)])
+    ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dt]
+    for got, one, unit in zip(runs[0], runs[1], (ulp, 0.0, 0.0, 0.0)):
+        scale = one.abs().amax()
+        assert bool(((got - one).abs() <= unit * one.abs() + 4e-6 * scale).all())
+    ref = ops.selective_scan_ref(u, delta, A, B, C, D, z, bias, True)
+    rt, at = GRID["tolerances"][itype]
+    assert torch.allclose(runs[0][0].float(), ref.float(), rtol=rt, atol=at)
+
+    got = _gpu_grads(u, delta, A, B, C, D, z, bias, dout, True)
+    ss.set_save_states(False)
+    try:
+        again = _gpu_grads(u, delta, A, B, C, D, z, bias, dout, True)
+    finally:
+        ss.set_save_states(True)
+    for i, (a, b) in enumerate(zip(got, again)):  # (dz comes from the rounded output where it was kept)
+        assert a is b is None or i == 6 or torch.equal(a, b), NAMES[i]
+    bref = ops.selective_scan_bwd_ref(u, delta, A, B, C, dout, D, z, bias, True)
+    tols = _tols(itype, z is not None)
+    for name in ("dA", "dD", "ddelta_bias"):  # sums over many more steps than the grid's shapes
+        r, a = tols[name]
+        tols[name] = (r, a * max(1.0, batch * seqlen / 512) ** 0.5)
+    _check(got, bref, tols, (u, delta, A, B, C, D, z, bias))
