@@ -142,6 +142,26 @@ __device__ __forceinline__ u32x2 lds_read_tr(uint32_t addr) {
   return v;
 }
 
+// Four rows x four columns of a lane quad, transposed and rounded to T: lane j
+// of the quad holds column j's rows 0 .. 3 in x and returns row j's columns
+// 0 .. 3 in order. Pairs of 16-bit values are exchanged with lane j ^ 1, then
+// pairs of pairs with lane j ^ 2 (all lanes must be active).
+template <typename T>
+__device__ __forceinline__ u32x2 quad_rows(const float (&x)[4], int lane) {
+  auto swap = [](uint32_t v, auto ctrl) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xF, 0xF, false);
+  };
+  using Xor1 = std::integral_constant<int, kDppXor1>;
+  using Xor2 = std::integral_constant<int, kDppXor2>;
+  const uint32_t p01 = pack2<T>(x[0], x[1]), p23 = pack2<T>(x[2], x[3]);
+  const uint32_t sel = lane & 1 ? 0x03020706u : 0x05040100u;
+  const uint32_t a01 = __builtin_amdgcn_perm(swap(p01, Xor1{}), p01, sel);  // row 0 (1 in odd lanes), its column pair
+  const uint32_t a23 = __builtin_amdgcn_perm(swap(p23, Xor1{}), p23, sel);  // row 2 (3)
+  const bool up = lane & 2;
+  const uint32_t r = swap(up ? a01 : a23, Xor2{});
+  return up ? u32x2{r, a23} : u32x2{a01, r};
+}
+
 template <typename T, bool kAMn>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 lmhead_grad_gemm_kernel(GemmArgs g) {
@@ -382,15 +402,40 @@ lmhead_grad_gemm_kernel(GemmArgs g) {
     const int ml = wv * 128 + 4 * khalf;  // + 32 vb + 8 (r / 4) + r % 4
     const int nl = wt * 128 + fr;         // + 32 tb
     if (x.pslot >= 0) {
-      float* pt = g.part + (int64_t)x.pslot * (kGT * kGT) + ml * kGT + nl;
+      // partial tiles lie as the registers do, [wave][vb][tb][r / 4][lane][r % 4]:
+      // 16-byte stores of whole kilobytes, read back alike by the reduce pass
+      float4* const pt = reinterpret_cast<float4*>(g.part) + (int64_t)x.pslot * (kGT * kGT / 4) + wave * 4096 + lane;
 #pragma unroll
       for (int vb = 0; vb < 4; ++vb)
 #pragma unroll
         for (int tb = 0; tb < 4; ++tb) {
-          float* q = pt + 32 * vb * kGT + 32 * tb;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) q[(8 * (r >> 2) + (r & 3)) * kGT] = acc_read(acc[vb][tb][r]);
+          for (int r4 = 0; r4 < 4; ++r4)
+            pt[((vb * 4 + tb) * 4 + r4) * 64] =
+                make_float4(acc_read(acc[vb][tb][4 * r4]), acc_read(acc[vb][tb][4 * r4 + 1]),
+                            acc_read(acc[vb][tb][4 * r4 + 2]), acc_read(acc[vb][tb][4 * r4 + 3]));
           __builtin_amdgcn_sched_barrier(0);  // one block's addresses live at a time
+        }
+    } else if (g.out_mode == kOutT) {
+      // rows of four columns a lane (quad_rows): 64 8-byte stores a lane instead
+      // of 256 2-byte ones, and no per-element tests (d % 4 == 0). grad_W of 1024
+      // tokens x 32768 x 768 bf16 @@GW@@.
+      const int nq = n0 + wt * 128 + (fr & ~3), mq = m0 + ml + (lane & 3);
+      T* const cq = static_cast<T*>(g.c) + (int64_t)mq * g.ldc + nq;
+#pragma unroll
+      for (int vb = 0; vb < 4; ++vb)
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) {
+          T* const q = cq + (int64_t)(32 * vb) * g.ldc + 32 * tb;
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const float v[4] = {acc_read(acc[vb][tb][4 * r4]), acc_read(acc[vb][tb][4 * r4 + 1]),
+                                acc_read(acc[vb][tb][4 * r4 + 2]), acc_read(acc[vb][tb][4 * r4 + 3])};
+            const u32x2 w = quad_rows<T>(v, lane);
+            if (mq + 32 * vb + 8 * r4 < g.m && nq + 32 * tb < g.n)
+              *reinterpret_cast<u32x2_any*>(q + (int64_t)(8 * r4) * g.ldc) = w;
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
     } else {
 #pragma unroll
@@ -406,8 +451,7 @@ lmhead_grad_gemm_kernel(GemmArgs g) {
             const float v = acc_read(acc[vb][tb][r]);
             if (mb + dm < g.m && n < g.n) {
               const int64_t oo = o + (int64_t)dm * g.ldc;
-              if (g.out_mode == kOutT) static_cast<T*>(g.c)[oo] = from_f32<T>(v);
-              else if (g.out_mode == kOutF32) static_cast<float*>(g.c)[oo] = v;
+              if (g.out_mode == kOutF32) static_cast<float*>(g.c)[oo] = v;
               else static_cast<float*>(g.c)[oo] += v;
             }
           }
@@ -420,20 +464,20 @@ lmhead_grad_gemm_kernel(GemmArgs g) {
 }
 
 // Sum of the S partial tiles of each split tile, in the order of their K
-// ranges, into C. Grid (rest tiles, 64) x 256 threads: one float4 of the
-// 256 x 256 tile per thread.
+// ranges, into C. Grid (rest tiles, 64) x 256 threads: one float4 (four rows
+// of a column, as the tile kernel stored them) per thread.
 template <typename T>
 __global__ void __launch_bounds__(256) lmhead_grad_reduce_kernel(GemmArgs g) {
   const int rest = g.n_tm * g.n_tn - g.n_full;
   const int ti = blockIdx.x;  // split tile index (partial slot of range 0)
   const int q = blockIdx.y * 256 + threadIdx.x;
-  const int row = q >> 6, col = 4 * (q & 63);
+  const int lane = q & 63, r4 = (q >> 6) & 3, blk = (q >> 8) & 15, wave = q >> 12;
   const int t = g.n_full + ti;
-  const int m = (t / g.n_tn) * kGT + row;
-  const int n = (t % g.n_tn) * kGT + col;
-  if (m >= g.m || n >= g.n) return;  // n < N implies n + 3 < N (N % 8 == 0)
+  const int m = (t / g.n_tn) * kGT + (wave >> 1) * 128 + 32 * (blk >> 2) + 8 * r4 + 4 * (lane >> 5);
+  const int n = (t % g.n_tn) * kGT + (wave & 1) * 128 + 32 * (blk & 3) + (lane & 31);
   const float4* p = reinterpret_cast<const float4*>(g.part) + (int64_t)ti * (kGT * kGT / 4) + q;
   float4 s = p[0];
+#pragma unroll 4
   for (int k = 1; k < g.split; ++k) {
     const float4 v = p[(int64_t)k * rest * (kGT * kGT / 4)];
     s.x += v.x;
@@ -441,26 +485,21 @@ __global__ void __launch_bounds__(256) lmhead_grad_reduce_kernel(GemmArgs g) {
     s.z += v.z;
     s.w += v.w;
   }
-  const int64_t o = (int64_t)m * g.ldc + n;
+  const float v[4] = {s.x, s.y, s.z, s.w};
   if (g.out_mode == kOutT) {
-    T* c = static_cast<T*>(g.c) + o;
-    c[0] = from_f32<T>(s.x);
-    c[1] = from_f32<T>(s.y);
-    c[2] = from_f32<T>(s.z);
-    c[3] = from_f32<T>(s.w);
-  } else {
-    float* c = static_cast<float*>(g.c) + o;
-    if (g.out_mode == kOutF32Add) {
-      c[0] += s.x;
-      c[1] += s.y;
-      c[2] += s.z;
-      c[3] += s.w;
-    } else {
-      c[0] = s.x;
-      c[1] = s.y;
-      c[2] = s.z;
-      c[3] = s.w;
-    }
+    const u32x2 w = quad_rows<T>(v, lane);
+    const int mr = m + (lane & 3), nq = n & ~3;
+    if (mr < g.m && nq < g.n)  // nq < N implies nq + 3 < N (N % 8 == 0)
+      *reinterpret_cast<u32x2_any*>(static_cast<T*>(g.c) + (int64_t)mr * g.ldc + nq) = w;
+    return;
+  }
+  if (n >= g.n) return;
+  float* const c = static_cast<float*>(g.c) + n;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (m + i >= g.m) break;
+    float* const e = c + (int64_t)(m + i) * g.ldc;
+    *e = g.out_mode == kOutF32Add ? *e + v[i] : v[i];
   }
 }
 
