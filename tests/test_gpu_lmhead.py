@@ -369,6 +369,32 @@ def test_lmhead_ce_grad_logits_pitch_fallback():
     assert torch.equal(a, b[:, :1152])
 
 
+@pytest.mark.parametrize("n,vocab", [(256, 257), (300, 383), (255, 385), (256, 391), (300, 516), (257, 640), (7, 1030)])
+def test_lmhead_ce_grad_logits_vocab_edges(n, vocab):
+    """Vocabularies around the 128-row halves and 256-row tiles, rows at an odd
+    element address and pitch: whole halves, groups of four and single elements
+    each stay inside their row. Within one bf16 rounding of float64."""
+    need_gpu()
+    from kernels.hip import _lib
+    d = 64
+    g = torch.Generator().manual_seed(n * vocab)
+    h = torch.randn(n, d, generator=g).bfloat16()
+    W = (0.05 * torch.randn(vocab, d, generator=g)).bfloat16()
+    t = torch.randint(0, vocab, (n,), generator=g)
+    t[0], t[-1] = 0, vocab - 1
+    say("lmhead grad logits edges", n, vocab)
+    _, lse, nv, _ = _run(h, W, t)
+    den = nv.to(torch.float32).clamp(min=1.0).reshape(1)
+    ldv = vocab + 6 - vocab % 2  # pitch even, rows all at odd elements
+    buf = torch.full((n * ldv + 1,), 5.0, dtype=torch.bfloat16, device=DEV)
+    dz = buf[1:].view(n, ldv)
+    _lib.lmhead_ce_bwd(h.to(DEV), W.to(DEV), t.to(DEV), lse, torch.ones(1, device=DEV), den, dz, -100)
+    ref = _dz_ref(h, W, t, lse.cpu(), 1.0 / float(den))
+    err = (dz[:, :vocab].double().cpu() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + 1e-6 / float(den)).all()), float(err.max())
+    assert bool((dz[:, vocab:].float() == 5.0).all()) and float(buf[0]) == 5.0
+
+
 def test_lmhead_ce_grad_bad_target_rows_are_nan():
     need_gpu()
     from kernels.hip import _lib
