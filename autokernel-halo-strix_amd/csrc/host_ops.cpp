@@ -34,7 +34,7 @@ using Maybe = std::optional<Tensor>;
   X(ak_ce_count_valid) X(ak_ce_mean) X(ak_scale_inplace) X(ak_diag_scan_fwd)                       \
   X(ak_diag_scan_bwd_workspace_bytes) X(ak_diag_scan_bwd) X(ak_selective_scan_fwd_ws) X(ak_selective_scan_fwd_workspace_bytes)                 \
   X(ak_selective_scan_bwd_workspace_bytes) X(ak_selective_scan_bwd)                                \
-  X(ak_lmhead_ce_workspace_bytes) X(ak_lmhead_ce_fwd) X(ak_lmhead_ce_bwd_range)                    \
+  X(ak_lmhead_ce_workspace_bytes) X(ak_lmhead_ce_fwd_denom) X(ak_lmhead_ce_bwd_range)                    \
   X(ak_lmhead_grad_workspace_bytes) X(ak_lmhead_grad_hidden) X(ak_lmhead_grad_weight)
 
 #define AK_FIELD(n) decltype(&::n) n = nullptr;
@@ -535,10 +535,11 @@ struct LmHead : torch::autograd::Function<LmHead> {
     Tensor loss = f32_like(h, {}), lse = f32_like(h, {n});
     const size_t bytes = api.ak_lmhead_ce_workspace_bytes(n, v);
     Tensor ws = bytes_like(h, bytes);
-    check(api.ak_lmhead_ce_fwd(h.data_ptr(), w.data_ptr(), i64p(t), f32p(loss), f32p(lse), nullptr, nullptr, ws.data_ptr(), bytes,
-                               n, v, d, d, d, ignore, (float)cap, (float)smoothing, code_of(h.scalar_type()), stream_of(h)),
-          "ak_lmhead_ce_fwd");
-    ctx->save_for_backward({h, w, t, lse});
+    Tensor denom = f32_like(h, {1});
+    check(api.ak_lmhead_ce_fwd_denom(h.data_ptr(), w.data_ptr(), i64p(t), f32p(loss), f32p(lse), nullptr, nullptr, f32p(denom),
+                                     ws.data_ptr(), bytes, n, v, d, d, d, ignore, (float)cap, (float)smoothing,
+                                     code_of(h.scalar_type()), stream_of(h)), "ak_lmhead_ce_fwd");
+    ctx->save_for_backward({h, w, t, lse, denom});
     ctx->saved_data["ignore"] = ignore;
     ctx->saved_data["p"] = std::vector<double>{cap, smoothing};
     return loss;
@@ -549,13 +550,11 @@ struct LmHead : torch::autograd::Function<LmHead> {
     const auto p = ctx->saved_data["p"].toDoubleVector();
     const bool need_h = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
     const Tensor h = s[0].contiguous(), w = s[1].contiguous(), t = s[2].contiguous(), lse = s[3].contiguous();
+    const Tensor denom = s[4].contiguous();  // max(1, #counted rows)
     const Tensor up = g[0].detach().to(at::kFloat).contiguous();
     const int64_t n = h.size(0), d = h.size(1), v = w.size(0);
     const int code = code_of(h.scalar_type());
     void* st = stream_of(h);
-    // [max(1, #counted rows), its reciprocal]
-    Tensor denom = f32_like(h, {2});
-    check(api.ak_ce_count_valid(i64p(t), n, ignore, f32p(denom), st), "ak_ce_count_valid");
     // dlogits: the pitch covers whole 64-column K blocks and stays off powers
     // of two, whose rows would all start in the same memory channels
     const int64_t padded = (v + 63) / 64 * 64;

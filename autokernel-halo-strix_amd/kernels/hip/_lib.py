@@ -70,6 +70,7 @@ _SIGNATURES = {
     "ak_lmhead_ce_fwd": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                          _c_void_p, ctypes.c_size_t, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32,
                          _int, _c_void_p],
+    "ak_lmhead_ce_fwd_denom": [_c_void_p] * 9 + [ctypes.c_size_t] + [_i64] * 6 + [_f32, _f32, _int, _c_void_p],
     "ak_lmhead_ce_bwd": [_c_void_p] * 7 + [_i64] * 7 + [_f32, _f32, _int, _c_void_p],
     "ak_lmhead_ce_bwd_range": [_c_void_p] * 7 + [_i64] * 9 + [_f32, _f32, _int, _c_void_p],
     "ak_lmhead_grad_workspace_bytes": [_i64, _i64, _i64],

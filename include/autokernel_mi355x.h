@@ -264,6 +264,14 @@ int ak_lmhead_ce_fwd(const void* hidden, const void* weight, const int64_t* targ
                      int64_t n_rows, int64_t vocab, int64_t d,
                      int64_t ld_h, int64_t ld_w, int64_t ignore_index,
                      float softcap, float label_smoothing, int dtype, void* stream);
+/* ak_lmhead_ce_fwd that also writes denom[0] = max(1, #non-ignored rows) as
+ * fp32 (nullable), the divisor that ak_lmhead_ce_bwd takes. */
+int ak_lmhead_ce_fwd_denom(const void* hidden, const void* weight, const int64_t* targets,
+                           float* loss, float* lse, float* losses, int64_t* n_valid, float* denom,
+                           void* workspace, size_t workspace_bytes,
+                           int64_t n_rows, int64_t vocab, int64_t d,
+                           int64_t ld_h, int64_t ld_w, int64_t ignore_index,
+                           float softcap, float label_smoothing, int dtype, void* stream);
 
 /*
  * Fused lm-head + cross-entropy backward, first half: the gradient of the

@@ -395,6 +395,31 @@ def test_lmhead_ce_grad_logits_vocab_edges(n, vocab):
     assert bool((dz[:, vocab:].float() == 5.0).all()) and float(buf[0]) == 5.0
 
 
+@pytest.mark.parametrize("n,counted", [(1, 1), (5, 0), (1025, 1), (1025, 1024)])
+def test_lmhead_ce_denominator_of_the_backward(n, counted):
+    """Gradients of the mean loss around one thread's and one workgroup's share
+    of the counted rows, none of them counted too (divisor 1, all zeros)."""
+    need_gpu()
+    from kernels.hip.chunked_linear_cross_entropy import ChunkedLinearCrossEntropyLoss
+    g = torch.Generator().manual_seed(n + counted)
+    h, W = torch.randn(n, 64, generator=g).bfloat16(), (0.05 * torch.randn(256, 64, generator=g)).bfloat16()
+    t = torch.full((n,), -100)
+    t[n - counted:] = torch.randint(0, 256, (counted,), generator=g)
+    say("lmhead denominator", n, counted)
+    hd, wd = h.to(DEV).requires_grad_(), W.to(DEV).requires_grad_()
+    loss = ChunkedLinearCrossEntropyLoss()(hd, wd, t.to(DEV))
+    gh, gw = torch.autograd.grad(loss, (hd, wd))
+    h64, w64 = h.double().requires_grad_(), W.double().requires_grad_()
+    ref = torch.nn.functional.cross_entropy(h64 @ w64.t(), t, ignore_index=-100, reduction="sum") / max(1, counted)
+    rh, rw = torch.autograd.grad(ref, (h64, w64))
+    # dlogits and the result round to bf16 (2^-8 each); a sum of K products of
+    # rounded dlogits is within 2^-8 of the sum of their magnitudes
+    p = torch.softmax(h64 @ w64.t(), -1).detach()
+    dz = (p - torch.nn.functional.one_hot(t.clamp(min=0), 256)) * (t != -100).double()[:, None] / max(1, counted)
+    for got, r, mag in ((gh, rh, dz.abs() @ W.double().abs()), (gw, rw, dz.abs().t() @ h.double().abs())):
+        assert bool(((got.double().cpu() - r).abs() <= 2.0 ** -8 * (r.abs() + 1.01 * mag) + 1e-9).all())
+
+
 def test_lmhead_ce_grad_bad_target_rows_are_nan():
     need_gpu()
     from kernels.hip import _lib
