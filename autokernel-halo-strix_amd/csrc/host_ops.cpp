@@ -94,6 +94,10 @@ float* f32p(const Tensor& t) { return static_cast<float*>(ptr(t)); }
 Tensor f32_like(const Tensor& t, at::IntArrayRef size) { return at::empty(size, t.options().dtype(at::kFloat)); }
 Tensor bytes_like(const Tensor& t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
 
+// A saved tensor as a kernel takes it: saved-tensor hooks may hand back another
+// layout or type.
+Tensor saved_as(const Tensor& t, at::ScalarType type) { return t.defined() ? t.to(type).contiguous() : t; }
+
 // t as rows of cols elements the row kernels take (last dimension contiguous,
 // rows that do not overlap), copied only if it is not; ld gets the row pitch.
 Tensor rows_of(const Tensor& t, int64_t cols, int64_t& ld) {
@@ -205,7 +209,8 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
       variable_list r = by_formula("rmsnorm", {s[0], s[1], g[0]}, eps);
       return {r[0], r[1], Tensor()};
     }
-    auto [gx, gw] = norm_backward(s[0], s[1], Tensor(), g[0], eps);
+    const Tensor x = s[0].contiguous(), w = saved_as(s[1], x.scalar_type());
+    auto [gx, gw] = norm_backward(x, w, Tensor(), g[0], eps);
     return {gx, gw, Tensor()};
   }
 };
@@ -231,7 +236,8 @@ struct AddRmsNorm : torch::autograd::Function<AddRmsNorm> {
       variable_list r = by_formula("fused_res_rmsnorm", {s[0], s[1], g[0], g[1]}, eps);
       return {r[0], r[1], r[2], Tensor()};
     }
-    auto [gx, gw] = norm_backward(s[0], s[1], g[0], g[1], eps);
+    const Tensor h = s[0].contiguous(), w = saved_as(s[1], h.scalar_type());
+    auto [gx, gw] = norm_backward(h, w, g[0], g[1], eps);
     return {gx, gx, gw, Tensor()};
   }
 };
@@ -326,7 +332,7 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
       }
       out[0] = grad;
     } else {
-      Tensor x = saved[0].contiguous(), t = saved[1].contiguous(), rest = saved[2].contiguous();
+      Tensor x = saved[0].contiguous(), t = saved_as(saved[1], at::kLong), rest = saved_as(saved[2], at::kFloat);
       const int64_t n = x.size(0), v = x.size(1);
       float* denom = f32p(rest);
       float* mx = denom + 2 + n;
@@ -375,8 +381,8 @@ struct DiagScan : torch::autograd::Function<DiagScan> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto s = ctx->get_saved_variables();
     if (!hip_backward) return by_formula("selective_scan", {s[0], s[1], s[2], s[3], s[4], g[0]}, 0.0);
-    variable_list in;  // saved-tensor hooks may hand back another layout
-    for (const Tensor& t : s) in.push_back(t.contiguous());
+    variable_list in;
+    for (const Tensor& t : s) in.push_back(saved_as(t, at::kFloat));
     Tensor gy = g[0].to(at::kFloat).contiguous();
     variable_list out;
     for (const Tensor& t : in) out.push_back(at::empty(t.sizes(), t.options()));
@@ -472,11 +478,12 @@ struct SelectiveScan : torch::autograd::Function<SelectiveScan> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
     const bool softplus = ctx->saved_data["softplus"].toBool();
-    // saved-tensor hooks may hand back another layout
+    // the kernels take rows at any pitch; saved-tensor hooks may hand back another layout or type
     const auto rows = [](const Tensor& t) { return !t.defined() || last_dense(t) ? t : t.contiguous(); };
-    const Tensor u = rows(s[0]), delta = rows(s[1]), A = rows(s[2]), B = rows(s[3]), C = rows(s[4]), z = rows(s[6]);
-    const auto dense = [](const Tensor& t) { return t.defined() ? t.contiguous() : t; };
-    const Tensor D = dense(s[5]), bias = dense(s[7]), ckpt = dense(s[8]), prez = dense(s[9]);
+    const Tensor u = rows(s[0]), delta = rows(s[1]), B = rows(s[3]), C = rows(s[4].to(B.scalar_type()));
+    const Tensor A = rows(s[2].to(at::kFloat)), z = s[6].defined() ? rows(s[6].to(u.scalar_type())) : s[6];
+    const Tensor D = saved_as(s[5], at::kFloat), bias = saved_as(s[7], at::kFloat), ckpt = saved_as(s[8], at::kFloat);
+    const Tensor prez = saved_as(s[9], u.scalar_type());
     Tensor dout = rows(grads[0].to(u.scalar_type()));
     const ScanDims k{u.size(0), u.size(1), u.size(2), A.size(1), B.dim() == 4 ? B.size(1) : 1};
     Tensor du = at::empty(u.sizes(), u.options()), ddelta = at::empty(u.sizes(), delta.options());
@@ -549,8 +556,8 @@ struct LmHead : torch::autograd::Function<LmHead> {
     const int64_t ignore = ctx->saved_data["ignore"].toInt();
     const auto p = ctx->saved_data["p"].toDoubleVector();
     const bool need_h = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
-    const Tensor h = s[0].contiguous(), w = s[1].contiguous(), t = s[2].contiguous(), lse = s[3].contiguous();
-    const Tensor denom = s[4].contiguous();  // max(1, #counted rows)
+    const Tensor h = s[0].contiguous(), w = saved_as(s[1], h.scalar_type()), t = saved_as(s[2], at::kLong);
+    const Tensor lse = saved_as(s[3], at::kFloat), denom = saved_as(s[4], at::kFloat);  // denom: max(1, #counted rows)
     const Tensor up = g[0].detach().to(at::kFloat).contiguous();
     const int64_t n = h.size(0), d = h.size(1), v = w.size(0);
     const int code = code_of(h.scalar_type());

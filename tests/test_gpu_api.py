@@ -141,3 +141,57 @@ def test_optimize_training_step_bf16():
     loss.backward()
     for name, p in model.named_parameters():
         assert p.grad is not None and torch.isfinite(p.grad).all() and p.grad.abs().sum() > 0, name
+
+
+@pytest.mark.parametrize("form", ["layout", "type"])
+@pytest.mark.parametrize("op", ["rmsnorm", "add_rmsnorm", "diag", "scan", "ce_tiny", "lmhead"])
+def test_backward_of_repacked_saved_tensors(op, form):
+    """Saved-tensor hooks that hand back another layout (columns first) or a
+    wider type (which every value survives): the gradients are those without
+    hooks, as the values that the backward reads are."""
+    need_gpu()
+    import kernels.hip._torch_ops  # noqa: F401
+    from kernels.ce_fused import ce_full
+    from kernels.hip.chunked_linear_cross_entropy import ChunkedLinearCrossEntropyLoss
+    from kernels.hip.selective_scan import selective_scan_fn
+    g = torch.Generator().manual_seed(5)
+
+    def r(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, generator=g).to(dtype).to(DEV).requires_grad_()
+
+    f32 = torch.float32
+    t = torch.randint(0, 96, (40,), generator=g).to(DEV)
+    if op == "rmsnorm":
+        args, fn = (r(40, 96), r(96)), torch.ops.autokernel.rmsnorm
+    elif op == "add_rmsnorm":
+        args, fn = (r(40, 96), r(40, 96), r(96)), lambda *a: torch.ops.autokernel.fused_res_rmsnorm(*a)[1]
+    elif op == "diag":
+        args = tuple(r(2, 40, 32, dtype=f32) for _ in range(3)) + (r(32, dtype=f32), r(2, 40, 32, dtype=f32))
+        fn = torch.ops.autokernel.selective_scan
+    elif op == "scan":
+        args = (r(2, 32, 40), r(2, 32, 40), r(32, 16, dtype=f32), r(2, 16, 40), r(2, 16, 40), r(32, dtype=f32),
+                r(2, 32, 40), r(32, dtype=f32))
+
+        def fn(u, delta, A, *rest):
+            return selective_scan_fn(u, delta, -A.abs(), *rest, True)
+    elif op == "ce_tiny":
+        args, fn = (r(40, 96),), lambda x: ce_full(x, t, mode="tiny")
+    else:
+        args, fn = (r(40, 64), r(96, 64)), lambda h, w: ChunkedLinearCrossEntropyLoss()(h, w, t)
+
+    def pack(v):
+        if form == "layout":
+            return v.transpose(0, 1).contiguous().transpose(0, 1) if v.dim() > 1 else v.clone()
+        return v.to(f32) if v.is_floating_point() and v.dim() == 1 else v.to(torch.int32) if v.dtype == torch.long else v
+
+    def grads(out):
+        up = torch.ones_like(out)
+        return torch.autograd.grad(out, args, up)
+
+    say("repacked saved tensors", op, form)
+    want = grads(fn(*args))
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda v: v):
+        out = fn(*args)
+    got = grads(out)
+    for a, w, v in zip(args, want, got):
+        assert v.dtype == a.dtype and torch.equal(w, v)
