@@ -54,8 +54,13 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
   const int n = lane % 16;
   const int tpg = p.tiles_per_group;  // whole kCh-channel tiles
   const int per_batch = p.ngroups * tpg;
-  const ScanSeg sg(p, blockIdx.x / per_batch);
-  const int b = sg.b;
+  // Only the four-wave form takes a sequence in segments (the launcher's rule);
+  // with the segments' bounds read at run time the eight-wave form took 450
+  // instead of 440 us ([4, 2048, 4096] with dz).
+  constexpr bool kSeg = kWv == 4;
+  const int bs = blockIdx.x / per_batch;  // batch and segment
+  const ScanSeg sg(p, bs);
+  const int b = kSeg ? sg.b : bs;
   const int g = (blockIdx.x % per_batch) / tpg;
   const int tile = blockIdx.x % tpg;
   const int d0 = g * p.ch_per_group + tile * kCh;
@@ -136,9 +141,10 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
 
   // the adjoint of the segments behind this one, as the product of a step's
   // state gradient and the decay that follows it
-  float gs = n_ok ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f, a_next = 1.0f;
+  float gs = 0.0f, a_next = kSeg ? 1.0f : 0.0f;
+  if constexpr (kSeg) gs = n_ok ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f;
   float dA_acc = 0.0f, dD_acc = 0.0f, dbias_acc = 0.0f;
-  const int t_lo = sg.first, nt = sg.end;  // tiles nt - 1 down to t_lo
+  const int t_lo = kSeg ? sg.first : 0, nt = kSeg ? sg.end : p.seqlen / kScanT;  // tiles nt - 1 down to t_lo
   Raw4<TBC> bv{}, cv{};
   if (stager) {
     bv = bload4<TBC>(rs_B, vo_B, (uint32_t)(nt - 1) * kScanT * sizeof(TBC));
@@ -329,7 +335,7 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
       }
     }
   }
-  const int64_t bd_row = (int64_t)(blockIdx.x / per_batch) * p.dim + d;  // partials per batch and segment
+  const int64_t bd_row = (int64_t)bs * p.dim + d;  // partials per batch and segment
   if (n_ok) p.dA_part[bd_row * p.dstate + n] = dA_acc;
   dD_acc = row16_sum(dD_acc);
   dbias_acc = row16_sum(dbias_acc);
