@@ -195,7 +195,11 @@ struct ScanSeg {
 };
 
 // The state that enters the segment: the segments before it (kBwd: the adjoint
-// that enters it from those behind it), folded in order.
+// that enters it from those behind it), folded in order. A segment's decay may
+// leave fp32's range although what it carries does not (a growing recurrence:
+// A > 0, or a negative delta'), and an infinite state meets only decays above
+// zero step by step: past 2^126 the decay's whole powers of two go to the state's
+// exponent, so that the product alone over- or underflows.
 template <bool kBwd>
 __device__ __forceinline__ float seg_enter(const ScanParams& p, const ScanSeg& sg, int d, int n, float a_scaled) {
   float h = 0.0f;
@@ -203,9 +207,9 @@ __device__ __forceinline__ float seg_enter(const ScanParams& p, const ScanSeg& s
 #pragma unroll 4
   for (int i = 0; i < count; ++i) {
     const int64_t at = ((int64_t)sg.b * p.segs + (kBwd ? p.segs - 1 - i : i)) * p.dim + d;
-    // (a zero state stays out of the product: a growing decay, A > 0, may overflow)
-    const float in = p.seg_state[at * p.dstate + n], decay = __builtin_amdgcn_exp2f(a_scaled * p.seg_dsum[at]);
-    h = h == 0.0f ? in : fmaf(decay, h, in);
+    const float t = fminf(fmaxf(a_scaled * p.seg_dsum[at], -1000.0f), 1000.0f);  // 2^1000 takes any fp32 to its end
+    const float k = fabsf(t) < 126.0f ? 0.0f : truncf(t);
+    h = fmaf(__builtin_amdgcn_exp2f(t - k), ldexpf(h, (int)k), p.seg_state[at * p.dstate + n]);
   }
   return h;
 }

@@ -439,3 +439,48 @@ def test_segments_and_ragged_lengths(itype, batch, dim, seqlen, groups, opts):
         r, a = tols[name]
         tols[name] = (r, a * max(1.0, batch * seqlen / 512) ** 0.5)
     _check(got, bref, tols, (u, delta, A, B, C, D, z, bias))
+
+
+def test_segments_of_a_growing_recurrence():
+    """A decay that grows (A > 0 with a positive delta, or a negative delta) and
+    passes fp32's range over one segment of four, while the states and adjoints
+    that it carries do not: a sum of A delta of 96 is a factor of 5e41 on inputs
+    and upstream gradients of 1e-10. Per step the exponent is off by 2^-23 of
+    itself at most and the exponential by 2 units, so 64 steps by about 3e-5."""
+    need_gpu()
+    from kernels.hip.selective_scan import selective_scan_fn
+    u, delta = torch.zeros(1, 16, 256), torch.zeros(1, 16, 256)
+    A = torch.ones(16, 16) * torch.linspace(0.25, 1.0, 16)
+    A[8:] *= -1  # these channels grow by a negative delta
+    u[..., :64] = 1e-10
+    delta[..., :64], delta[..., 64:128], delta[..., 128:] = 0.01, 1.5, 0.001
+    delta[:, 8:] *= -1
+    u[:, 8:] *= -1  # delta u and all that it feeds stay positive: no sum over channels cancels, so the bound is relative
+    B, C = torch.ones(1, 1, 16, 256), torch.ones(1, 1, 16, 256)
+    dout = torch.zeros(1, 16, 256)
+    dout[..., 192:] = 1e-10
+    say("scan segments, growing")
+    args = [t.to(DEV) for t in (u, delta, A, B, C)]
+    out, last = selective_scan_fn(*args, return_last_state=True)
+    rout, rlast = ops.selective_scan_ref(u, delta, A, B, C, return_last_state=True, compute_dtype=torch.float64)
+    assert bool(((out.double().cpu() - rout).abs() <= 1e-4 * rout.abs()).all())
+    assert bool(((last.double().cpu() - rlast).abs() <= 1e-4 * rlast.abs()).all())
+    got = _gpu_grads(u, delta, A, B, C, None, None, None, dout, False)
+    ref = ops.selective_scan_bwd_ref(u, delta, A, B, C, dout)
+    for name, g, r in zip(NAMES, got, ref):
+        if g is not None:
+            assert bool(((g.double() - r).abs() <= 2e-4 * r.abs().amax()).all()), name
+
+
+def test_segments_keep_an_infinite_state():
+    """A state that has overflowed stays infinite through a segment whose decay
+    underflows as one number but not step by step, as in the uncut recurrence."""
+    need_gpu()
+    from kernels.hip.selective_scan import selective_scan_fn
+    u, delta = torch.zeros(1, 16, 256, device=DEV), torch.full((1, 16, 256), 2.0, device=DEV)
+    u[..., 3] = 3e38
+    A = -torch.ones(16, 16, device=DEV)
+    B, C = torch.full((1, 16, 256), 4.0, device=DEV), torch.ones(1, 16, 256, device=DEV)
+    say("scan segments, infinite state")
+    _, last = selective_scan_fn(u, delta, A, B, C, return_last_state=True)
+    assert bool((last == float("inf")).all())
