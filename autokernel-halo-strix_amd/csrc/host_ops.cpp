@@ -227,9 +227,8 @@ struct AddRmsNorm : torch::autograd::Function<AddRmsNorm> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto s = ctx->get_saved_variables();
     const double eps = ctx->saved_data["eps"].toDouble();
-    if (!g[1].defined()) {  // only the sum was used
-      if (!g[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
-      Tensor gx = g[0].to(s[0].scalar_type());
+    if (!g[1].defined()) {  // only the sum was used, or neither output's gradient came
+      Tensor gx = g[0].defined() ? g[0].to(s[0].scalar_type()) : at::zeros_like(s[0]);
       return {gx, gx, at::zeros_like(s[1]), Tensor()};
     }
     if (!hip_backward) {

@@ -92,7 +92,6 @@ def _register_native(op, entry: str, defaults: tuple, setup, backward) -> None:
             with torch._C._AutoDispatchBelowAutograd():
                 out = op._opoverload(*args)
             setup(ctx, args, out)
-            ctx.set_materialize_grads(False)
             return out
 
         @staticmethod

@@ -195,3 +195,45 @@ def test_backward_of_repacked_saved_tensors(op, form):
     got = grads(out)
     for a, w, v in zip(args, want, got):
         assert v.dtype == a.dtype and torch.equal(w, v)
+
+
+class _NoGradient(torch.autograd.Function):
+    """Takes any tensors and hands back no gradient for them."""
+
+    @staticmethod
+    def forward(ctx, *xs):
+        ctx.n = len(xs)
+        return sum(x.float().sum() for x in xs)
+
+    @staticmethod
+    def backward(ctx, g):
+        return (None,) * ctx.n
+
+
+@pytest.mark.parametrize("form", ["plain", "transposed", "mixed"])
+@pytest.mark.parametrize("op", ["rmsnorm", "add_rmsnorm", "diag"])
+def test_ops_whose_consumer_gives_no_gradient(op, form):
+    """Every input's gradient is zeros then, by each route: plain calls, and
+    transposed and mixed-type ones, which the native host side leaves alone."""
+    need_gpu()
+    import kernels.hip._torch_ops  # noqa: F401
+    k = torch.ops.autokernel
+    wt = torch.float32 if form == "mixed" else torch.bfloat16
+    if op == "diag":
+        shapes, dts = [(2, 8, 16)] * 3 + [(16,), (2, 8, 16)], [torch.float32] * 5
+        dts[3] = torch.bfloat16 if form == "mixed" else torch.float32
+        fn = k.selective_scan
+    elif op == "rmsnorm":
+        shapes, dts, fn = [(40, 96), (96,)], [torch.bfloat16, wt], k.rmsnorm
+    else:
+        shapes, dts, fn = [(40, 96)] * 2 + [(96,)], [torch.bfloat16] * 2 + [wt], k.fused_res_rmsnorm
+    leaves = [torch.randn(*s, device=DEV).to(dt) for s, dt in zip(shapes, dts)]
+    if form == "transposed":
+        leaves[0] = leaves[0].transpose(-1, -2).contiguous()
+    leaves = [v.requires_grad_() for v in leaves]
+    args = [leaves[0].transpose(-1, -2) if form == "transposed" else leaves[0]] + leaves[1:]
+    say("no gradient from the consumer", op, form)
+    out = fn(*args)
+    loss = _NoGradient.apply(*(out if isinstance(out, (tuple, list)) else (out,)))
+    for leaf, g in zip(leaves, torch.autograd.grad(loss, leaves)):
+        assert g.shape == leaf.shape and g.dtype == leaf.dtype and not g.any()
