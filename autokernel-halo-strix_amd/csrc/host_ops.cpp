@@ -530,9 +530,9 @@ std::optional<std::vector<Tensor>> selective_scan(const Tensor& u, const Tensor&
 // ---------------------------------------------------------------------------
 // lm-head + cross-entropy
 // ---------------------------------------------------------------------------
-bool dense16(const Tensor& t) {
-  return t.dim() == 2 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
-}
+bool at16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+bool dense16(const Tensor& t) { return t.dim() == 2 && t.is_contiguous() && at16(t); }
+Tensor realigned(const Tensor& t) { return at16(t) ? t : t.clone(); }
 
 struct LmHead : torch::autograd::Function<LmHead> {
   static Tensor forward(AutogradContext* ctx, const Tensor& h, const Tensor& w, const Tensor& t, int64_t ignore, double cap,
@@ -555,7 +555,9 @@ struct LmHead : torch::autograd::Function<LmHead> {
     const int64_t ignore = ctx->saved_data["ignore"].toInt();
     const auto p = ctx->saved_data["p"].toDoubleVector();
     const bool need_h = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
-    const Tensor h = s[0].contiguous(), w = saved_as(s[1], h.scalar_type()), t = saved_as(s[2], at::kLong);
+    // (saved-tensor hooks may hand back any address too, where the tile kernels need 16-byte rows)
+    const Tensor h = realigned(s[0].contiguous()), w = realigned(saved_as(s[1], h.scalar_type()));
+    const Tensor t = saved_as(s[2], at::kLong);
     const Tensor lse = saved_as(s[3], at::kFloat), denom = saved_as(s[4], at::kFloat);  // denom: max(1, #counted rows)
     const Tensor up = g[0].detach().to(at::kFloat).contiguous();
     const int64_t n = h.size(0), d = h.size(1), v = w.size(0);

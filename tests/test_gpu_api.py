@@ -143,12 +143,12 @@ def test_optimize_training_step_bf16():
         assert p.grad is not None and torch.isfinite(p.grad).all() and p.grad.abs().sum() > 0, name
 
 
-@pytest.mark.parametrize("form", ["layout", "type"])
+@pytest.mark.parametrize("form", ["layout", "type", "address"])
 @pytest.mark.parametrize("op", ["rmsnorm", "add_rmsnorm", "diag", "scan", "ce_tiny", "lmhead"])
 def test_backward_of_repacked_saved_tensors(op, form):
-    """Saved-tensor hooks that hand back another layout (columns first) or a
-    wider type (which every value survives): the gradients are those without
-    hooks, as the values that the backward reads are."""
+    """Saved-tensor hooks that hand back another layout (columns first), a
+    wider type (which every value survives) or an odd address: the gradients are
+    those without hooks, as the values that the backward reads are."""
     need_gpu()
     import kernels.hip._torch_ops  # noqa: F401
     from kernels.ce_fused import ce_full
@@ -182,6 +182,8 @@ def test_backward_of_repacked_saved_tensors(op, form):
     def pack(v):
         if form == "layout":
             return v.transpose(0, 1).contiguous().transpose(0, 1) if v.dim() > 1 else v.clone()
+        if form == "address":
+            return torch.cat((v.new_zeros(1), v.reshape(-1)))[1:].view(v.shape)
         return v.to(f32) if v.is_floating_point() and v.dim() == 1 else v.to(torch.int32) if v.dtype == torch.long else v
 
     def grads(out):
