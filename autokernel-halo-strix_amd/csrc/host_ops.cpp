@@ -505,7 +505,7 @@ struct SelectiveScan : torch::autograd::Function<SelectiveScan> {
   }
 };
 
-// (out, last state or nothing). save: training keeps its states; max_bytes: up to this size (below 0: any).
+// (out, last state or nothing). save: training keeps its states; max_bytes: up to this size.
 std::optional<std::vector<Tensor>> selective_scan(const Tensor& u, const Tensor& delta, const Tensor& A, const Tensor& B,
                                                   const Tensor& C, const Maybe& D, const Maybe& z, const Maybe& bias,
                                                   bool softplus, bool want_last, bool save, double max_bytes) {
@@ -517,7 +517,7 @@ std::optional<std::vector<Tensor>> selective_scan(const Tensor& u, const Tensor&
   if (records({&u, &delta, &A, &B, &C, &d, &zz, &bb})) {
     const double bytes = 4.0 * k.b * k.d * k.n * ((k.l + kStep - 1) / kStep);
     return SelectiveScan::apply(u, delta, A, B, C, D, z, bias, softplus, want_last,
-                                save && (max_bytes < 0 || bytes <= max_bytes));
+                                save && bytes <= max_bytes);
   }
   Tensor out = at::empty(u.sizes(), u.options()), last;
   if (want_last) last = f32_like(u, {k.b, k.d, k.n});
@@ -590,12 +590,12 @@ struct LmHead : torch::autograd::Function<LmHead> {
 };
 
 // budget: the bytes of dlogits that the backward may hold at once.
-Maybe lmhead_ce(const Tensor& h, const Tensor& w, const Tensor& t, int64_t ignore, double cap, double smoothing, int64_t budget) {
+Maybe lmhead_ce(const Tensor& h, const Tensor& w, const Tensor& t, int64_t ignore, double cap, double smoothing, double budget) {
   if (!ours(h, w, t) || !dense16(h) || !dense16(w) || h.scalar_type() != w.scalar_type() || h.size(0) == 0 || w.size(0) == 0 ||
       (h.scalar_type() != at::kHalf && h.scalar_type() != at::kBFloat16) || h.size(1) != w.size(1) || h.size(1) == 0 ||
       h.size(1) % 64 || t.scalar_type() != at::kLong || t.dim() != 1 || !t.is_contiguous() || t.size(0) != h.size(0))
     return std::nullopt;
-  if (records({&h, &w}) && h.size(0) * 2 * ((w.size(0) + 255) / 256 * 256) > budget) return std::nullopt;  // vocab ranges
+  if (records({&h, &w}) && 2.0 * h.size(0) * ((w.size(0) + 255) / 256 * 256) > budget) return std::nullopt;  // vocab ranges
   return LmHead::apply(h, w, t, ignore, cap, smoothing);
 }
 

@@ -143,8 +143,8 @@ def _native(logits, targets, softcap, ignore_index, label_smoothing, fused, z_lo
     host = _lib.native(logits, targets)
     if host is None:
         return None
-    return host.ce_full(logits, targets, softcap, _NO_IGNORE if ignore_index is None else ignore_index,
-                        label_smoothing, fused, z_loss_weight, _top_hooks(False) is None)
+    return host.ce_full(logits, targets, float(softcap), _NO_IGNORE if ignore_index is None else int(ignore_index),
+                        float(label_smoothing), fused, z_loss_weight, _top_hooks(False) is None)
 
 
 class _CrossEntropyHIP(torch.autograd.Function):

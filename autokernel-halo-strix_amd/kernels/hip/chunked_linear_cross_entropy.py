@@ -357,7 +357,7 @@ class ChunkedLinearCrossEntropyLoss(nn.Module):
             host = _lib.native(hidden, weight, targets)
             if host is not None:
                 loss = host.lmhead_ce(hidden, weight, targets, self.ignore_index, self.softcap,
-                                      self.label_smoothing, GRAD_LOGITS_BUDGET)
+                                      self.label_smoothing, float(GRAD_LOGITS_BUDGET))
                 if loss is not None:
                     return loss
         return _ChunkedLinearCrossEntropy.apply(

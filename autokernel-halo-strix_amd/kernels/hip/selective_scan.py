@@ -52,6 +52,7 @@ Two entry points, both drop-ins:
   recomputes instead.
 """
 
+import math
 import os
 
 import torch
@@ -313,7 +314,7 @@ def selective_scan_fn(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta_
     if host is not None:
         res = host.selective_scan(u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus),
                                   bool(return_last_state), SAVE_STATES,
-                                  -1.0 if SAVE_STATES_MAX_BYTES is None else SAVE_STATES_MAX_BYTES)
+                                  math.inf if SAVE_STATES_MAX_BYTES is None else float(SAVE_STATES_MAX_BYTES))
         if res is not None:
             return tuple(res) if return_last_state else res[0]
     return SelectiveScanFn.apply(u, delta, A, B, C, D, z, delta_bias, delta_softplus,

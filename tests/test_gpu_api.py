@@ -239,3 +239,44 @@ def test_ops_whose_consumer_gives_no_gradient(op, form):
     loss = _NoGradient.apply(*(out if isinstance(out, (tuple, list)) else (out,)))
     for leaf, g in zip(leaves, torch.autograd.grad(loss, leaves)):
         assert g.shape == leaf.shape and g.dtype == leaf.dtype and not g.any()
+
+
+def test_arguments_that_are_converted():
+    """Numbers of another kind than the kernels' arguments, and limits beyond
+    64 bits, are taken as the Python conversions take them."""
+    need_gpu()
+    from kernels.ce_fused import ce_full
+    from kernels.hip import chunked_linear_cross_entropy as clc, selective_scan as ss
+    g = torch.Generator().manual_seed(9)
+    x, t = torch.randn(40, 96, generator=g).bfloat16().to(DEV), torch.randint(0, 96, (40,), generator=g).to(DEV)
+    t[3] = -100
+    say("converted arguments")
+    want = ce_full(x, t, softcap=3.0, label_smoothing=0.5)
+    assert torch.equal(ce_full(x, t, softcap="3", label_smoothing="0.5", ignore_index=-100.0), want)
+    with pytest.raises(TypeError):
+        ce_full(x, t, softcap=None)
+
+    def lmhead():
+        h, w = (torch.ones(40, 64, device=DEV, dtype=torch.bfloat16).requires_grad_() for _ in range(2))
+        return torch.autograd.grad(clc.ChunkedLinearCrossEntropyLoss()(h, w, t % 40), (h, w))
+
+    want = lmhead()
+    for budget in (4e9, float("inf"), 1 << 70):
+        with pytest.MonkeyPatch.context() as m:
+            m.setattr(clc, "GRAD_LOGITS_BUDGET", budget)
+            for a, b in zip(lmhead(), want):
+                assert torch.equal(a, b)
+
+    def kept(limit):  # bytes that a recorded scan holds beside its output
+        ss.set_save_states(True, limit)
+        try:
+            u = torch.zeros(1, 64, 1024, device=DEV).requires_grad_()
+            A, B = -torch.ones(64, 16, device=DEV), torch.zeros(1, 16, 1024, device=DEV)
+            before = torch.cuda.memory_allocated()
+            out = ss.selective_scan_fn(u, u, A, B, B)
+            return torch.cuda.memory_allocated() - before - out.numel() * out.element_size()
+        finally:
+            ss.set_save_states(True, None)
+
+    assert kept(-1) == kept(0) == 0
+    assert kept(None) == kept(1 << 70) == kept(4 * 64 * 64 * 16) > 0 == kept(4 * 64 * 64 * 16 - 1)
