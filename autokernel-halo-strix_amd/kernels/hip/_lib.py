@@ -159,12 +159,16 @@ def host():
     return _host
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def native(*tensors):
     """:func:`host` where a call on these tensors may be its, else None: GPU
-    tensors, and not while torch.compile traces the call (the Python forms below
-    it are the traced ones)."""
+    tensors of torch's own classes (a subclass may take part in each torch call),
+    and not while torch.compile traces the call (the Python forms below it are
+    the traced ones)."""
     for t in tensors:
-        if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        if type(t) not in _PLAIN or not t.is_cuda:
             return None
     return None if _is_compiling() else (_host or host())
 

@@ -45,7 +45,7 @@ def kernel_fn(x: torch.Tensor, weight: torch.Tensor, eps: float = DEFAULT_EPS) -
     weight = weight.contiguous()
     shape = x.shape
     x2 = _lib.as_rows(x, shape[-1])
-    y = torch.empty(shape, dtype=x.dtype, device=x.device)
+    y = torch.empty_like(x, memory_format=torch.contiguous_format)
     if y.numel():
         _lib.rmsnorm(x2, weight, y.view(-1, shape[-1]), eps)
     return y

@@ -280,3 +280,25 @@ def test_arguments_that_are_converted():
 
     assert kept(-1) == kept(0) == 0
     assert kept(None) == kept(1 << 70) == kept(4 * 64 * 64 * 16) > 0 == kept(4 * 64 * 64 * 16 - 1)
+
+
+def test_tensor_subclasses_keep_their_route():
+    """A tensor subclass (no dispatch of its own) comes back as one where the
+    result is made like the input, as torch makes it."""
+    need_gpu()
+    from kernels.hip.rmsnorm import kernel_fn as rmsnorm
+    from kernels.hip.selective_scan import kernel_fn as diag
+
+    class Tagged(torch.Tensor):
+        pass
+
+    x, w = torch.randn(8, 64, device=DEV), torch.randn(64, device=DEV)
+    v = [torch.rand(2, 8, 16, device=DEV) for _ in range(4)]
+    D = torch.rand(16, device=DEV)
+    say("tensor subclasses")
+    y = rmsnorm(x.as_subclass(Tagged), w)
+    s = diag(v[0].as_subclass(Tagged), v[1], v[2], D, v[3])
+    assert type(y) is Tagged and type(s) is Tagged
+    assert torch.equal(y.as_subclass(torch.Tensor), rmsnorm(x, w))
+    assert torch.equal(s.as_subclass(torch.Tensor), diag(*v[:3], D, v[3]))
+    assert type(rmsnorm(x, torch.nn.Parameter(w))) is torch.Tensor
