@@ -43,9 +43,8 @@ def kernel_fn(x: torch.Tensor, weight: torch.Tensor, eps: float = DEFAULT_EPS) -
     if weight.dtype != x.dtype:
         weight = weight.to(x.dtype)
     weight = weight.contiguous()
-    shape = x.shape
-    x2 = _lib.as_rows(x, shape[-1])
     y = torch.empty_like(x, memory_format=torch.contiguous_format)
     if y.numel():
-        _lib.rmsnorm(x2, weight, y.view(-1, shape[-1]), eps)
+        cols = x.shape[-1]
+        _lib.rmsnorm(_lib.as_rows(x, cols), weight, y.view(-1, cols), eps)
     return y

@@ -302,3 +302,10 @@ def test_tensor_subclasses_keep_their_route():
     assert torch.equal(y.as_subclass(torch.Tensor), rmsnorm(x, w))
     assert torch.equal(s.as_subclass(torch.Tensor), diag(*v[:3], D, v[3]))
     assert type(rmsnorm(x, torch.nn.Parameter(w))) is torch.Tensor
+
+
+def test_rows_of_no_columns():
+    need_gpu()
+    from kernels.hip.rmsnorm import kernel_fn as rmsnorm
+    say("rows of no columns")
+    assert rmsnorm(torch.empty(4, 0, device=DEV), torch.empty(0, device=DEV)).shape == (4, 0)
