@@ -283,9 +283,11 @@ bool last_backward(const Tensor& t) {
 }
 
 struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
-  // need: a gradient will be asked for; own: nobody but the graph holds what it saves
-  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& t, double softcap, int64_t ignore,
-                               double smoothing, bool fused, double zw, bool need, bool own) {
+  // need: a gradient will be asked for; own: nobody but the graph holds what it
+  // saves. lse_out: the row statistics, which have no gradient and are no output
+  // of the node (compiled autograd takes no C++ node with one that is marked so).
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& t, double softcap, int64_t ignore,
+                        double smoothing, bool fused, double zw, bool need, bool own, Tensor* lse_out) {
     const int64_t n = x.size(0), v = x.size(1);
     const int code = code_of(x.scalar_type());
     void* s = stream_of(x);
@@ -302,21 +304,21 @@ struct CrossEntropy : torch::autograd::Function<CrossEntropy> {
     check(api.ak_ce_fwd(x.data_ptr(), i64p(t), losses, f32p(lse), mx, sm, ptr(grad), n, v, v, v, (float)softcap, ignore,
                         (float)smoothing, 1.0f, (float)zw, grad.defined() ? denom + 1 : nullptr, code, s), "ak_ce_fwd");
     check(api.ak_ce_mean(losses, f32p(lse), i64p(t), n, ignore, (float)zw, f32p(loss), nullptr, s), "ak_ce_mean");
-    ctx->mark_non_differentiable({lse});
+    *lse_out = lse;
     if (need) {
       if (fused) ctx->save_for_backward({grad});
       else ctx->save_for_backward({x, t, rest});
       ctx->saved_data["p"] = std::vector<double>{softcap, smoothing, zw};
       ctx->saved_data["i"] = std::vector<int64_t>{ignore, fused, own};
     }
-    return {loss, lse};
+    return loss;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto p = ctx->saved_data["p"].toDoubleVector();
     const auto i = ctx->saved_data["i"].toIntVector();
     const auto saved = ctx->get_saved_variables();
     Tensor up = g[0].detach().to(at::kFloat);
-    variable_list out(9);
+    variable_list out(10);
     if (i[1]) {
       // The saved gradient carries 1 / #counted rows already. The upstream
       // gradient scales it in place where this backward is the graph's last: 1
@@ -350,8 +352,9 @@ Pair ce_full(const Tensor& x, const Tensor& t, double softcap, int64_t ignore, d
              bool own) {
   if (!ours(x, t) || !ce_args(x, t)) return std::nullopt;
   const bool need = records({&x});
-  variable_list v = CrossEntropy::apply(x, t, softcap, ignore, smoothing, fused, zw, need, own);
-  return std::make_tuple(v[0], v[1]);
+  Tensor lse;
+  const Tensor loss = CrossEntropy::apply(x, t, softcap, ignore, smoothing, fused, zw, need, own, &lse);
+  return std::make_tuple(loss, lse);
 }
 
 // ---------------------------------------------------------------------------
@@ -456,13 +459,14 @@ void run_scan(const Tensor& u, const Tensor& delta, const Tensor& A, const Tenso
 }
 
 struct SelectiveScan : torch::autograd::Function<SelectiveScan> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& u, const Tensor& delta, const Tensor& A, const Tensor& B,
-                               const Tensor& C, const Maybe& D_, const Maybe& z_, const Maybe& bias_, bool softplus,
-                               bool want_last, bool keep) {
+  // last_out: takes the last state where it is wanted (no output of the node, as in CrossEntropy)
+  static Tensor forward(AutogradContext* ctx, const Tensor& u, const Tensor& delta, const Tensor& A, const Tensor& B,
+                        const Tensor& C, const Maybe& D_, const Maybe& z_, const Maybe& bias_, bool softplus,
+                        Tensor* last_out, bool keep) {
     const Tensor D = D_.value_or(Tensor()), z = z_.value_or(Tensor()), bias = bias_.value_or(Tensor());
     const ScanDims k{u.size(0), u.size(1), u.size(2), A.size(1), B.dim() == 4 ? B.size(1) : 1};
     Tensor out = at::empty(u.sizes(), u.options()), last, prez, ckpt;
-    if (want_last) last = f32_like(u, {k.b, k.d, k.n});
+    if (last_out) last = *last_out = f32_like(u, {k.b, k.d, k.n});
     if (keep) {
       if (z.defined()) prez = at::empty(u.sizes(), u.options());
       ckpt = f32_like(u, {k.b, (k.l + kStep - 1) / kStep, k.d, k.n});
@@ -470,9 +474,7 @@ struct SelectiveScan : torch::autograd::Function<SelectiveScan> {
     run_scan(u, delta, A, B, C, D, z, bias, softplus, k, out, last, prez, ckpt);
     ctx->save_for_backward({u, delta, A, B, C, D, z, bias, ckpt, prez});
     ctx->saved_data["softplus"] = softplus;
-    if (!want_last) return {out};
-    ctx->mark_non_differentiable({last});
-    return {out, last};
+    return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
@@ -514,14 +516,15 @@ std::optional<std::vector<Tensor>> selective_scan(const Tensor& u, const Tensor&
       !scan_args(u, delta, A, B, C, D, z, bias, k))
     return std::nullopt;
   const Tensor d = D.value_or(Tensor()), zz = z.value_or(Tensor()), bb = bias.value_or(Tensor());
+  Tensor out, last;
   if (records({&u, &delta, &A, &B, &C, &d, &zz, &bb})) {
     const double bytes = 4.0 * k.b * k.d * k.n * ((k.l + kStep - 1) / kStep);
-    return SelectiveScan::apply(u, delta, A, B, C, D, z, bias, softplus, want_last,
-                                save && bytes <= max_bytes);
+    out = SelectiveScan::apply(u, delta, A, B, C, D, z, bias, softplus, want_last ? &last : nullptr, save && bytes <= max_bytes);
+  } else {
+    out = at::empty(u.sizes(), u.options());
+    if (want_last) last = f32_like(u, {k.b, k.d, k.n});
+    run_scan(u, delta, A, B, C, d, zz, bb, softplus, k, out, last, Tensor(), Tensor());
   }
-  Tensor out = at::empty(u.sizes(), u.options()), last;
-  if (want_last) last = f32_like(u, {k.b, k.d, k.n});
-  run_scan(u, delta, A, B, C, d, zz, bb, softplus, k, out, last, Tensor(), Tensor());
   std::vector<Tensor> r{out};
   if (want_last) r.push_back(last);
   return r;

@@ -309,3 +309,46 @@ def test_rows_of_no_columns():
     from kernels.hip.rmsnorm import kernel_fn as rmsnorm
     say("rows of no columns")
     assert rmsnorm(torch.empty(4, 0, device=DEV), torch.empty(0, device=DEV)).shape == (4, 0)
+
+
+@pytest.mark.parametrize("op", ["rmsnorm", "add_rmsnorm", "diag", "scan", "scan_last", "ce", "ce_tiny", "lmhead"])
+def test_compiled_autograd(op):
+    """A backward that torch's compiled autograd records gives the eager one's bits."""
+    need_gpu()
+    import kernels.hip._torch_ops  # noqa: F401
+    import torch._dynamo.compiled_autograd as compiled
+    from kernels.ce_fused import ce_full
+    from kernels.hip.chunked_linear_cross_entropy import ChunkedLinearCrossEntropyLoss
+    from kernels.hip.selective_scan import selective_scan_fn
+    g = torch.Generator().manual_seed(6)
+    t = torch.randint(0, 96, (40,), generator=g).to(DEV)
+
+    def r(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, generator=g).to(dtype).to(DEV).requires_grad_()
+
+    f32 = torch.float32
+    if op == "rmsnorm":
+        args, fn = (r(40, 96), r(96)), torch.ops.autokernel.rmsnorm
+    elif op == "add_rmsnorm":
+        args, fn = (r(40, 96), r(40, 96), r(96)), lambda *a: torch.ops.autokernel.fused_res_rmsnorm(*a)[1]
+    elif op == "diag":
+        args = tuple(r(2, 40, 32, dtype=f32) for _ in range(3)) + (r(32, dtype=f32), r(2, 40, 32, dtype=f32))
+        fn = torch.ops.autokernel.selective_scan
+    elif op.startswith("scan"):
+        args = (r(2, 32, 40), r(2, 32, 40), r(32, 16, dtype=f32), r(2, 16, 40), r(2, 16, 40), r(32, dtype=f32),
+                r(2, 32, 40), r(32, dtype=f32))
+
+        def fn(u, delta, A, *rest):
+            y = selective_scan_fn(u, delta, -A.abs(), *rest, True, op == "scan_last")
+            return y[0] if op == "scan_last" else y
+    elif op.startswith("ce"):
+        args, fn = (r(40, 96),), lambda x: ce_full(x, t, mode="tiny" if op == "ce_tiny" else "fused")
+    else:
+        args, fn = (r(40, 64), r(96, 64)), lambda h, w: ChunkedLinearCrossEntropyLoss()(h, w, t)
+    say("compiled autograd", op)
+    want = torch.autograd.grad(fn(*args).sum(), args)
+    loss = fn(*args).sum()
+    with compiled._enable(torch.compile(backend="eager")):
+        loss.backward()
+    for a, w in zip(args, want):
+        assert torch.equal(a.grad, w)
