@@ -34,7 +34,7 @@ namespace {
 // kPrep: the preparation pass of the backward. Instead of the output it
 // writes the state before every 64-step tile to p.ck and, with a gate,
 // dz = dout * y * silu'(z) (y the output before the gate).
-template <typename TU, typename TD, typename TBC, bool kPrep = false>
+template <typename TU, typename TD, typename TBC, bool kPrep, bool kSeg>
 __global__ void __launch_bounds__(256)
 mamba_scan_fwd_kernel(ScanParams p) {
   __shared__ float Bs[16 * kBStride];
@@ -48,7 +48,7 @@ mamba_scan_fwd_kernel(ScanParams p) {
   const int n = lane % 16;  // state owned by this lane
 
   const int per_batch = p.ngroups * p.tiles_per_group;
-  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const ScanSeg<kSeg> sg(p, blockIdx.x / per_batch);
   const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
   const int tile = blockIdx.x % p.tiles_per_group;
@@ -145,7 +145,7 @@ mamba_scan_fwd_kernel(ScanParams p) {
     for (int i = 0; i < sg.seg; ++i) dsum += p.seg_dsum[((int64_t)b * p.segs + i) * p.dim + d];
   TileRegs cur, nxt{};
   load_tile(sg.first * kScanT, cur);
-  const int l_end = min(sg.end * kScanT, p.seqlen);
+  const int l_end = kSeg ? min(sg.end * kScanT, p.seqlen) : p.seqlen;
   for (int l0 = sg.first * kScanT; l0 < l_end; l0 += kScanT) {
     __syncthreads();  // previous tile's readers of Bs / Cs are done
 #pragma unroll
@@ -683,7 +683,7 @@ mamba_scan_fast_kernel(ScanParams p) {
 // [4, 1536, 300] bf16 23.8 -> 16.8.
 enum { kPrepGated = 3 };
 
-template <typename TU, typename TD, typename TBC, bool kSoftplus, int kMode, bool kRag>
+template <typename TU, typename TD, typename TBC, bool kSoftplus, int kMode, bool kRag, bool kSeg>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 mamba_scan_split_kernel(ScanParams p) {
   constexpr bool kPrep = kMode == kPrepGated;
@@ -703,7 +703,7 @@ mamba_scan_split_kernel(ScanParams p) {
   const int c = lane / 16;
   const int n = lane % 16;
   const int per_batch = p.ngroups * p.tiles_per_group;
-  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const ScanSeg<kSeg> sg(p, blockIdx.x / per_batch);
   const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
   const int tile = blockIdx.x % p.tiles_per_group;
@@ -712,7 +712,7 @@ mamba_scan_split_kernel(ScanParams p) {
   const int d = d0 + wc;
   const bool n_ok = n < p.dstate;
   const uint32_t L = (uint32_t)p.seqlen;
-  const int t0 = sg.first, nt = sg.end - sg.first;  // tiles t0 .. t0 + nt - 1; t below counts from t0
+  const int t0 = sg.first, nt = kSeg || kRag ? sg.end - sg.first : p.seqlen / kScanT;  // tiles t0 .. t0 + nt - 1; t below counts from t0
   auto row_rsrc = [&](const void* base, int64_t bs, int64_t ds, int esz) {
     const char* q = static_cast<const char*>(base) + ((int64_t)b * bs + (int64_t)d0 * ds) * esz;
     return make_rsrc(q, (uint32_t)(((kScanCh - 1) * ds + L) * esz));
@@ -1862,7 +1862,7 @@ mamba_scan_seg_kernel(ScanParams p) {
 // LDS, and over channel tiles in the final pass (scan_bwd_finalize_kernel)
 // in a fixed order, so every gradient is deterministic.
 // ---------------------------------------------------------------------------
-template <typename TU, typename TD, typename TBC, bool kSoftplus>
+template <typename TU, typename TD, typename TBC, bool kSoftplus, bool kSeg>
 __global__ void __launch_bounds__(256)
 mamba_scan_bwd_kernel(ScanParams p) {
   __shared__ float Bs[16 * kBStride];                  // B[n][t] of the tile
@@ -1877,7 +1877,7 @@ mamba_scan_bwd_kernel(ScanParams p) {
   const int n = lane % 16;
 
   const int per_batch = p.ngroups * p.tiles_per_group;
-  const ScanSeg sg(p, blockIdx.x / per_batch);
+  const ScanSeg<kSeg> sg(p, blockIdx.x / per_batch);
   const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / p.tiles_per_group;
   const int tile = blockIdx.x % p.tiles_per_group;
@@ -1955,7 +1955,7 @@ mamba_scan_bwd_kernel(ScanParams p) {
   // gradient of the state after the step being processed, decay of the step
   // after it; they start from the adjoint of the segments behind this one
   float gs = (ch_ok && n_ok) ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f;
-  float a_next = 1.0f;
+  float a_next = kSeg ? 1.0f : 0.0f;
   float dA_acc = 0.0f;
   float dD_acc = 0.0f, dbias_acc = 0.0f;  // reducer role: channel c, steps 16 blk + n
 
@@ -2277,6 +2277,13 @@ bool scan_fast_ok(const ScanParams& p, bool prep = false, int wgc = kScanCh, boo
          fits(p.dstate, p.B_ns, sizeof(TBC)) && fits(p.dstate, p.C_ns, sizeof(TBC));
 }
 
+// Calls f with whether the scan is cut into segments, as a type.
+template <typename F>
+void by_cut(const ScanParams& p, F&& f) {
+  if (p.segs > 1) f(std::true_type{});
+  else f(std::false_type{});
+}
+
 // Producer / consumer waves for whole tiles, and in their kRag form for other
 // lengths and alignments. Returns whether they take the call.
 template <typename TU, typename TD, typename TBC, int kMode>
@@ -2285,11 +2292,22 @@ bool launch_split(const ScanParams& p, int grid, hipStream_t s) {
   const bool whole = scan_fast_ok<TU, TD, TBC>(p, kPrep);
   if (!whole && !scan_fast_ok<TU, TD, TBC>(p, kPrep, kScanCh, true)) return false;
   const dim3 g(grid), t(512);
-  if (whole && p.softplus) mamba_scan_split_kernel<TU, TD, TBC, true, kMode, false><<<g, t, 0, s>>>(p);
-  else if (whole) mamba_scan_split_kernel<TU, TD, TBC, false, kMode, false><<<g, t, 0, s>>>(p);
-  else if (p.softplus) mamba_scan_split_kernel<TU, TD, TBC, true, kMode, true><<<g, t, 0, s>>>(p);
-  else mamba_scan_split_kernel<TU, TD, TBC, false, kMode, true><<<g, t, 0, s>>>(p);
+  by_cut(p, [&](auto cut) {
+    constexpr bool kSeg = decltype(cut)::value;
+    if (whole && p.softplus) mamba_scan_split_kernel<TU, TD, TBC, true, kMode, false, kSeg><<<g, t, 0, s>>>(p);
+    else if (whole) mamba_scan_split_kernel<TU, TD, TBC, false, kMode, false, kSeg><<<g, t, 0, s>>>(p);
+    else if (p.softplus) mamba_scan_split_kernel<TU, TD, TBC, true, kMode, true, kSeg><<<g, t, 0, s>>>(p);
+    else mamba_scan_split_kernel<TU, TD, TBC, false, kMode, true, kSeg><<<g, t, 0, s>>>(p);
+  });
   return true;
+}
+
+// The general forward, or the backward's preparation pass (kPrep).
+template <typename TU, typename TD, typename TBC, bool kPrep>
+void launch_general(const ScanParams& p, int grid, hipStream_t s) {
+  by_cut(p, [&](auto cut) {
+    mamba_scan_fwd_kernel<TU, TD, TBC, kPrep, decltype(cut)::value><<<dim3(grid), dim3(256), 0, s>>>(p);
+  });
 }
 
 template <typename TU, typename TD, typename TBC>
@@ -2305,7 +2323,7 @@ void launch_scan(const ScanParams& p, hipStream_t s) {
   const bool done = lean ? launch_split<TU, TD, TBC, kFwdLean>(p, grid, s)
                   : train ? launch_split<TU, TD, TBC, kFwdTrain>(p, grid, s)
                           : launch_split<TU, TD, TBC, kFwdAny>(p, grid, s);
-  if (!done) mamba_scan_fwd_kernel<TU, TD, TBC><<<dim3(grid), dim3(256), 0, s>>>(p);
+  if (!done) launch_general<TU, TD, TBC, false>(p, grid, s);
 }
 
 // dstate in (16, 64] with variable B / C: the specialised kernel with 2 or 4
@@ -2415,23 +2433,24 @@ void launch_scan_bwd(const ScanParams& p, void* dB, void* dC, float* dA, float* 
     if (p.z && launch_split<TU, TD, TBC, kPrepGated>(p, grid, s)) {
       // producer / consumer waves
     } else if (p.z) {
-      mamba_scan_fwd_kernel<TU, TD, TBC, true><<<dim3(grid), dim3(256), 0, s>>>(p);
-    }
-    else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1 && p.softplus)
+      launch_general<TU, TD, TBC, true>(p, grid, s);
+    } else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1 && p.softplus)
       mamba_scan_fast_kernel<TU, TD, TBC, true, true><<<dim3(grid), dim3(256), 0, s>>>(p);
     else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1)
       mamba_scan_fast_kernel<TU, TD, TBC, false, true><<<dim3(grid), dim3(256), 0, s>>>(p);
     else
-      mamba_scan_fwd_kernel<TU, TD, TBC, true><<<dim3(grid), dim3(256), 0, s>>>(p);
+      launch_general<TU, TD, TBC, true>(p, grid, s);
   }
   if (p.segs > 1) mamba_scan_seg_kernel<TU, TD, TBC, true><<<seg_grid, dim3(256), 0, s>>>(p);
   ScanParams q = p;  // the whole-tile pass may write fewer, wider dB / dC partial rows
   if (launch_scan_bwd_fast(q, dtype_code_of<TU>(), dtype_code_of<TD>(), dtype_code_of<TBC>(), s)) {
     // whole tiles: the buffer-resource reverse pass
-  } else if (p.softplus) {
-    mamba_scan_bwd_kernel<TU, TD, TBC, true><<<dim3(grid), dim3(256), 0, s>>>(p);
   } else {
-    mamba_scan_bwd_kernel<TU, TD, TBC, false><<<dim3(grid), dim3(256), 0, s>>>(p);
+    by_cut(p, [&](auto cut) {
+      constexpr bool kSeg = decltype(cut)::value;
+      if (p.softplus) mamba_scan_bwd_kernel<TU, TD, TBC, true, kSeg><<<dim3(grid), dim3(256), 0, s>>>(p);
+      else mamba_scan_bwd_kernel<TU, TD, TBC, false, kSeg><<<dim3(grid), dim3(256), 0, s>>>(p);
+    });
   }
   scan_bwd_finish<TBC>(q, dB, dC, dA, dD, dbias, s);
 }

@@ -36,8 +36,9 @@
 namespace ak {
 namespace {
 
-// kWv waves (4 or 8) of 4 channels each per workgroup.
-template <typename TU, typename TD, typename TBC, bool kSoftplus, bool kGate, bool kDz, int kWv>
+// kWv waves (4 or 8) of 4 channels each per workgroup; kSeg: a sequence in
+// segments (four waves only, the launcher's rule).
+template <typename TU, typename TD, typename TBC, bool kSoftplus, bool kGate, bool kDz, int kWv, bool kSeg>
 __global__ void __launch_bounds__(64 * kWv)
 mamba_scan_bwd_fast_kernel(ScanParams p) {
   static_assert(kWv == 4 || kWv == 8, "16 or 32 channels per workgroup");
@@ -54,13 +55,9 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
   const int n = lane % 16;
   const int tpg = p.tiles_per_group;  // whole kCh-channel tiles
   const int per_batch = p.ngroups * tpg;
-  // Only the four-wave form takes a sequence in segments (the launcher's rule);
-  // with the segments' bounds read at run time the eight-wave form took 450
-  // instead of 440 us ([4, 2048, 4096] with dz).
-  constexpr bool kSeg = kWv == 4;
   const int bs = blockIdx.x / per_batch;  // batch and segment
-  const ScanSeg sg(p, bs);
-  const int b = kSeg ? sg.b : bs;
+  const ScanSeg<kSeg> sg(p, bs);
+  const int b = sg.b;
   const int g = (blockIdx.x % per_batch) / tpg;
   const int tile = blockIdx.x % tpg;
   const int d0 = g * p.ch_per_group + tile * kCh;
@@ -141,10 +138,9 @@ mamba_scan_bwd_fast_kernel(ScanParams p) {
 
   // the adjoint of the segments behind this one, as the product of a step's
   // state gradient and the decay that follows it
-  float gs = 0.0f, a_next = kSeg ? 1.0f : 0.0f;
-  if constexpr (kSeg) gs = n_ok ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f;
+  float gs = n_ok ? seg_enter<true>(p, sg, d, n, a_scaled) : 0.0f, a_next = kSeg ? 1.0f : 0.0f;
   float dA_acc = 0.0f, dD_acc = 0.0f, dbias_acc = 0.0f;
-  const int t_lo = kSeg ? sg.first : 0, nt = kSeg ? sg.end : p.seqlen / kScanT;  // tiles nt - 1 down to t_lo
+  const int t_lo = sg.first, nt = kSeg ? sg.end : p.seqlen / kScanT;  // tiles nt - 1 down to t_lo
   Raw4<TBC> bv{}, cv{};
   if (stager) {
     bv = bload4<TBC>(rs_B, vo_B, (uint32_t)(nt - 1) * kScanT * sizeof(TBC));
@@ -390,9 +386,11 @@ bool launch_fast(ScanParams& p, hipStream_t s) {
   auto go = [&](auto sp, auto gt, auto dzt) {
     constexpr bool kSp = decltype(sp)::value, kGt = decltype(gt)::value, kDzt = decltype(dzt)::value;
     if (wide)
-      mamba_scan_bwd_fast_kernel<TU, TD, TBC, kSp, kGt, kDzt, 8><<<dim3(grid), dim3(512), 0, s>>>(p);
+      mamba_scan_bwd_fast_kernel<TU, TD, TBC, kSp, kGt, kDzt, 8, false><<<dim3(grid), dim3(512), 0, s>>>(p);
+    else if (p.segs > 1)
+      mamba_scan_bwd_fast_kernel<TU, TD, TBC, kSp, kGt, kDzt, 4, true><<<dim3(grid), dim3(256), 0, s>>>(p);
     else
-      mamba_scan_bwd_fast_kernel<TU, TD, TBC, kSp, kGt, kDzt, 4><<<dim3(grid), dim3(256), 0, s>>>(p);
+      mamba_scan_bwd_fast_kernel<TU, TD, TBC, kSp, kGt, kDzt, 4, false><<<dim3(grid), dim3(256), 0, s>>>(p);
   };
   using T = std::true_type;
   using F = std::false_type;
