@@ -70,26 +70,35 @@ struct ScanParams {
 // segment's state from zero and its sum of delta' (all of its decay: the
 // product of exp(delta' A) is exp(A sum delta')); the scan's workgroups then
 // fold the segments before theirs into their entering state. The recurrence's
-// exponentials are paid twice and a launch is added, so: up to 128 workgroups
-// of 16 channels, about 512 segments in all (two workgroups a CU) from 4 tiles
-// on; up to 192 workgroups, about 1024 from 24 tiles on. Measured (us, one
-// segment -> cut): training [1, 384, 4096] 422 -> 85, [1, 2048, 1024] 124 -> 82,
-// [1, 768, 671] 113 -> 46, [2, 1536, 2048] (192) 237 -> 203; inference [1, 2048,
-// 1777] 88 -> 52, [1, 768, 4096] 100 -> 43, [1, 384, 512] 15.1 -> 10.6. Cut,
-// training [4, 768, 512] (192) would go 69 -> 72, [1, 1536, 128] 27.6 -> 29.7,
-// inference [2, 2048, 1024] (256) 30 -> 40. A function of the shape alone: the
-// bits of a result depend on it.
+// exponentials are paid twice and a launch is added, so what pays depends on the
+// pass (us, uncut -> cut, bf16, 64-step tiles x workgroups of 16 channels):
+// * forward, about 512 segments in all (two workgroups a CU). Up to 64 workgroups
+//   from 6 tiles on (6 x 64: 11.5 -> 11.4, x 24: 11.5 -> 9.4; 4 x 24 would go
+//   8.6 -> 9.4); up to 128 from 16 on (16 x 96: 25.9 -> 24.1, x 128: 26.1 -> 24.4;
+//   12 x 128 20.4 -> 20.5), from 12 on with a partial tile, whose kernel is the
+//   slower one (12 x 128: 22.7 -> 21.1); about 1024 segments up to 144 from 64 tiles
+//   (64 x 144: 95.9 -> 88; 32 x 144 49.6 -> 52), with a partial tile from 32 (57.3
+//   -> 54). 64 x 160 would go 96.5 -> 99, 24 x 192 38.4 -> 49.
+// * reverse pass, with three exponentials a step to the segment pass's one: about
+//   512 segments up to 128 workgroups from 4 tiles on (4 x 128: 34.6 -> 28.6, with
+//   its preparation pass 43 -> 39), about 1024 up to 192 from 24 on (24 x 192:
+//   128 -> 103, 170 -> 151; 24 x 144 126 -> 89).
+// A function of the shape alone: the bits of a result depend on it. Where the
+// forward is cut, the reverse pass is cut alike.
 struct ScanSegs {
   int n, tiles;
 };
-inline ScanSegs scan_segments(int64_t batch, int64_t dim, int64_t seqlen, int64_t dstate,
+inline ScanSegs scan_segments(bool reverse, int64_t batch, int64_t dim, int64_t seqlen, int64_t dstate,
                               int64_t ngroups, int bc_flags) {
   const int64_t tiles = (seqlen + kScanT - 1) / kScanT;
   const int64_t groups = batch * ngroups * ((dim / ngroups + kScanCh - 1) / kScanCh);
+  const bool whole = seqlen % kScanT == 0;
   int64_t n = 1;
   if (dstate <= 16 && !(bc_flags & (AK_SCAN_B_CONST | AK_SCAN_C_CONST)) && groups > 0) {
-    if (groups <= 128 && tiles >= 4) n = (512 + groups / 2) / groups;
-    else if (groups <= 192 && tiles >= 24) n = 1024 / groups;
+    const int64_t few = reverse ? 4 : groups <= 64 ? 6 : whole ? 16 : 12;  // tiles from which on a cut pays
+    const int64_t many = reverse ? 24 : whole ? 64 : 32;
+    if (groups <= 128 && tiles >= few) n = (512 + groups / 2) / groups;
+    else if (groups <= (reverse ? 192 : 144) && tiles >= many) n = 1024 / groups;
     if (n > 32) n = 32;
     if (n > tiles) n = tiles;
     if (n < 1) n = 1;
@@ -245,7 +254,7 @@ inline ScanBwdWs scan_bwd_ws(int64_t batch, int64_t dim, int64_t seqlen, int64_t
   w.ck = a256(batch * nck * dim * dstate * 4);
   w.partB = bc ? 0 : a256(tiles * batch * ngroups * dstate * seqlen * 4);
   w.partC = cc ? 0 : a256(tiles * batch * ngroups * dstate * seqlen * 4);
-  const ScanSegs sg = scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags);
+  const ScanSegs sg = scan_segments(true, batch, dim, seqlen, dstate, ngroups, bc_flags);
   w.seg = scan_seg_ws(sg, batch, dim, dstate);
   w.dA = a256(batch * sg.n * dim * dstate * 4);  // a partial per batch and segment
   w.dD = a256(batch * sg.n * dim * 4);

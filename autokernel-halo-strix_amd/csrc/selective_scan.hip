@@ -2424,22 +2424,31 @@ constexpr int dtype_code_of() {
 // states and computes dz itself.
 template <typename TU, typename TD, typename TBC>
 void launch_scan_bwd(const ScanParams& p, void* dB, void* dC, float* dA, float* dD, float* dbias,
-                     bool saved_states, hipStream_t s) {
+                     bool saved_states, bool cut_forward, hipStream_t s) {
   const int groups = p.batch * p.ngroups * p.tiles_per_group;
   const int grid = groups * p.segs;
   const dim3 seg_grid(groups * (p.segs - 1));
-  if (!saved_states) {  // preparation pass: states every 16 steps and dz
-    if (p.segs > 1) mamba_scan_seg_kernel<TU, TD, TBC, false><<<seg_grid, dim3(256), 0, s>>>(p);
-    if (p.z && launch_split<TU, TD, TBC, kPrepGated>(p, grid, s)) {
+  if (!saved_states) {
+    // preparation pass: states every 16 steps and dz. It cuts the sequence as the
+    // forward does (there, into the reverse pass's segments), so that the states
+    // have the bits of saved ones.
+    ScanParams f = p;
+    if (!cut_forward) {
+      f.segs = 1;
+      f.seg_tiles = (p.seqlen + kScanT - 1) / kScanT;
+    }
+    const int grid = groups * f.segs;
+    if (f.segs > 1) mamba_scan_seg_kernel<TU, TD, TBC, false><<<seg_grid, dim3(256), 0, s>>>(f);
+    if (f.z && launch_split<TU, TD, TBC, kPrepGated>(f, grid, s)) {
       // producer / consumer waves
-    } else if (p.z) {
-      launch_general<TU, TD, TBC, true>(p, grid, s);
-    } else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1 && p.softplus)
-      mamba_scan_fast_kernel<TU, TD, TBC, true, true><<<dim3(grid), dim3(256), 0, s>>>(p);
-    else if (scan_fast_ok<TU, TD, TBC>(p, true) && p.segs == 1)
-      mamba_scan_fast_kernel<TU, TD, TBC, false, true><<<dim3(grid), dim3(256), 0, s>>>(p);
+    } else if (f.z) {
+      launch_general<TU, TD, TBC, true>(f, grid, s);
+    } else if (scan_fast_ok<TU, TD, TBC>(f, true) && f.segs == 1 && f.softplus)
+      mamba_scan_fast_kernel<TU, TD, TBC, true, true><<<dim3(grid), dim3(256), 0, s>>>(f);
+    else if (scan_fast_ok<TU, TD, TBC>(f, true) && f.segs == 1)
+      mamba_scan_fast_kernel<TU, TD, TBC, false, true><<<dim3(grid), dim3(256), 0, s>>>(f);
     else
-      launch_general<TU, TD, TBC, true>(p, grid, s);
+      launch_general<TU, TD, TBC, true>(f, grid, s);
   }
   if (p.segs > 1) mamba_scan_seg_kernel<TU, TD, TBC, true><<<seg_grid, dim3(256), 0, s>>>(p);
   ScanParams q = p;  // the whole-tile pass may write fewer, wider dB / dC partial rows
@@ -2457,15 +2466,16 @@ void launch_scan_bwd(const ScanParams& p, void* dB, void* dC, float* dA, float* 
 
 template <typename TU>
 int dispatch_scan_bwd(const ScanParams& p, int u_dtype, int delta_dtype, int bc_dtype, void* dB,
-                      void* dC, float* dA, float* dD, float* dbias, bool saved_states, hipStream_t s) {
+                      void* dC, float* dA, float* dD, float* dbias, bool saved_states, bool cut_forward,
+                      hipStream_t s) {
   const bool d32 = delta_dtype == AK_DTYPE_F32;
   const bool bc32 = bc_dtype == AK_DTYPE_F32;
   if (!d32 && delta_dtype != u_dtype) return -1;
   if (!bc32 && bc_dtype != u_dtype) return -1;
-  if (d32 && bc32) launch_scan_bwd<TU, float, float>(p, dB, dC, dA, dD, dbias, saved_states, s);
-  else if (d32) launch_scan_bwd<TU, float, TU>(p, dB, dC, dA, dD, dbias, saved_states, s);
-  else if (bc32) launch_scan_bwd<TU, TU, float>(p, dB, dC, dA, dD, dbias, saved_states, s);
-  else launch_scan_bwd<TU, TU, TU>(p, dB, dC, dA, dD, dbias, saved_states, s);
+  if (d32 && bc32) launch_scan_bwd<TU, float, float>(p, dB, dC, dA, dD, dbias, saved_states, cut_forward, s);
+  else if (d32) launch_scan_bwd<TU, float, TU>(p, dB, dC, dA, dD, dbias, saved_states, cut_forward, s);
+  else if (bc32) launch_scan_bwd<TU, TU, float>(p, dB, dC, dA, dD, dbias, saved_states, cut_forward, s);
+  else launch_scan_bwd<TU, TU, TU>(p, dB, dC, dA, dD, dbias, saved_states, cut_forward, s);
   return 0;
 }
 
@@ -2562,7 +2572,7 @@ int scan_fwd_entry(
   p.softplus = delta_softplus ? 1 : 0;
   hipStream_t s = ak_stream(stream);
   if (workspace && a_dtype != AK_DTYPE_C64) {
-    const ak::ScanSegs sg = ak::scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags);
+    const ak::ScanSegs sg = ak::scan_segments(false, batch, dim, seqlen, dstate, ngroups, bc_flags);
     const ak::ScanSegWs ws = ak::scan_seg_ws(sg, batch, dim, dstate);
     if (workspace_bytes < ws.state + ws.dsum)
       return ak_set_error(AK_ERR_WORKSPACE, "%s: workspace %zu bytes < required %zu", name,
@@ -2624,7 +2634,7 @@ extern "C" size_t ak_selective_scan_fwd_workspace_bytes(int64_t batch, int64_t d
   if (batch <= 0 || dim <= 0 || seqlen <= 0 || dstate <= 0 || ngroups <= 0 || dim % ngroups) return 0;
   if (bc_flags & AK_SCAN_A_COMPLEX) return 0;
   const ak::ScanSegWs ws = ak::scan_seg_ws(
-      ak::scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags), batch, dim, dstate);
+      ak::scan_segments(false, batch, dim, seqlen, dstate, ngroups, bc_flags), batch, dim, dstate);
   return ws.state + ws.dsum;
 }
 
@@ -2881,22 +2891,23 @@ extern "C" int ak_selective_scan_bwd(
   p.dbias_part = take(ws.dD);
   p.dBc_part = take(ws.dBc);
   p.dCc_part = take(ws.dCc);
-  ak::use_segments(p, ak::scan_segments(batch, dim, seqlen, dstate, ngroups, bc_flags), ws.seg, w + off);
+  ak::use_segments(p, ak::scan_segments(true, batch, dim, seqlen, dstate, ngroups, bc_flags), ws.seg, w + off);
   // saved forward states: the reverse pass reads them (and out_prez) in place
   if (checkpoints) {
     p.ck = const_cast<float*>(checkpoints);
     p.out_prez = const_cast<void*>(out_prez);
   }
   const bool saved = checkpoints != nullptr;
+  const bool cut_forward = ak::scan_segments(false, batch, dim, seqlen, dstate, ngroups, bc_flags).n > 1;
   if (ak::scan_needs_wide(p)) {
     if (!saved) rc = ak::launch_scan_wide_fwd(p, true, u_dtype, delta_dtype, bc_eff, s);
     if (!rc) rc = ak::launch_scan_wide_bwd(p, u_dtype, delta_dtype, bc_eff, s);
     if (!rc) rc = ak::finish_for(bc_eff, p, dB, dC, dA, dD, ddelta_bias, s);
   } else {
     switch (u_dtype) {
-      case AK_DTYPE_F32: rc = ak::dispatch_scan_bwd<float>(p, u_dtype, delta_dtype, bc_eff, dB, dC, dA, dD, ddelta_bias, saved, s); break;
-      case AK_DTYPE_F16: rc = ak::dispatch_scan_bwd<ak::f16>(p, u_dtype, delta_dtype, bc_eff, dB, dC, dA, dD, ddelta_bias, saved, s); break;
-      default: rc = ak::dispatch_scan_bwd<ak::bf16>(p, u_dtype, delta_dtype, bc_eff, dB, dC, dA, dD, ddelta_bias, saved, s); break;
+      case AK_DTYPE_F32: rc = ak::dispatch_scan_bwd<float>(p, u_dtype, delta_dtype, bc_eff, dB, dC, dA, dD, ddelta_bias, saved, cut_forward, s); break;
+      case AK_DTYPE_F16: rc = ak::dispatch_scan_bwd<ak::f16>(p, u_dtype, delta_dtype, bc_eff, dB, dC, dA, dD, ddelta_bias, saved, cut_forward, s); break;
+      default: rc = ak::dispatch_scan_bwd<ak::bf16>(p, u_dtype, delta_dtype, bc_eff, dB, dC, dA, dD, ddelta_bias, saved, cut_forward, s); break;
     }
   }
   if (rc) return ak_set_error(AK_ERR_UNSUPPORTED, "%s: delta and a variable B/C must be fp32 or the dtype of u", name);

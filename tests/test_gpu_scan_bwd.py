@@ -368,8 +368,9 @@ def test_saved_states_c_abi():
     (1, 16, 4, 1, "Dzb"), (1, 16, 63, 1, "z"), (2, 32, 193, 1, "Dzb"), (1, 16, 255, 1, "Dzb"), (1, 32, 256, 2, "Dzb"),
     (1, 16, 321, 1, ""), (1, 24, 700, 1, "Dzb"), (1, 16, 2111, 1, "Dzb"), (3, 64, 1025, 2, "zb"), (8, 384, 1537, 1, "Dzb")])
 def test_segments_and_ragged_lengths(itype, batch, dim, seqlen, groups, opts):
-    """Sequences cut into segments (from 4 tiles on, one to several tiles each;
-    (8, 384, 1537) takes the plan of 192 channel groups) and every length's
+    """Sequences cut into segments (the forward from 6 tiles on, the reverse pass
+    from 4, one to several tiles each; (8, 384, 1537) takes the reverse plan of 192
+    channel groups over an uncut forward) and every length's
     partial tile, from views that start off the alignment grid: outputs, last
     state, chunk states and gradients against the one-segment call (states and
     outputs equal to fp32 rounding: |h| times 2e-6 a step boundary, and one
@@ -443,22 +444,22 @@ def test_segments_and_ragged_lengths(itype, batch, dim, seqlen, groups, opts):
 
 def test_segments_of_a_growing_recurrence():
     """A decay that grows (A > 0 with a positive delta, or a negative delta) and
-    passes fp32's range over one segment of four, while the states and adjoints
+    passes fp32's range over one segment of six, while the states and adjoints
     that it carries do not: a sum of A delta of 96 is a factor of 5e41 on inputs
     and upstream gradients of 1e-10. Per step the exponent is off by 2^-23 of
     itself at most and the exponential by 2 units, so 64 steps by about 3e-5."""
     need_gpu()
     from kernels.hip.selective_scan import selective_scan_fn
-    u, delta = torch.zeros(1, 16, 256), torch.zeros(1, 16, 256)
+    u, delta = torch.zeros(1, 16, 384), torch.zeros(1, 16, 384)
     A = torch.ones(16, 16) * torch.linspace(0.25, 1.0, 16)
     A[8:] *= -1  # these channels grow by a negative delta
     u[..., :64] = 1e-10
     delta[..., :64], delta[..., 64:128], delta[..., 128:] = 0.01, 1.5, 0.001
     delta[:, 8:] *= -1
     u[:, 8:] *= -1  # delta u and all that it feeds stay positive: no sum over channels cancels, so the bound is relative
-    B, C = torch.ones(1, 1, 16, 256), torch.ones(1, 1, 16, 256)
-    dout = torch.zeros(1, 16, 256)
-    dout[..., 192:] = 1e-10
+    B, C = torch.ones(1, 1, 16, 384), torch.ones(1, 1, 16, 384)
+    dout = torch.zeros(1, 16, 384)
+    dout[..., 320:] = 1e-10
     say("scan segments, growing")
     args = [t.to(DEV) for t in (u, delta, A, B, C)]
     out, last = selective_scan_fn(*args, return_last_state=True)
@@ -477,10 +478,50 @@ def test_segments_keep_an_infinite_state():
     underflows as one number but not step by step, as in the uncut recurrence."""
     need_gpu()
     from kernels.hip.selective_scan import selective_scan_fn
-    u, delta = torch.zeros(1, 16, 256, device=DEV), torch.full((1, 16, 256), 2.0, device=DEV)
+    u, delta = torch.zeros(1, 16, 384, device=DEV), torch.full((1, 16, 384), 2.0, device=DEV)
     u[..., 3] = 3e38
     A = -torch.ones(16, 16, device=DEV)
-    B, C = torch.full((1, 16, 256), 4.0, device=DEV), torch.ones(1, 16, 256, device=DEV)
+    B, C = torch.full((1, 16, 384), 4.0, device=DEV), torch.ones(1, 16, 384, device=DEV)
     say("scan segments, infinite state")
     _, last = selective_scan_fn(u, delta, A, B, C, return_last_state=True)
     assert bool((last == float("inf")).all())
+
+
+@pytest.mark.parametrize("batch,dim,seqlen,segs", [
+    (1, 16, 320, 1), (1, 1024, 321, 6), (1, 1040, 704, 1), (1, 1040, 705, 6), (1, 2048, 960, 1), (1, 2048, 1024, 4),
+    (1, 2064, 1984, 1), (1, 2064, 1985, 7), (2, 1152, 4032, 1), (2, 1152, 4096, 7), (1, 2320, 4095, 1)])
+def test_forward_cuts_at_the_edges_of_the_rule(batch, dim, seqlen, segs):
+    """64, 128 and 144 channel groups, whole and partial last tiles: how many
+    segments the forward's scratch is for, and the cut scan against the one
+    without scratch (states equal to fp32 rounding, 4e-6 of the largest, outputs
+    to one more rounding)."""
+    need_gpu()
+    from kernels.hip import _lib
+    g = torch.Generator(device=DEV).manual_seed(dim + seqlen)
+
+    def r(*shape):
+        return torch.randn(*shape, generator=g, device=DEV).bfloat16()
+
+    say("forward cuts", batch, dim, seqlen)
+    u, delta, z, B, C = r(batch, dim, seqlen), r(batch, dim, seqlen), r(batch, dim, seqlen), r(batch, 16, seqlen), r(batch, 16, seqlen)
+    A = -torch.arange(1, 17, device=DEV).float().repeat(dim, 1)
+    D, bias = torch.ones(dim, device=DEV), torch.full((dim,), -4.0, device=DEV)
+    lib = _lib.load()
+    need = int(lib.ak_selective_scan_fwd_workspace_bytes(batch, dim, seqlen, 16, 1, 0))
+    a256 = lambda v: -(-v // 256) * 256  # noqa: E731
+    assert need == (0 if segs == 1 else a256(4 * batch * segs * dim * 16) + a256(4 * batch * segs * dim))
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    runs = []
+    for scratch in (ws.data_ptr() if need else None, None):
+        out, last = torch.empty_like(u), torch.empty(batch, dim, 16, device=DEV)
+        p = [t.data_ptr() for t in (u, delta, A, B, C, D, z, bias, out, last)]
+        rc = lib.ak_selective_scan_fwd_ws(
+            *p, None, None, None, batch, dim, seqlen, 16, 1, dim * seqlen, seqlen, dim * seqlen, seqlen, 16,
+            16 * seqlen, 16 * seqlen, seqlen, 16 * seqlen, 16 * seqlen, seqlen, dim * seqlen, seqlen, dim * seqlen, seqlen,
+            1, 0, *[_lib.dtype_code(u.dtype)] * 3, _lib.dtype_code(A.dtype), scratch, need if scratch else 0,
+            torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        runs.append((out.double(), last.double()))
+    (out, last), (one_out, one_last) = runs
+    assert bool(((last - one_last).abs() <= 4e-6 * one_last.abs().amax()).all())
+    assert bool(((out - one_out).abs() <= 2.0 ** -7 * one_out.abs() + 4e-6 * one_out.abs().amax()).all())
