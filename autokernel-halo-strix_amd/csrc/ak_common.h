@@ -104,6 +104,11 @@ __device__ __forceinline__ void store16_any_nt(T* p, const Vec16<T>& v) {
   __builtin_nontemporal_store(v.u, reinterpret_cast<u32x4_any*>(p));
 }
 
+template <typename T>
+__device__ __forceinline__ void store16_any(T* p, const Vec16<T>& v) {
+  *reinterpret_cast<u32x4_any*>(p) = v.u;
+}
+
 // Makes a held vector opaque, so that what a later pass derives from it is
 // derived again instead of being kept in registers from the pass before.
 template <typename T>

@@ -103,12 +103,13 @@ __device__ __forceinline__ float grad_value(const CeParams& p, const RowGrad& r,
 }
 
 // One vector of gradients; te: the target's place in it, or anything outside
-// [0, VE). Only the wave that holds the target compares element by element.
-template <typename T, bool CAP>
+// [0, VE). RARE: only the wave that holds the target compares element by
+// element, at the price of a second copy of the arithmetic.
+template <typename T, bool CAP, bool RARE>
 __device__ __forceinline__ Vec16<T> grad_vec(const CeParams& p, const RowGrad& r, const Vec16<T>& xv, int te) {
   constexpr int VE = Vec16<T>::VE;
   Vec16<T> o;
-  if ((unsigned)te < (unsigned)VE) {
+  if (!RARE || (unsigned)te < (unsigned)VE) {
 #pragma unroll
     for (int e = 0; e < VE; ++e) o.e[e] = from_f32<T>(grad_value<CAP>(p, r, to_f32(xv.e[e]), e == te));
   } else {
@@ -120,49 +121,59 @@ __device__ __forceinline__ Vec16<T> grad_vec(const CeParams& p, const RowGrad& r
 
 // Gradient of the row's elements [v0, v1) (vectors) and, where `ends` is set,
 // of the elements around the vectors: zero for ignored rows, NaN for
-// out-of-range targets, otherwise the softmax gradient. Four vectors of a
-// thread are loaded before the first is used.
-template <typename T, bool CAP>
+// out-of-range targets, otherwise the softmax gradient. U vectors of a thread
+// are loaded before the first is used. NT: past the caches. RAG: rows at any
+// address and of any width; otherwise whole aligned vectors.
+template <typename T, bool CAP, bool NT, bool RAG, int U, typename I>
 __device__ void write_grad_row(const CeParams& p, const T* __restrict__ row, T* __restrict__ grow,
-                               int64_t vocab, int64_t tgt, bool ignored, bool bad, float m,
-                               float s, int64_t v0, int64_t v1, bool ends, int threads) {
+                               I vocab, I tgt, bool ignored, bool bad, float m,
+                               float s, I v0, I v1, bool ends, int threads) {
   constexpr int VE = Vec16<T>::VE;
-  constexpr int U = 4;
-  const RowSplit<T, int64_t> sp(row, vocab);
   const int t = threadIdx.x;
-  const int64_t ex = ends && t < sp.nx ? sp.extra(t) : -1;
-  row += sp.head;  // row / grow: the vectors' first element
-  T* const gv = grow + sp.head;
-  if (v1 > sp.nvec) v1 = sp.nvec;
+  I nvec = vocab / VE, ex = -1, head = 0;
+  if constexpr (RAG) {
+    const RowSplit<T, I> sp(row, vocab);
+    nvec = sp.nvec;
+    head = sp.head;
+    if (ends && t < sp.nx) ex = sp.extra(t);
+  }
+  auto ld = [](const T* q) { return NT ? load16_any_nt(q) : load16_any(q); };
+  auto st = [](T* q, const Vec16<T>& w) {
+    if (NT) store16_any_nt(q, w);
+    else store16_any(q, w);
+  };
+  row += head;  // row / grow: the vectors' first element
+  T* const gv = grow + head;
+  if (v1 > nvec) v1 = nvec;
   if (ignored || bad) {
     const T c = from_f32<T>(ignored ? 0.0f : NAN);
     Vec16<T> o;
 #pragma unroll
     for (int e = 0; e < VE; ++e) o.e[e] = c;
-    for (int64_t v = v0 + t; v < v1; v += threads) store16_any_nt(gv + v * VE, o);
-    if (ex >= 0) grow[ex] = c;
+    for (I v = v0 + t; v < v1; v += threads) st(gv + (int64_t)v * VE, o);
+    if (RAG && ex >= 0) grow[ex] = c;
     return;
   }
-  const RowGrad r(p, m, s);
   float xe = 0.0f;
-  if (ex >= 0) xe = to_f32(row[ex - sp.head]);
-  const int64_t tv = tgt - sp.head;  // relative to the vectors
-  int64_t v = v0 + t;
-  for (; v + (U - 1) * threads < v1; v += U * threads) {
+  if (RAG && ex >= 0) xe = to_f32(row[ex - head]);
+  const I tv = tgt - head;  // relative to the vectors
+  auto place = [&](I v) {
+    const I d = tv - v * VE;
+    return d >= 0 && d < VE ? (int)d : -1;
+  };
+  I v = v0 + t;
+  const RowGrad r(p, m, s);
+  for (; U > 1 && v + (U - 1) * threads < v1; v += U * threads) {
     Vec16<T> x[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) x[u] = load16_any_nt(row + (v + u * threads) * VE);
+    for (int u = 0; u < U; ++u) x[u] = ld(row + (int64_t)(v + u * threads) * VE);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t at = (v + u * threads) * VE, d = tv - at;
-      store16_any_nt(gv + at, grad_vec<T, CAP>(p, r, x[u], d >= 0 && d < VE ? (int)d : -1));
-    }
+    for (int u = 0; u < U; ++u)
+      st(gv + (int64_t)(v + u * threads) * VE, grad_vec<T, CAP, true>(p, r, x[u], place(v + u * threads)));
   }
-  for (; v < v1; v += threads) {
-    const int64_t d = tv - v * VE;
-    store16_any_nt(gv + v * VE, grad_vec<T, CAP>(p, r, load16_any_nt(row + v * VE), d >= 0 && d < VE ? (int)d : -1));
-  }
-  if (ex >= 0) grow[ex] = from_f32<T>(grad_value<CAP>(p, r, xe, ex == tgt));
+  for (; v < v1; v += threads)
+    st(gv + (int64_t)v * VE, grad_vec<T, CAP, (U > 1)>(p, r, ld(row + (int64_t)v * VE), place(v)));
+  if (RAG && ex >= 0) grow[ex] = from_f32<T>(grad_value<CAP>(p, r, xe, ex == tgt));
 }
 
 // A row held in registers: TPR threads, VPT vectors each, packed between the
@@ -288,7 +299,7 @@ ce_row_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
         for (int k = 0; k < VPT; ++k)
           if (t + k * TPR < sp.nvec)
             store16_any_nt(gv + k * TPR * VE + (unsigned)(t * VE),
-                           grad_vec<T, CAP>(p, r, raw[k], tv - (t + k * TPR) * VE));
+                           grad_vec<T, CAP, true>(p, r, raw[k], tv - (t + k * TPR) * VE));
         if (ex >= 0) grow[ex] = from_f32<T>(grad_value<CAP>(p, r, to_f32(xe), ex == (int)tgt));
       } else {
         Vec16<T> o;
@@ -368,9 +379,9 @@ __device__ void ce_fwd_row(const T* __restrict__ row, int64_t b, const int64_t* 
   }
   if (grow) {
     if (p.use_softcap)
-      write_grad_row<T, true>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s, 0, vocab, true, kCeThreads);
+      write_grad_row<T, true, true, true, 4, int64_t>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s, 0, vocab, true, kCeThreads);
     else
-      write_grad_row<T, false>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s, 0, vocab, true, kCeThreads);
+      write_grad_row<T, false, true, true, 4, int64_t>(p, row, grow, vocab, tgt, ignored, bad, st.m, st.s, 0, vocab, true, kCeThreads);
   }
 }
 
@@ -390,19 +401,19 @@ ce_fwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
 
 // The gradient from the saved row statistics: blockIdx.y takes `span` vectors
 // of the row, so that few rows still fill the GPU.
-template <typename T, bool CAP>
+template <typename T, bool CAP, bool NT, bool RAG, int U, typename I>
 __global__ void __launch_bounds__(kCeThreads)
 ce_bwd_tiny_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
                    const float* __restrict__ row_max, const float* __restrict__ row_sum,
-                   T* __restrict__ grad, int64_t rows, int64_t vocab, int64_t ld, int64_t ld_g,
-                   int64_t span, CeParams p) {
-  const int64_t v0 = (int64_t)blockIdx.y * span;
+                   T* __restrict__ grad, int64_t rows, I vocab, int64_t ld, int64_t ld_g,
+                   I span, CeParams p) {
+  const I v0 = (I)blockIdx.y * span;
   for (int64_t b = blockIdx.x; b < rows; b += gridDim.x) {
     const int64_t tgt = targets[b];
     const bool ignored = tgt == p.ignore_index;
     const bool bad = !ignored && (tgt < 0 || tgt >= vocab);
-    write_grad_row<T, CAP>(p, logits + b * ld, grad + b * ld_g, vocab, tgt, ignored, bad, row_max[b],
-                           row_sum[b], v0, v0 + span, blockIdx.y == 0, kCeThreads);
+    write_grad_row<T, CAP, NT, RAG, U, I>(p, logits + b * ld, grad + b * ld_g, vocab, (I)tgt, ignored, bad, row_max[b],
+                              row_sum[b], v0, v0 + span, blockIdx.y == 0, kCeThreads);
   }
 }
 
@@ -527,6 +538,10 @@ int check(const void* logits, const int64_t* targets, void* grad, int64_t rows, 
   return AK_OK;
 }
 
+// Whether that many bytes pass the 256 MiB last-level cache, so that nothing of
+// them would be found there again.
+bool past_cache(int64_t bytes) { return bytes > (int64_t)300 << 20; }
+
 // The row-resident forward with the fewest vectors a thread that its workgroup
 // sizes allow (256 threads up to 1024 vectors, for more rows in flight).
 template <typename T, bool CAP>
@@ -555,13 +570,14 @@ void launch_fwd(const void* logits, const int64_t* targets, float* losses, float
                 const CeParams& p, hipStream_t s) {
   const T* lg = static_cast<const T*>(logits);
   T* g = static_cast<T*>(grad);
+  constexpr int VE = Vec16<T>::VE;
+  const bool aligned = vocab % VE == 0 && ld % VE == 0 && aligned16(logits);
   const bool done = p.use_softcap
       ? launch_row<T, true>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, s)
       : launch_row<T, false>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, s);
   if (done) return;
-  constexpr int VE = Vec16<T>::VE;
   const dim3 grid(row_grid(rows)), block(kCeThreads);
-  if (vocab % VE == 0 && ld % VE == 0 && aligned16(logits))
+  if (aligned)
     ce_fwd_kernel<T, true><<<grid, block, 0, s>>>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p);
   else
     ce_fwd_kernel<T, false><<<grid, block, 0, s>>>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p);
@@ -579,10 +595,32 @@ void launch_bwd(const void* logits, const int64_t* targets, const float* mx, con
   const int64_t ny = std::min<int64_t>(nvec / (4 * kCeThreads), 65535);
   const int64_t span = ny > 1 ? (nvec + ny - 1) / ny : nvec;
   const dim3 grid(row_grid(rows), ny > 1 ? (unsigned)ny : 1), block(kCeThreads);
-  if (p.use_softcap)
-    ce_bwd_tiny_kernel<T, true><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, vocab, ld, ld_g, span, p);
-  else
-    ce_bwd_tiny_kernel<T, false><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, vocab, ld, ld_g, span, p);
+  auto go = [&](auto nt, auto rag, auto unroll, auto index) {
+    using I = decltype(index);
+    constexpr bool NT = decltype(nt)::value, RAG = decltype(rag)::value;
+    constexpr int U = decltype(unroll)::value;
+    if (p.use_softcap)
+      ce_bwd_tiny_kernel<T, true, NT, RAG, U, I><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, (I)vocab, ld, ld_g, (I)span, p);
+    else
+      ce_bwd_tiny_kernel<T, false, NT, RAG, U, I><<<grid, block, 0, s>>>(lg, targets, mx, sm, g, rows, (I)vocab, ld, ld_g, (I)span, p);
+  };
+  // One vector at a time where a row has no round of four (fewer registers, more
+  // rows in flight: [4096, 1024] fp32 8.1 -> 6.6 us). Nontemporal accesses where the logits
+  // and their gradient pass the 256 MiB last-level cache ([4096, 32768] bf16 90.8 us
+  // so, 100.8 without; [2048, 16384] fp32, 268 MB: 45.5 and 41.3, as the forward's
+  // logits are still there). 32-bit columns, a shorter chain of address arithmetic,
+  // up to 2^30 of them.
+  using One = std::integral_constant<int, 1>;
+  using Four = std::integral_constant<int, 4>;
+  const bool big = past_cache(2 * rows * vocab * (int64_t)sizeof(T));
+  using Yes = std::true_type;
+  using No = std::false_type;
+  const bool aligned = vocab % Vec16<T>::VE == 0 && ld % Vec16<T>::VE == 0 && aligned16(logits);
+  if (vocab >= (int64_t)1 << 30) go(Yes{}, Yes{}, Four{}, int64_t{});
+  else if (nvec < 4 * kCeThreads && aligned) go(No{}, No{}, One{}, int{});
+  else if (nvec < 4 * kCeThreads) go(No{}, Yes{}, One{}, int{});
+  else if (big) go(Yes{}, Yes{}, Four{}, int64_t{});
+  else go(No{}, Yes{}, Four{}, int64_t{});
 }
 
 }  // namespace

@@ -298,3 +298,41 @@ def test_ce_fused_backward_kept_graphs_and_hooks():
         loss = ce_full(x, t, mode="fused")
     assert torch.equal(torch.autograd.grad(loss, x, two)[0], want * 2)
     assert torch.equal(held[0], want)
+
+
+@pytest.mark.parametrize("dtype,rows,vocab,softcap", [
+    (torch.bfloat16, 1400, 60000, 0.0),      # logits and gradient past the last-level cache
+    (torch.bfloat16, 1400, 60001, 20.0)])
+def test_ce_rows_by_size(dtype, rows, vocab, softcap):
+    """Row statistics without a gradient and the gradient from them, in the forms
+    that the number of rows and bytes choose, against float64: sums of positive
+    terms to 1e-5, the gradient to one rounding of its type beside 1e-5 of it
+    (fp16's subnormals: 2^-25 absolute)."""
+    need_gpu()
+    from kernels.hip import _lib
+    g = torch.Generator(device=DEV).manual_seed(rows + vocab)
+    x = (2 * torch.randn(rows, vocab, generator=g, device=DEV)).to(dtype)
+    t = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    t[5] = -100
+    say("ce rows by size", dtype, rows, vocab, softcap)
+    losses, lse, mx, sm = (torch.empty(rows, device=DEV) for _ in range(4))
+    grad = torch.empty_like(x)
+    _lib.ce_fwd(x, t, losses, lse, mx, sm, None, softcap, -100, 0.0, 1.0)
+    _lib.ce_bwd_tiny(x, t, mx, sm, grad, softcap, -100, 0.0, 0.5)
+    unit = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    for i in range(0, rows, 128):
+        r = slice(i, min(i + 128, rows))
+        xs, ts = x[r].double(), t[r]
+        th = torch.tanh(xs / softcap) if softcap else None
+        z = softcap * th if softcap else xs
+        ref = z.logsumexp(-1)
+        assert bool(((lse[r].double() - ref).abs() <= 1e-5 * ref.abs()).all())
+        keep = ts != -100
+        zt = z.gather(1, ts.clamp(min=0)[:, None])[:, 0]
+        assert bool(((losses[r].double() - torch.where(keep, ref - zt, 0.0)).abs() <= 2e-5 * ref.abs()).all())
+        p = torch.exp(z - ref[:, None])
+        d = p - torch.nn.functional.one_hot(ts.clamp(min=0), vocab)
+        want = d * (1 - th * th if softcap else 1.0) * 0.5 * keep[:, None]
+        # (the target's difference is formed in fp32 from terms of up to 1)
+        err = (grad[r].double() - want).abs()
+        assert bool((err <= (unit + 1e-5) * want.abs() + 2.0 ** -25 + 2.0 ** -22 * (d < 0)).all()), float(err.max())
