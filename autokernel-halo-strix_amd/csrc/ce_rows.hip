@@ -32,6 +32,7 @@ struct CeParams {
   const float* scale_dev;  // optional device factor of scale
   int64_t ignore_index;
   bool use_softcap, use_ls;
+  bool nt;  // the logits (and their gradient) pass the last-level cache
 };
 
 __device__ __forceinline__ float cap(const CeParams& p, float x) {
@@ -341,7 +342,7 @@ __device__ void ce_fwd_row(const T* __restrict__ row, int64_t b, const int64_t* 
   if (VEC) {
     const int64_t nvec = vocab / VE;
     for (int64_t v = threadIdx.x; v < nvec; v += kCeThreads) {
-      Vec16<T> xv = load16(row + v * VE);
+      const Vec16<T> xv = p.nt ? load16_nt(row + v * VE) : load16(row + v * VE);
       float xs[VE];
 #pragma unroll
       for (int e = 0; e < VE; ++e) {
@@ -543,13 +544,18 @@ int check(const void* logits, const int64_t* targets, void* grad, int64_t rows, 
 bool past_cache(int64_t bytes) { return bytes > (int64_t)300 << 20; }
 
 // The row-resident forward with the fewest vectors a thread that its workgroup
-// sizes allow (256 threads up to 1024 vectors, for more rows in flight).
+// sizes allow (256 threads up to 1024 vectors, for more rows in flight; 512 up to
+// 4096, since 4 vectors in each of 1024 threads took 122 us for [4096, 32768] bf16 with a
+// softcap, where 8 in 512 take 72). Returns false for the streaming kernel: past 16384
+// vectors, and past 8192 without a gradient in many whole rows, where one held row
+// a CU leaves its loads and its exponentials in turn ([1024, 65536] fp32 54.7 us held,
+// 42.6 streamed, [1024, 131072] bf16 69 and 52; 512 rows 28.4 and 33.5).
 template <typename T, bool CAP>
 bool launch_row(const T* lg, const int64_t* targets, float* losses, float* lse, float* mx,
                 float* sm, T* g, int64_t rows, int64_t vocab, int64_t ld, int64_t ld_g,
-                const CeParams& p, hipStream_t s) {
+                const CeParams& p, bool stream_ok, hipStream_t s) {
   const int64_t nvec = vocab / Vec16<T>::VE;
-  if (nvec > 16384) return false;
+  if (nvec > 16384 || (nvec > 8192 && !g && rows >= 1024 && stream_ok)) return false;
 #define AK_LAUNCH(VPT, TPR)                                                                   \
   ce_row_kernel<T, VPT, TPR, CAP><<<dim3(row_grid(rows)), dim3(TPR), 0, s>>>(                 \
       lg, targets, losses, lse, mx, sm, g, rows, (int)vocab, ld, ld_g, p)
@@ -557,7 +563,7 @@ bool launch_row(const T* lg, const int64_t* targets, float* losses, float* lse, 
   else if (nvec <= 512) AK_LAUNCH(2, 256);
   else if (nvec <= 1024) AK_LAUNCH(4, 256);
   else if (nvec <= 2048) AK_LAUNCH(4, 512);
-  else if (nvec <= 4096) AK_LAUNCH(4, 1024);
+  else if (nvec <= 4096) AK_LAUNCH(8, 512);
   else if (nvec <= 8192) AK_LAUNCH(8, 1024);
   else AK_LAUNCH(16, 1024);
 #undef AK_LAUNCH
@@ -567,14 +573,15 @@ bool launch_row(const T* lg, const int64_t* targets, float* losses, float* lse, 
 template <typename T>
 void launch_fwd(const void* logits, const int64_t* targets, float* losses, float* lse, float* mx,
                 float* sm, void* grad, int64_t rows, int64_t vocab, int64_t ld, int64_t ld_g,
-                const CeParams& p, hipStream_t s) {
+                CeParams p, hipStream_t s) {
   const T* lg = static_cast<const T*>(logits);
   T* g = static_cast<T*>(grad);
+  p.nt = past_cache((grad ? 2 : 1) * rows * vocab * (int64_t)sizeof(T));
   constexpr int VE = Vec16<T>::VE;
   const bool aligned = vocab % VE == 0 && ld % VE == 0 && aligned16(logits);
   const bool done = p.use_softcap
-      ? launch_row<T, true>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, s)
-      : launch_row<T, false>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, s);
+      ? launch_row<T, true>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, aligned, s)
+      : launch_row<T, false>(lg, targets, losses, lse, mx, sm, g, rows, vocab, ld, ld_g, p, aligned, s);
   if (done) return;
   const dim3 grid(row_grid(rows)), block(kCeThreads);
   if (aligned)

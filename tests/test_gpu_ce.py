@@ -301,6 +301,9 @@ def test_ce_fused_backward_kept_graphs_and_hooks():
 
 
 @pytest.mark.parametrize("dtype,rows,vocab,softcap", [
+    (torch.float32, 1023, 8193 * 4, 0.0),    # a held row of more than 8192 vectors
+    (torch.float32, 1024, 8193 * 4, 20.0),   # as many rows as are streamed where no gradient is asked for
+    (torch.float16, 1024, 8193 * 8, 0.0),
     (torch.bfloat16, 1400, 60000, 0.0),      # logits and gradient past the last-level cache
     (torch.bfloat16, 1400, 60001, 20.0)])
 def test_ce_rows_by_size(dtype, rows, vocab, softcap):
