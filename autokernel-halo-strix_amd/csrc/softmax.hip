@@ -27,18 +27,18 @@ namespace {
 // 152 us, 5.4 TB/s, as a copy runs here (523 us with element accesses and two
 // passes); [98304, 777] fp16 56.7 us, 5.4 TB/s.
 //
-// From 4 vectors a thread of 16-bit elements on, the row stays packed between
+// PACKED, from 4 vectors a thread on: the row stays packed between
 // the passes and exp(x - max) is formed twice: 32 registers for 8 vectors
 // instead of 64, so two 1024-thread workgroups fit a CU and one's loads run
-// under the other's arithmetic ([4096, 50256] fp16: 179 -> 151 us).
-template <typename T, int VPT, int TPR, bool RAG>
-__global__ void __launch_bounds__(TPR >= 256 ? TPR : 256, VPT == 8 ? 8 : 1)
+// under the other's arithmetic ([4096, 50256] fp16: 179 -> 151 us). Rows too few
+// for that keep their exponentials ([8, 32000] bf16: 4.9 us, packed 5.7).
+template <typename T, int VPT, int TPR, bool RAG, bool PACKED>
+__global__ void __launch_bounds__(TPR >= 256 ? TPR : 256, VPT == 8 && PACKED ? 8 : 1)
 softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int cols,
                    int64_t ld_x, int64_t ld_y) {
   constexpr int VE = Vec16<T>::VE;
   constexpr int RPW = TPR >= 256 ? 1 : 256 / TPR;
   constexpr int WPR = TPR / 64;
-  constexpr bool PACKED = VPT >= 4;
   static_assert(TPR % 64 == 0, "rows are owned by whole waves");
   __shared__ float part[RPW][WPR];
   const int t = threadIdx.x % TPR;
@@ -224,9 +224,15 @@ void launch_vec(bool aligned, const T* x, T* y, int64_t rows, int cols, int64_t 
   constexpr int RPW = TPR >= 256 ? 1 : 256 / TPR;
   const dim3 grid(row_grid((rows + RPW - 1) / RPW)), block(TPR * RPW);
   if (aligned)
-    softmax_vec_kernel<T, VPT, TPR, false><<<grid, block, 0, s>>>(x, y, rows, cols, ld_x, ld_y);
+    softmax_vec_kernel<T, VPT, TPR, false, (VPT >= 4)><<<grid, block, 0, s>>>(x, y, rows, cols, ld_x, ld_y);
   else
-    softmax_vec_kernel<T, VPT, TPR, true><<<grid, block, 0, s>>>(x, y, rows, cols, ld_x, ld_y);
+    softmax_vec_kernel<T, VPT, TPR, true, (VPT >= 4)><<<grid, block, 0, s>>>(x, y, rows, cols, ld_x, ld_y);
+}
+
+// Few aligned rows: most threads a row, what each holds converted once.
+template <typename T, int VPT, int TPR>
+void launch_few(const T* x, T* y, int64_t rows, int cols, int64_t ld_x, int64_t ld_y, hipStream_t s) {
+  softmax_vec_kernel<T, VPT, TPR, false, false><<<dim3(row_grid(rows)), dim3(TPR), 0, s>>>(x, y, rows, cols, ld_x, ld_y);
 }
 
 template <typename T>
@@ -244,8 +250,20 @@ int dispatch(const void* xv, void* yv, int64_t rows, int64_t cols, int64_t ld_x,
   // fp32 rows) past one wave's 128: with one a thread, half of a workgroup's time
   // went to its reductions. [16384, 8192] bf16 103 -> 84 us, [24000, 3001] fp16
   // 68.9 -> 49.4, [32768, 777] fp32 47.8 -> 36.8, [8192, 4097] fp32 59.6 -> 46.4.
+  // Up to about one workgroup a SIMD the latency of one row counts: one vector a
+  // thread (two and four past 1024 and 2048), unpacked. us, so and as below: [1536,
+  // 2048] bf16 3.8 and 4.3 ([3072, 2048] 7.0 and 5.3), [512, 1536] fp32 3.5 and 3.6,
+  // [64, 16384] bf16 4.1 and 4.4, [512, 32000] 11.3 and 12.0, [8, 65536] 7.1 and 8.9
+  // ([64, 65536] 10.9 and 10.5).
+  auto few = [&](int64_t most) { return aligned && rows <= most; };
+#define AK_FEW(VPT, TPR) launch_few<T, VPT, TPR>(x, y, rows, c, ld_x, ld_y, s)
   if (nvec <= 64) AK_LAUNCH(1, 64);
   else if (nvec <= 128) AK_LAUNCH(2, 64);
+  else if (nvec <= 256 && few(VE == 8 ? 2048 : 256)) AK_FEW(1, 256);
+  else if (nvec > 256 && nvec <= 512 && few(512)) AK_FEW(1, 512);
+  else if (nvec > 1024 && nvec <= 2048 && few(512)) AK_FEW(2, 1024);
+  else if (nvec > 2048 && nvec <= 4096 && few(512)) AK_FEW(4, 1024);
+  else if (nvec > 4096 && nvec <= 8192 && few(32)) AK_FEW(8, 1024);
   else if (nvec <= 256) {
     if (VE == 4) AK_LAUNCH(4, 64);
     else AK_LAUNCH(2, 128);
@@ -260,6 +278,7 @@ int dispatch(const void* xv, void* yv, int64_t rows, int64_t cols, int64_t ld_x,
   else if (nvec <= 8192) AK_LAUNCH(8, 1024);
   else if (nvec <= 16384) AK_LAUNCH(16, 1024);
   else softmax_generic_kernel<T><<<dim3(row_grid(rows)), dim3(256), 0, s>>>(x, y, rows, c, ld_x, ld_y);
+#undef AK_FEW
 #undef AK_LAUNCH
   return ak_check_launch("ak_softmax_fwd");
 }

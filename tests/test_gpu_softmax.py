@@ -146,3 +146,32 @@ def test_softmax_rows_at_any_address(dtype, vecs, over):
             assert bool((d <= 1e-5 * ref[live].double().abs() + 1e-7).all())
         else:
             assert max_ulp(y[live], ref[live]) <= 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vecs,few", [(129, None), (256, None), (257, 512), (512, 512), (1025, 512), (2048, 512),
+                                      (2049, 512), (4096, 512), (4097, 32), (8192, 32)])
+def test_softmax_few_and_many_aligned_rows(dtype, vecs, few):
+    """Whole aligned rows at the widths' edges, as many as the forms for few rows
+    take and one more (up to 256 vectors 2048 rows of 16-bit elements and 256 of
+    fp32), against float64: each value within one rounding beside the fp32
+    exponential's and sum's 1e-6."""
+    need_gpu()
+    from kernels.hip import _lib
+    size = torch.empty((), dtype=dtype).element_size()
+    cols, few = vecs * (16 // size), few or (2048 if size == 2 else 256)
+    g = torch.Generator(device=DEV).manual_seed(cols)
+    x = (4 * torch.randn(few + 1, cols, generator=g, device=DEV)).to(dtype)
+    x[1, ::2] = float("-inf")
+    x[2] = torch.finfo(dtype).min
+    x[3, cols // 2] = float("nan")
+    unit = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    for rows in (few, few + 1):
+        say("softmax few and many rows", dtype, rows, cols)
+        y = torch.full((rows + 1, cols), 7.0, dtype=dtype, device=DEV)
+        _lib.softmax(x[:rows], y[:rows])
+        assert bool((y[rows] == 7).all()) and bool(torch.isnan(y[3]).all())
+        for i in range(0, rows, 256):
+            r = [k for k in range(i, min(i + 256, rows)) if k != 3]
+            ref = torch.softmax(x[r].double(), -1)
+            assert bool(((y[r].double() - ref).abs() <= (unit + 1e-6) * ref + 2.0 ** -25).all())
