@@ -136,9 +136,9 @@ rownorm_vec_kernel(const T* __restrict__ x, const T* __restrict__ r,
   }
 }
 
-// Rows of more than 8192 vectors: a 256-thread workgroup per row (rows by grid
-// stride), scalar accesses, the hidden state recomputed (bit-identically) in
-// the second pass.
+// Rows of more than 8192 vectors, and few short ragged ones: a 256-thread
+// workgroup per row (rows by grid stride), scalar accesses, the hidden state
+// recomputed (bit-identically) in the second pass.
 template <typename T, bool RES>
 __global__ void __launch_bounds__(256)
 rownorm_generic_kernel(const T* __restrict__ x, const T* __restrict__ r,
@@ -213,9 +213,17 @@ int dispatch(const void* xv, const void* rv, const void* wv, void* nrv, void* yv
   // 512 vectors ([8192, 5120] bf16 fused 64.5 -> 57.1 us), and for the plain
   // norm (one input stream) of enough rows ([16384, 2048] bf16 28.3 -> 25.7 us,
   // [16384, 4097] 68.7 -> 56.1; a wave a row in fp32, [8192, 1024] 13.8 -> 11.2).
-  // Few rows stay on one vector a thread: 64 x 4096 takes 3.2 us so and 3.5.
-  const bool two = !RES && rows >= 1024;
-  if (nvec <= 64) AK_LAUNCH(1, 64);
+  // Fewer rows stay on one vector a thread ([1536, 2048] 4.3 us so and 4.8, [3072,
+  // 2048] 7.7 and 6.4; [1024, 4096] 5.3 and 5.6, [1536, 4096] 7.4 and 6.7).
+  const bool two = !RES && rows > (nvec <= 256 ? 2048 : 1024);
+  // A few short ragged rows: a wave's head, vectors and tail in turn take longer than
+  // one element in each of 256 threads (fused [64, 33] bf16 4.0 and 2.6 us, [1024, 129]
+  // 3.6 and 3.2, [64, 401] 3.4 and 3.2; [8192, 33] 6.1 and 7.3).
+  const bool narrow = !aligned && rows <= 1024 && cols <= (rows <= 256 ? 512 : 256);
+  if (narrow) {
+    rownorm_generic_kernel<T, RES><<<dim3(row_grid(rows)), dim3(256), 0, s>>>(
+        x, r, w, nr, y, rows, c, ld_x, ld_r, ld_nr, ld_y, eps);
+  } else if (nvec <= 64) AK_LAUNCH(1, 64);
   else if (nvec <= 128) AK_LAUNCH(1, 128);
   else if (nvec <= 256) {
     if (two && VE == 4) AK_LAUNCH(4, 64);

@@ -211,7 +211,7 @@ rownorm_bwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w,
   }
 }
 
-// Very wide rows (plan_bwd): 256 threads per row with scalar accesses. The row
+// Very wide rows and few short ragged ones (plan_bwd): 256 threads per row with scalar accesses. The row
 // is read twice (sums, then gradients); the workgroup's partial dw row lives
 // in the workspace and is updated by the thread that owns each column.
 template <typename T, bool ADD_DH>
@@ -341,8 +341,9 @@ BwdPlan plan_bwd(const void* x, const void* w, const void* dy, const void* dh, c
   if (dh) p.aligned = p.aligned && ld_dh % VE == 0 && aligned16(dh);
   const int64_t nvec = cols / VE;
   // (ragged 16-bit rows past 4096 vectors spill in the vector kernel: [1000, 40001]
-  // bf16 forward and backward 1036 us with it, 911 with the generic one)
-  if (nvec > 8192 || (!p.aligned && VE == 8 && nvec > 4096)) {
+  // bf16 forward and backward 1036 us with it, 911 with the generic one; a few short
+  // ragged ones take longer there too, [64, 33] bf16 6.8 and 6.3)
+  if (nvec > 8192 || (!p.aligned && ((VE == 8 && nvec > 4096) || (rows <= 64 && cols <= 256)))) {
     p.generic = true;
     p.grid = (int)(rows < kBwdMaxGrid ? rows : kBwdMaxGrid);
     p.nparts = p.grid;

@@ -160,11 +160,11 @@ def test_rownorm_expanded_views_and_grid_stride():
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("vecs,over", [(0, 3), (1, 1), (64, 3), (65, 0), (128, 1), (129, 2), (256, 3), (513, 1),
                                        (1024, 3), (1025, 2), (4097, 1)])
-@pytest.mark.parametrize("rows", [5, 1027])
+@pytest.mark.parametrize("rows", [5, 1027, 2051])
 def test_rownorm_rows_at_any_address(dtype, vecs, over, rows):
     """Ragged rows at the edges of every vectors-per-thread variant (``vecs``
-    16-byte vectors plus ``over`` elements; 1024 and more rows choose others),
-    all operands in pitched views that start off the 16-byte grid, each its own
+    16-byte vectors plus ``over`` elements; more than 1024 and 2048 rows choose
+    others, few short ones the scalar kernel), all operands in pitched views that start off the 16-byte grid, each its own
     way; the elements around the output rows keep their values."""
     need_gpu()
     from kernels.hip import _lib

@@ -227,7 +227,7 @@ def test_backward_of_broadcast_upstream_gradient():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("rows,vecs,over", [(5, 0, 3), (2100, 1, 1), (2100, 64, 3), (8300, 65, 1), (2100, 128, 3),
+@pytest.mark.parametrize("rows,vecs,over", [(5, 0, 3), (64, 31, 3), (65, 31, 3), (2100, 1, 1), (2100, 64, 3), (8300, 65, 1), (2100, 128, 3),
                                             (4200, 130, 1), (2100, 193, 0), (4200, 256, 2), (700, 257, 3), (300, 513, 1),
                                             (40, 1025, 3), (7, 2049, 1)])
 def test_bwd_rows_at_any_address(dtype, rows, vecs, over):
