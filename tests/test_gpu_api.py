@@ -352,3 +352,102 @@ def test_compiled_autograd(op):
         loss.backward()
     for a, w in zip(args, want):
         assert torch.equal(a.grad, w)
+
+
+def _entry_point(name, g):
+    """(leaves, function of them to one or several outputs) of an entry point."""
+    from kernels import ce_fused
+    from kernels.hip import fused_residual_add_rmsnorm as add, rmsnorm, selective_scan as ss, softmax
+    from kernels.hip.chunked_linear_cross_entropy import ChunkedLinearCrossEntropyLoss
+    f32, k = torch.float32, torch.ops.autokernel
+
+    def r(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, generator=g).to(dtype).to(DEV).requires_grad_()
+
+    t = torch.randint(0, 96, (40,), generator=g).to(DEV)
+    t[7] = -100
+    norm = (r(40, 96), r(96))
+    add_norm = (r(40, 96), r(40, 96), r(96))
+    diag = tuple(r(2, 40, 32, dtype=f32) for _ in range(3)) + (r(32, dtype=f32), r(2, 40, 32, dtype=f32))
+    scan = (r(2, 32, 70), r(2, 32, 70), r(32, 16, dtype=f32), r(2, 16, 70), r(2, 16, 70), r(32, dtype=f32), r(2, 32, 70),
+            r(32, dtype=f32))
+
+    def mamba(last):
+        return lambda u, d, A, *rest: ss.selective_scan_fn(u, d, -A.abs(), *rest, True, last)
+
+    def plain(fn):  # no gradient: outputs alone
+        def call(*a):
+            with torch.no_grad():
+                return fn(*a)
+        return call
+
+    return {
+        "rmsnorm": (norm, plain(rmsnorm.kernel_fn)), "add_rmsnorm": (add_norm, plain(add.kernel_fn)),
+        "add_rmsnorm_dual": (add_norm, plain(add.kernel_fn_dual)), "softmax": (norm[:1], plain(softmax.kernel_fn)),
+        "diag": (diag, plain(ss.kernel_fn)), "rmsnorm_op": (norm, k.rmsnorm), "add_rmsnorm_op": (add_norm, k.fused_res_rmsnorm),
+        "diag_op": (diag, k.selective_scan), "scan": (scan, mamba(False)), "scan_last": (scan, mamba(True)),
+        "ce": (norm[:1], lambda x: ce_fused.kernel_fn(x, t)),
+        "ce_fused": (norm[:1], lambda x: ce_fused.ce_full(x, t, softcap=5.0, z_loss_weight=1e-3, return_z=True)),
+        "ce_tiny": (norm[:1], lambda x: ce_fused.ce_full(x, t, mode="tiny", label_smoothing=0.1)),
+        "lmhead": ((r(40, 64), r(96, 64)), lambda h, w: ChunkedLinearCrossEntropyLoss(softcap=5.0)(h, w, t)),
+    }[name]
+
+
+@pytest.mark.parametrize("name", ["rmsnorm", "add_rmsnorm", "add_rmsnorm_dual", "softmax", "diag", "rmsnorm_op", "add_rmsnorm_op",
+                                  "diag_op", "scan", "scan_last", "ce", "ce_fused", "ce_tiny", "lmhead"])
+def test_native_and_python_routes_agree(name, monkeypatch):
+    """Every entry point with the native host side and with it switched off (the
+    form that takes converted, wrapped and traced calls): the same kernels, so the
+    same bits of every output and gradient."""
+    need_gpu()
+    import kernels.hip._torch_ops  # noqa: F401
+    from kernels.hip import _lib
+    leaves, fn = _entry_point(name, torch.Generator().manual_seed(12))
+
+    def run():
+        out = fn(*leaves)
+        out = out if isinstance(out, (tuple, list)) else (out,)
+        diff = [o for o in out if o.requires_grad]
+        return [o.detach() for o in out] + list(torch.autograd.grad(diff, leaves, [torch.full_like(o, 0.5) for o in diff]) if diff else [])
+
+    say("native and python routes", name)
+    native = run()
+    used = []
+    monkeypatch.setattr(_lib, "native", lambda *a: used.append(1))
+    python = run()
+    assert used and len(native) == len(python)
+    for a, b in zip(native, python):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("op", ["rmsnorm_op", "add_rmsnorm_op", "diag_op"])
+def test_formula_backwards_of_native_graphs(op, monkeypatch):
+    """Graphs that the native side recorded before the backward kernels were
+    switched off take the torch formulas, as graphs recorded after it do; both
+    are the kernels' gradients within two roundings of the type (fp32: 1e-4 of
+    the largest, over 40-step products)."""
+    need_gpu()
+    import kernels.hip._torch_ops as ops_module
+    from kernels.hip import _lib
+    leaves, fn = _entry_point(op, torch.Generator().manual_seed(13))
+
+    def record():
+        out = fn(*leaves)
+        return out if isinstance(out, (tuple, list)) else (out,)
+
+    def grads(out):
+        return torch.autograd.grad(out, leaves, [torch.full_like(o, 0.5) for o in out])
+
+    say("formula backwards", op)
+    want = grads(record())
+    recorded = record()
+    monkeypatch.setattr(ops_module, "_BWD_KERNELS_ENABLED", True)  # restored at the end
+    ops_module.disable_hip_backward()
+    try:
+        before, after = grads(recorded), grads(record())
+    finally:
+        _lib.host().set_hip_backward(True)
+    unit = 2.0 ** -7 if leaves[0].dtype == torch.bfloat16 else 1e-4
+    for w, a, b in zip(want, before, after):
+        assert a.dtype == b.dtype == w.dtype and torch.equal(a, b)
+        assert bool(((a.double() - w.double()).abs() <= 2 * unit * w.double().abs() + unit * 0.1 * w.double().abs().amax()).all())

@@ -349,9 +349,9 @@ def test_c4_full_size_softcap():
     assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-6 * scale).all())
 
 
-def test_lmhead_ce_grad_logits_pitch_fallback():
-    """A grad_logits pitch that is a multiple of 4 but not of 8 takes the
-    element-wise store path; the result is the same as the vector path's."""
+def test_lmhead_ce_grad_logits_unaligned_rows():
+    """A grad_logits pitch that is a multiple of 4 but not of 8 puts every other
+    row's 16-byte stores off the 16-byte grid; the result is the aligned rows'."""
     need_gpu()
     from kernels.hip import _lib
     g = torch.Generator().manual_seed(21)

@@ -102,27 +102,45 @@ def test_fast_path_shapes(batch, dim, dstate, seqlen, groups, itype):
         assert torch.allclose(out.float(), ref, rtol=rtol, atol=atol)
 
 
+def _as_one(a, b, ref, rlast):
+    """(out, last) of two paths: both within the grid's tolerance of the oracle,
+    states equal to fp32 rounding, bf16 outputs to one rounding step."""
+    (fast, lf), (gen, lg) = a, b
+    assert torch.allclose(fast.float(), ref, rtol=3e-2, atol=5e-2)
+    assert torch.allclose(gen.float(), ref, rtol=3e-2, atol=5e-2)
+    assert torch.allclose(lf, rlast, rtol=1e-4, atol=1e-4)
+    assert torch.allclose(lf, lg, rtol=1e-5, atol=1e-5)
+    assert ((fast.float() - gen.float()).abs() <= 2 ** -7 * fast.float().abs() + 1e-6).all()
+
+
 def test_fast_and_generic_paths_agree():
-    """The same scan through the whole-tile kernel (contiguous) and the generic
-    kernel (a view with a row pitch that is not a multiple of 4 elements)."""
+    """The same channels through the producer / consumer kernel (32 channels, whole
+    groups of 16) and through the general kernel (the first 24 of them alone)."""
     need_gpu()
     u, delta, A, B, C, D, z, bias = _inputs(2, 32, 16, 320, 1, torch.bfloat16, 31)
     say("mamba fast vs generic")
-    from kernels.hip.selective_scan import selective_scan_fn
+    k = 24
     fast, lf = _gpu(u, delta, A, B, C, D, z, bias, True)
+    gen = _gpu(u[:, :k], delta[:, :k], A[:k], B, C, D[:k], z[:, :k], bias[:k], True)
+    ref, rl = c_oracle.selective_scan(u, delta, A, B, C, D, z, bias, True)
+    _as_one((fast[:, :k], lf[:, :k]), gen, ref[:, :k], rl[:, :k])
+
+
+def test_whole_and_ragged_paths_agree():
+    """The same scan through the producer / consumer kernel's whole-tile form
+    (contiguous) and its form for any alignment (a row pitch of odd elements)."""
+    need_gpu()
+    u, delta, A, B, C, D, z, bias = _inputs(2, 32, 16, 320, 1, torch.bfloat16, 31)
+    say("mamba whole vs ragged")
+    from kernels.hip.selective_scan import selective_scan_fn
     pad = torch.zeros(2, 32, 321, dtype=torch.bfloat16, device=DEV)
     pad[..., :320] = u.to(DEV)
     uv = pad[..., :320]
     assert uv.stride(1) == 321
     d = lambda t: t.to(DEV)
-    gen, lg = selective_scan_fn(uv, d(delta), d(A), d(B), d(C), d(D), d(z), d(bias), True, True)
-    gen, lg = gen.cpu(), lg.cpu()
+    rag = selective_scan_fn(uv, d(delta), d(A), d(B), d(C), d(D), d(z), d(bias), True, True)
     ref, rl = c_oracle.selective_scan(u, delta, A, B, C, D, z, bias, True)
-    assert torch.allclose(fast.float(), ref, rtol=3e-2, atol=5e-2)
-    assert torch.allclose(gen.float(), ref, rtol=3e-2, atol=5e-2)
-    assert torch.allclose(lf, lg, rtol=1e-5, atol=1e-5)
-    # bf16 outputs of the two paths differ by at most one rounding step
-    assert ((fast.float() - gen.float()).abs() <= 2 ** -7 * fast.float().abs() + 1e-6).all()
+    _as_one(_gpu(u, delta, A, B, C, D, z, bias, True), [t.cpu() for t in rag], ref, rl)
 
 
 @pytest.mark.parametrize("itype,softplus,groups", [("bfloat16", False, 1), ("float32", True, 2),
