@@ -182,9 +182,9 @@ __device__ void write_grad_row(const CeParams& p, const T* __restrict__ row, T* 
 // around the vectors one to a thread. HBM-bound: 4 VPT registers hold the row,
 // so up to 8 vectors two 1024-thread workgroups fit a CU and one's loads and
 // stores run under the other's exponentials. [4096, 32768] bf16 with its
-// gradient 155 -> 115 us, 4.7 TB/s (256 threads streamed the row and read it
+// gradient 155 -> 104 us, 5.2 TB/s (256 threads streamed the row and read it
 // again for the gradient); [4096, 50257] fp16 without one 334 -> 74 us, 5.6 TB/s,
-// and the backward from saved statistics 315 -> 164 us (both had element
+// and the backward from saved statistics 315 -> 168 us (both had element
 // accesses).
 template <typename T, int VPT, int TPR, bool CAP>
 __global__ void __launch_bounds__(TPR, VPT == 8 ? 8 : 1)
@@ -597,7 +597,7 @@ void launch_bwd(const void* logits, const int64_t* targets, const float* mx, con
   const T* lg = static_cast<const T*>(logits);
   T* g = static_cast<T*>(grad);
   // workgroups of one round of 4 vectors a thread where the row is that wide:
-  // [4096, 50257] fp16 takes 164 us so and 179 us with one workgroup a row
+  // [4096, 50257] fp16 takes 168 us so and 179 us with one workgroup a row
   const int64_t nvec = vocab / Vec16<T>::VE;
   const int64_t ny = std::min<int64_t>(nvec / (4 * kCeThreads), 65535);
   const int64_t span = ny > 1 ? (nvec + ny - 1) / ny : nvec;

@@ -207,8 +207,9 @@ def make_case(name):
         sets = _replicate(cpu, k)
         for s in sets:
             s["y"] = torch.empty_like(s["x"])
-        # the lean launcher kernels.hip.rmsnorm.kernel_fn uses for contiguous
-        # rows (dense pitch, no 2-D views): a 5 us kernel is issue-bound
+        # the bare ctypes launcher (dense pitch, no 2-D views, y allocated
+        # before): a 5 us kernel is issue-bound. kernel_fn goes through the
+        # native host side, which also checks and allocates
         launch = lambda s: _lib.rmsnorm_contig(s["x"], s["w"], s["y"], 768, s["eps"])
         return Case(name, "C1 RMSNorm fp32 [2048, 768]", "hbm", C1_BYTES, 2048, launch, sets,
                     "rownorm_vec_kernel")

@@ -139,7 +139,7 @@ int ak_fused_add_rmsnorm_bwd_gw(const void* hidden, const void* weight,
  * or training loops, harnesses that forbid hipMalloc); it calls no hipMalloc,
  * hipFree or allocating routine. grad_hidden = NULL gives the plain RMSNorm
  * backward of ak_rmsnorm_bwd (x passed as hidden). Shapes whose partial rows
- * (at most 256 workgroup slots, 1024 for rows of <= 512 bf16 / fp16 elements)
+ * (at most 1024 up to 192 16-byte vectors a row, 512 up to 256, 256 above)
  * times cols x 4 bytes exceed 16 MiB -- cols > 16384 for a full grid -- are
  * rejected with AK_ERR_WORKSPACE; use ak_fused_add_rmsnorm_bwd for those. The
  * array holds four 16 MiB slots per GPU; each stream that calls this on a
