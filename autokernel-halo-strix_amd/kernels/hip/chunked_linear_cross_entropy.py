@@ -105,6 +105,13 @@ def _kernel_operands(hidden: torch.Tensor, weight: torch.Tensor):
     return hidden, weight
 
 
+def _row_targets(targets: torch.Tensor, n: int) -> torch.Tensor:
+    """Contiguous int64 targets for n rows (the kernels read that many)."""
+    if targets.numel() < n:
+        raise ValueError(f"{targets.numel()} targets for {n} rows")
+    return targets.contiguous().to(torch.int64)
+
+
 def lmhead_ce_forward(hidden: torch.Tensor, weight: torch.Tensor, targets: torch.Tensor,
                       ignore_index: int = -100, return_losses: bool = False,
                       softcap: float = 0.0, label_smoothing: float = 0.0):
@@ -115,7 +122,7 @@ def lmhead_ce_forward(hidden: torch.Tensor, weight: torch.Tensor, targets: torch
     """
     _lib.require_device(hidden, weight, targets)
     hidden, weight = _kernel_operands(hidden, weight)
-    targets = targets.contiguous().to(torch.int64)
+    targets = _row_targets(targets, hidden.shape[0])
     n = hidden.shape[0]
     dev = hidden.device
     loss = torch.empty((), dtype=torch.float32, device=dev)
@@ -195,7 +202,7 @@ def lmhead_ce_backward(hidden: torch.Tensor, weight: torch.Tensor, targets: torc
     _lib.require_device(hidden, weight, targets, lse, denom, grad_loss)
     d_in = hidden.shape[1]
     hidden, weight = _kernel_operands(hidden, weight)
-    targets = targets.contiguous().to(torch.int64)
+    targets = _row_targets(targets, hidden.shape[0])
     n, d = hidden.shape
     vocab = weight.shape[0]
     if n == 0:

@@ -156,6 +156,19 @@ def test_chunked_linear_ce(fake_backend, dtype, softcap, ls, zw):
     assert torch.allclose(W.grad.double(), Wr.grad, atol=tol, rtol=tol)
 
 
+def test_lmhead_refuses_fewer_targets_than_rows(fake_backend):
+    """The kernels read a target for each row: fewer are refused before any launch."""
+    from kernels.hip import chunked_linear_cross_entropy as m
+    h, W, t = torch.randn(8, 64).bfloat16(), torch.randn(32, 64).bfloat16(), torch.arange(7)
+    one = torch.ones(1)
+    with pytest.raises(ValueError, match="7 targets for 8 rows"):
+        m.lmhead_ce_forward(h, W, t)
+    with pytest.raises(ValueError, match="7 targets for 8 rows"):
+        m.ChunkedLinearCrossEntropyLoss()(h, W, t)
+    with pytest.raises(ValueError, match="7 targets for 8 rows"):
+        m.lmhead_ce_backward(h, W, t, torch.zeros(8), one, one)
+
+
 def test_torch_ops_registered_with_fake_and_autograd(fake_backend):
     import kernels.hip._torch_ops  # noqa: F401
     x = torch.randn(6, 32, requires_grad=True)
