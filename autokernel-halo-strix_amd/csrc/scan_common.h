@@ -78,7 +78,9 @@ struct ScanParams {
 //   12 x 128 20.4 -> 20.5), from 12 on with a partial tile, whose kernel is the
 //   slower one (12 x 128: 22.7 -> 21.1); about 1024 segments up to 144 from 64 tiles
 //   (64 x 144: 95.9 -> 88; 32 x 144 49.6 -> 52), with a partial tile from 32 (57.3
-//   -> 54). 64 x 160 would go 96.5 -> 99, 24 x 192 38.4 -> 49.
+//   -> 54). 64 x 160 would go 96.5 -> 99, 24 x 192 38.4 -> 49. Channels that do not
+//   fill groups of 16 run the general kernel, slower still: as the reverse pass (4 x
+//   128: 14.7 -> 11.9, 24 x 188 72 -> 62).
 // * reverse pass, with three exponentials a step to the segment pass's one: about
 //   512 segments up to 128 workgroups from 4 tiles on (4 x 128: 34.6 -> 28.6, with
 //   its preparation pass 43 -> 39), about 1024 up to 192 from 24 on (24 x 192:
@@ -93,12 +95,13 @@ inline ScanSegs scan_segments(bool reverse, int64_t batch, int64_t dim, int64_t 
   const int64_t tiles = (seqlen + kScanT - 1) / kScanT;
   const int64_t groups = batch * ngroups * ((dim / ngroups + kScanCh - 1) / kScanCh);
   const bool whole = seqlen % kScanT == 0;
+  const bool early = reverse || (dim / ngroups) % kScanCh != 0;
   int64_t n = 1;
   if (dstate <= 16 && !(bc_flags & (AK_SCAN_B_CONST | AK_SCAN_C_CONST)) && groups > 0) {
-    const int64_t few = reverse ? 4 : groups <= 64 ? 6 : whole ? 16 : 12;  // tiles from which on a cut pays
-    const int64_t many = reverse ? 24 : whole ? 64 : 32;
+    const int64_t few = early ? 4 : groups <= 64 ? 6 : whole ? 16 : 12;  // tiles from which on a cut pays
+    const int64_t many = early ? 24 : whole ? 64 : 32;
     if (groups <= 128 && tiles >= few) n = (512 + groups / 2) / groups;
-    else if (groups <= (reverse ? 192 : 144) && tiles >= many) n = 1024 / groups;
+    else if (groups <= (early ? 192 : 144) && tiles >= many) n = 1024 / groups;
     if (n > 32) n = 32;
     if (n > tiles) n = tiles;
     if (n < 1) n = 1;
@@ -225,13 +228,27 @@ __device__ __forceinline__ float seg_enter(const ScanParams& p, const ScanSeg<kS
   float h = 0.0f;
   if constexpr (!kSeg) return h;
   const int count = kBwd ? p.segs - 1 - sg.seg : sg.seg;
-#pragma unroll 4
-  for (int i = 0; i < count; ++i) {
-    const int64_t at = ((int64_t)sg.b * p.segs + (kBwd ? p.segs - 1 - i : i)) * p.dim + d;
-    const float t = fminf(fmaxf(a_scaled * p.seg_dsum[at], -1000.0f), 1000.0f);  // 2^1000 takes any fp32 to its end
-    const float k = fabsf(t) < 126.0f ? 0.0f : truncf(t);
-    h = fmaf(__builtin_amdgcn_exp2f(t - k), ldexpf(h, (int)k), p.seg_state[at * p.dstate + n]);
-  }
+  auto fold = [&](int i0, auto batch) {  // segments i0 .. i0 + U - 1, loaded at once
+    constexpr int U = decltype(batch)::value;
+    float in[U], t[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int i = min(i0 + j, count - 1);
+      const int64_t at = ((int64_t)sg.b * p.segs + (kBwd ? p.segs - 1 - i : i)) * p.dim + d;
+      in[j] = p.seg_state[at * p.dstate + n];
+      t[j] = a_scaled * p.seg_dsum[at];
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const float c = fminf(fmaxf(t[j], -1000.0f), 1000.0f);  // 2^1000 takes any fp32 to its end
+      const float k = fabsf(c) < 126.0f ? 0.0f : truncf(c);
+      const float next = fmaf(__builtin_amdgcn_exp2f(c - k), ldexpf(h, (int)k), in[j]);
+      h = i0 + j < count ? next : h;
+    }
+  };
+  int i = 0;
+  for (; count - i > 4; i += 8) fold(i, std::integral_constant<int, 8>{});
+  if (i < count) fold(i, std::integral_constant<int, 4>{});
   return h;
 }
 

@@ -489,10 +489,11 @@ def test_segments_keep_an_infinite_state():
 
 @pytest.mark.parametrize("batch,dim,seqlen,segs", [
     (1, 16, 320, 1), (1, 1024, 321, 6), (1, 1040, 704, 1), (1, 1040, 705, 6), (1, 2048, 960, 1), (1, 2048, 1024, 4),
-    (1, 2064, 1984, 1), (1, 2064, 1985, 7), (2, 1152, 4032, 1), (2, 1152, 4096, 7), (1, 2320, 4095, 1)])
+    (1, 2064, 1984, 1), (1, 2064, 1985, 7), (2, 1152, 4032, 1), (2, 1152, 4096, 7), (1, 2320, 4095, 1),
+    (1, 24, 192, 1), (1, 24, 193, 4), (1, 2040, 256, 4), (1, 2056, 1472, 1), (1, 3064, 1536, 5), (1, 3080, 1536, 1)])
 def test_forward_cuts_at_the_edges_of_the_rule(batch, dim, seqlen, segs):
-    """64, 128 and 144 channel groups, whole and partial last tiles: how many
-    segments the forward's scratch is for, and the cut scan against the one
+    """64, 128 and 144 channel groups, whole and partial last tiles, and 128 and 192
+    groups that are not whole: how many segments the forward's scratch is for, and the cut scan against the one
     without scratch (states equal to fp32 rounding, 4e-6 of the largest, outputs
     to one more rounding)."""
     need_gpu()
