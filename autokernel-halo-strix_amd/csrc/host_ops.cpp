@@ -72,8 +72,9 @@ bool plain(const Tensor& t) {
          !t._fw_grad(0).defined();
 }
 
+// (function modes are the loader's to look at: a default device is one, too)
 bool quiet() {
-  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
          !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
 

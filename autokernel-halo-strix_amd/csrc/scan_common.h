@@ -81,10 +81,10 @@ struct ScanParams {
 //   -> 54). 64 x 160 would go 96.5 -> 99, 24 x 192 38.4 -> 49. Channels that do not
 //   fill groups of 16 run the general kernel, slower still: as the reverse pass (4 x
 //   128: 14.7 -> 11.9, 24 x 188 72 -> 62).
-// * reverse pass, with three exponentials a step to the segment pass's one: about
-//   512 segments up to 128 workgroups from 4 tiles on (4 x 128: 34.6 -> 28.6, with
-//   its preparation pass 43 -> 39), about 1024 up to 192 from 24 on (24 x 192:
-//   128 -> 103, 170 -> 151; 24 x 144 126 -> 89).
+// * reverse pass, whose steps cost several times the segment pass's: about 512
+//   segments up to 128 workgroups from 4 tiles on (4 x 128: 32.0 -> 27.4, with its
+//   preparation pass 41 -> 39), about 1024 up to 192 from 24 on (24 x 192: 128 -> 103,
+//   169 -> 152; 24 x 144 126 -> 89).
 // A function of the shape alone: the bits of a result depend on it. Where the
 // forward is cut, the reverse pass is cut alike.
 struct ScanSegs {

@@ -26,6 +26,7 @@ import threading
 from typing import Optional
 
 import torch
+from torch.utils._device import DeviceContext
 
 LIB_NAME = "libautokernel_gfx950.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
@@ -160,17 +161,26 @@ def host():
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_modes = torch._C._len_torch_function_stack
+
+
+def _only_devices() -> bool:
+    """Whether the function modes in force are default devices alone, which say
+    where a tensor is made that names no device."""
+    return all(type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(_modes()))
 
 
 def native(*tensors):
     """:func:`host` where a call on these tensors may be its, else None: GPU
     tensors of torch's own classes (a subclass may take part in each torch call),
-    and not while torch.compile traces the call (the Python forms below it are
-    the traced ones)."""
+    no function mode that may either, and not while torch.compile traces the call
+    (the Python forms below it are the traced ones)."""
     for t in tensors:
-        if type(t) not in _PLAIN or not t.is_cuda:
+        if type(t) not in _PLAIN:
             return None
-    return None if _is_compiling() else (_host or host())
+    if _is_compiling() or (_modes() and not _only_devices()) or not tensors[0].is_cuda:
+        return None
+    return _host or host()  # (which looks at the other tensors' devices itself)
 
 
 def is_available() -> bool:

@@ -304,6 +304,39 @@ def test_tensor_subclasses_keep_their_route():
     assert type(rmsnorm(x, torch.nn.Parameter(w))) is torch.Tensor
 
 
+def test_function_modes_and_the_native_route(monkeypatch):
+    """A default device does not keep calls from the native side; a function mode
+    that looks at torch's calls sees them, from the Python form."""
+    need_gpu()
+    from torch.overrides import TorchFunctionMode
+    from kernels.hip import _lib
+    from kernels.hip.softmax import kernel_fn as softmax
+
+    class Watch(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    say("function modes")
+    x = torch.randn(4, 64, device=DEV)
+    want = softmax(x)
+    python = []
+    launch = _lib.softmax
+    monkeypatch.setattr(_lib, "softmax", lambda *a: python.append(1) or launch(*a))
+    with torch.device(DEV):
+        assert _lib.native(x) is not None and torch.equal(softmax(x), want)
+    with torch.device("cpu"):
+        y = softmax(x)
+    assert y.is_cuda and torch.equal(y, want) and not python
+    with Watch() as w, torch.device(DEV):
+        y = softmax(x)
+    assert torch.equal(y, want) and python and "empty" in w.seen
+
+
 def test_rows_of_no_columns():
     need_gpu()
     from kernels.hip.rmsnorm import kernel_fn as rmsnorm
